@@ -46,7 +46,13 @@ extern "C" {
     G2_ROWS_LIST(X, STORE, "store") G2_ROWS_LIST(X, LN_QKV, "ln_qkv")         \
     G2_ROWS_LIST(X, RESID, "resid") G2_ROWS_LIST(X, LN_GELU, "ln_gelu")       \
     G2_ROWS_LIST(X, LN_ARGMAX, "ln_argmax")                                   \
-    X(GEMM_KN_F32, "g2k_gemm_kn_f32") X(GEMM_KN_F16, "g2k_gemm_kn_f16")       \
+    X(XGEMM128_F32, "g2k_xgemm128_f32") X(XGEMM128_F16, "g2k_xgemm128_f16")   \
+    X(XGEMM64_F32, "g2k_xgemm64_f32") X(XGEMM64_F16, "g2k_xgemm64_f16")       \
+    X(XGEMM64_PART_F32, "g2k_xgemm64_part_f32")                               \
+    X(XGEMM64_PART_F16, "g2k_xgemm64_part_f16")                               \
+    X(XGEMM_SUM, "g2k_xgemm_sum")                                             \
+    X(XSKINNY1_F32, "g2k_xskinny1_f32") X(XSKINNY1_F16, "g2k_xskinny1_f16")   \
+    X(XSKINNY2_F32, "g2k_xskinny2_f32") X(XSKINNY2_F16, "g2k_xskinny2_f16")   \
     X(GEMM_NK_F32_STORE, "g2k_gemm_nk_f32_store")                             \
     X(GEMM_NK_F16_STORE, "g2k_gemm_nk_f16_store")                             \
     X(GEMM_NK_F32_GELU, "g2k_gemm_nk_f32_gelu")                               \

@@ -71,6 +71,7 @@ typedef struct {
     const uint16_t *Ah, *Al;
     uint16_t *Ch, *Cl;
 } g2_gemm_args;
+#define G2_XG_MAXKS 12 /* K splits that g2k_xgemm_sum adds */
 
 /* C[m,n] = C[m,n] + ((sum over z < ks in order of part[z*M*N + m*N + n]) +
  * bias[n]) for m < M, n < N.  g2k_splitk_resid_ln (grid M, N <=

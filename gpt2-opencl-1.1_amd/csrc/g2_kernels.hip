@@ -457,7 +457,8 @@ extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout
 }
 
 /* ======================================================================
- * MFMA GEMM (prefill and the reference matmul)
+ * MFMA GEMM (the fused prefill where the forms below do not apply; the
+ * reference matmul is in g2_matmul.hip)
  *
  * Tile 64x64x16, 256 threads = 2x2 waves of 32x32, each wave a 2x2 grid of
  * v_mfma_f32_16x16x4f32.  A [M,K] fp32 row-major; B [K,N] (BKN) or [N,K]
@@ -620,8 +621,6 @@ __device__ void gemm_impl(const g2_gemm_args &a)
 #define G2_GEMM(name, BT, BNK, EPI) \
     G2K void name(const g2_gemm_args a) { gemm_impl<BT, BNK, EPI>(a); }
 
-G2_GEMM(g2k_gemm_kn_f32, float, false, GEPI_STORE)
-G2_GEMM(g2k_gemm_kn_f16, _Float16, false, GEPI_STORE)
 G2_GEMM(g2k_gemm_nk_f32_store, float, true, GEPI_STORE)
 G2_GEMM(g2k_gemm_nk_f16_store, _Float16, true, GEPI_STORE)
 G2_GEMM(g2k_gemm_nk_f32_gelu, float, true, GEPI_GELU)
@@ -1996,6 +1995,7 @@ G2K void g2k_ln_fold_f32(const g2_lnfold_args a) { ln_fold_impl<float>(a); }
 G2K void g2k_ln_fold_f16(const g2_lnfold_args a) { ln_fold_impl<_Float16>(a); }
 
 /* Fused decode kernels (packed matvecs, single-query attention). */
+#include "g2_matmul.hip"
 #include "g2_decode.hip"
 
 /* The persistent decode step (one cooperative launch per token). */

@@ -1,0 +1,489 @@
+/*
+ * g2_matmul.hip -- fp32-accurate GEMM on the bf16 matrix cores (included by
+ * g2_kernels.hip, which provides the shared helpers and types).
+ *
+ * An fp32 value is the sum of three bf16 values: p1 = bf16(v), p2 = bf16(v -
+ * p1), p3 = bf16(v - p1 - p2), 8 significant bits each, both differences
+ * exact; an fp16 value is the sum of two.  A product of two fp32 values is
+ * then six bf16 products, p1q1 + p1q2 + p2q1 + p2q2 + p1q3 + p3q1 (five with
+ * an fp16 factor, whose q3 is zero); the ones left out are below 2^-25 of
+ * it.  The products are exact in fp32 and summed in fp32 by
+ * v_mfma_f32_16x16x32_bf16, which takes 32 k per instruction at 16 times the
+ * rate of the fp32 instruction (4 k): a sixth of 32 k against 4 k leaves
+ * 2.7 times the fp32 peak and fewer roundings of the running sum.
+ *
+ * What the parts cannot carry shows in the accumulator: infinities, NaN and
+ * magnitudes that round past bf16's largest make it not finite; factors so
+ * small (all of a row or column below 2^-109) that their low parts are
+ * subnormal bf16 leave it below 2^-60, unless the other factors exceed 2^40.
+ * Such an output, not zero, is computed again in fp32 (again()), so an
+ * infinity or NaN comes out as fp32 arithmetic has it.
+ */
+namespace xg {
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+/* vectors at any element's address */
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef _Float16 f16x2u __attribute__((ext_vector_type(2), aligned(2)));
+
+/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts. */
+template <int P>
+__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P])
+{
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        f32x2 r = {v[2 * e], v[2 * e + 1]};
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
+            o[p][e] = w;
+            if (p + 1 < P) {
+                r.x -= __builtin_bit_cast(float, w << 16);
+                r.y -= __builtin_bit_cast(float, w & 0xffff0000u);
+            }
+        }
+    }
+}
+
+__device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
+                                                   0, 0, 0);
+}
+
+/* acc[j] += a . b[j] over 32 k: the six (PB 3) or five (PB 2) products,
+ * small ones first.  Successive instructions take different accumulators:
+ * a chain of them on one accumulator waits for each result. */
+template <int PB, int J>
+__device__ __forceinline__ void mma_parts(f32x4 (&acc)[J], const u32x4 (&a)[3], const u32x4 (&b)[J][PB])
+{
+    constexpr int pa[6] = {2, 1, 0, 1, 0, 0}, pb[6] = {0, 0, 1, 1, 2, 0};
+#pragma unroll
+    for (int p = 0; p < 6; ++p)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+            if (pb[p] < PB) acc[j] = mma(a[pa[p]], b[j][pb[p] < PB ? pb[p] : 0], acc[j]);
+}
+
+/* The bit of an accumulator value that has to be computed again. */
+__device__ __forceinline__ bool odd_value(float v)
+{
+    const unsigned b = __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
+    return b >= 0x7f800000u || (b != 0 && b < (67u << 23));
+}
+
+/* Output (m, n) over k0 <= k < k1 in fp32, in order; a sum that has become
+ * NaN stays NaN. */
+template <typename BT, bool BNK>
+__device__ __noinline__ float again(const float *A, const BT *B, int N, int K, int m, int n, int k0, int k1)
+{
+    const float *a = A + (size_t)m * K;
+    const BT *b = B + (BNK ? (size_t)n * K : (size_t)n);
+    const size_t sb = BNK ? 1 : (size_t)N;
+    float s = 0.f;
+    int k = k0;
+    for (; k + 16 <= k1 && s == s; k += 16) {
+        float x[16], y[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            x[e] = a[k + e];
+            y[e] = ldw(b, (size_t)(k + e) * sb);
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s = fmaf(x[e], y[e], s);
+    }
+    for (; k < k1 && s == s; ++k) s = fmaf(a[k], ldw(b, (size_t)k * sb), s);
+    return s;
+}
+
+/* The k, within a step of 32, of element e of octet o is 4 o + koff(e), for
+ * both factors: the four lanes of a row then load 64 consecutive bytes. */
+__device__ __forceinline__ constexpr int koff(int e) { return e < 4 ? e : 12 + e; }
+
+/* Tile of work-group w of T tiles: XCD w % 8 (consecutive work-groups go to
+ * consecutive XCDs) takes a contiguous run of tiles, row blocks first, so
+ * the row blocks of a column block share one XCD's L2; the runs differ by
+ * at most one tile. */
+__device__ __forceinline__ int tile_of(int w, int T)
+{
+    const int x = w & 7, q = T >> 3, r = T & 7;
+    return x * q + min(x, r) + (w >> 3);
+}
+} /* namespace xg */
+
+/* LDS-tiled: BM x BN outputs per work-group of 2 x 2 waves, K in steps of 32,
+ * the steps of a split (gridDim.y splits of whole steps, GEPI_PARTIAL) in
+ * order.  A step's tiles are loaded to registers one step ahead, split into
+ * their parts and stored to LDS as [part][k octet][row] 16-byte fragments, so
+ * a fragment read takes 16 consecutive rows of an octet (no bank conflicts);
+ * the octet planes of row-major operands are padded by 64 bytes so that the
+ * four octets of four rows that 16 lanes store fall on distinct banks.  B
+ * [K,N]: a lane loads a column pair (BN 128) or a column (BN 64) of eight k
+ * rows, so the transposition is a choice of registers; column n of a 128-wide
+ * tile sits at position n / 2 + 64 (n odd), which makes a lane's two column
+ * blocks neighbours in memory.  N >= 2 for BN 128; nothing else is asked of
+ * M, N, K or alignment.
+ *
+ * Measured on MI355X (N(0,1) by N(0,0.02)): 1024 x 50257 x 1600 in 0.80 ms
+ * with fp32 B (1.24 PFLOP/s of bf16 products, above the 1.14 that a library
+ * bf16 product of 8192^3 reaches; the fp32-instruction kernel before: 3.35
+ * ms), 0.66 ms with fp16 B (3.05).  Taken back: two steps in flight, two LDS
+ * buffers, all fragments read ahead, raised wave priority (each within 5%),
+ * and two groups of four waves that alternate between splitting and
+ * multiplying on one tile (up to 30% faster at one tile per CU, 10% slower
+ * with many). */
+template <typename BT, bool BNK, int EPI, int BM, int BN>
+__device__ void xgemm_impl(const g2_gemm_args &a)
+{
+    using namespace xg;
+    constexpr int PB = sizeof(BT) == 4 ? 3 : 2;
+    constexpr int SA = BM * 16 + 64, SB = BN * 16 + (BNK ? 64 : 0); /* octet plane strides, bytes */
+    constexpr int RA = BM / 64, RB = BN / 64;                       /* octets (BNK, A) or columns a thread stages */
+    constexpr int IB = BM / 32, JB = BN / 32;                       /* 16-blocks of a wave */
+    constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
+    __shared__ __attribute__((aligned(16))) unsigned char lds[ST];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    const int M = a.M, N = a.N, K = a.K;
+    const int nmb = (M + BM - 1) / BM;
+    const int tile = tile_of(blockIdx.x, gridDim.x);
+    const int m0 = (tile % nmb) * BM, n0 = (tile / nmb) * BN;
+    const int nkt = (K + 31) >> 5, ks = gridDim.y;
+    const int s0 = (int)(((long)nkt * blockIdx.y) / ks), s1 = (int)(((long)nkt * (blockIdx.y + 1)) / ks);
+    const int sf = min(s1, K >> 5); /* steps s0 .. sf - 1 are whole */
+    const BT *B = (const BT *)a.B;
+
+    const int ar = tid >> 2, ao = (tid & 3) * 4; /* row-major staging: row (+ 64 i), k offset */
+    const float *ap[RA];
+#pragma unroll
+    for (int i = 0; i < RA; ++i) ap[i] = a.A + (size_t)min(m0 + ar + 64 * i, M - 1) * K + ao;
+    /* [K,N] staging: column (pair), octet; the pair that the last column
+     * begins is loaded one column early */
+    const int bc = tid & 63, bo = wave;
+    const bool late = !BNK && n0 + bc * RB + RB - 1 == N;
+    const BT *bp[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+        bp[i] = BNK ? B + (size_t)min(n0 + ar + 64 * i, N - 1) * K + ao : B + min(n0 + bc * RB, N - RB);
+
+    float av[RA][8], bv[RB][8];
+    /* whole step t (past the last one: that one again, unused) */
+    auto load = [&](int t) {
+        const int k = min(t, sf - 1) * 32;
+#pragma unroll
+        for (int i = 0; i < RA; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) *(f32x4 *)(av[i] + 4 * h) = *(const f32x4u *)(ap[i] + k + 16 * h);
+        if constexpr (BNK) {
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *(f32x4 *)(bv[i] + 4 * h) = *(const f32x4u *)((const float *)bp[i] + k + 16 * h);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const size_t o = (size_t)(k + 4 * bo + koff(e)) * N;
+                if constexpr (RB == 1) {
+                    bv[0][e] = ldw(bp[0], o);
+                } else if constexpr (sizeof(BT) == 4) {
+                    const f32x2 w = *(const f32x2u *)((const float *)bp[0] + o);
+                    bv[0][e] = w.x;
+                    bv[RB - 1][e] = w.y;
+                } else {
+                    const f16x2u w = *(const f16x2u *)((const _Float16 *)bp[0] + o);
+                    bv[0][e] = (float)w.x;
+                    bv[RB - 1][e] = (float)w.y;
+                }
+            }
+        }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int i = 0; i < RA; ++i) {
+            u32x4 p[3];
+            parts8<3>(av[i], p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
+        }
+        if constexpr (!BNK && RB == 2) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bv[0][e] = late ? bv[1][e] : bv[0][e];
+        }
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            u32x4 p[PB];
+            parts8<PB>(bv[i], p);
+#pragma unroll
+            for (int q = 0; q < PB; ++q)
+                *(u32x4 *)(lds + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
+        }
+    };
+
+    f32x4 acc[IB][JB];
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int j = 0; j < JB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    /* column block j of the wave: positions 16 j of its half (BNK, BN 64), or
+     * (JB 4) blocks 0, 1 of the even columns and 2, 3 of the odd ones */
+    constexpr bool PAIR = !BNK && RB == 2;
+    const int arow = (lane >> 4) * SA + (wm * (BM / 2) + (lane & 15)) * 16;
+    const int brow = 12 * SA + (lane >> 4) * SB + (wn * (PAIR ? BN / 4 : BN / 2) + (lane & 15)) * 16;
+    auto bblk = [](int j) { return PAIR ? (j & (JB / 2 - 1)) * 256 + (j / (JB / 2)) * (BN / 2) * 16 : j * 256; };
+    auto multiply = [&]() {
+        u32x4 b[JB][PB];
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+#pragma unroll
+            for (int q = 0; q < PB; ++q) b[j][q] = *(const u32x4 *)(lds + brow + 4 * q * SB + bblk(j));
+#pragma unroll
+        for (int i = 0; i < IB; ++i) {
+            u32x4 f[3];
+#pragma unroll
+            for (int q = 0; q < 3; ++q) f[q] = *(const u32x4 *)(lds + arow + 4 * q * SA + i * 256);
+            mma_parts<PB, JB>(acc[i], f, b);
+        }
+    };
+
+    if (sf > s0) {
+        load(s0);
+        for (int t = s0; t < sf; ++t) {
+            __syncthreads(); /* the previous step has been read */
+            store();
+            load(t + 1);
+            __syncthreads();
+            multiply();
+        }
+    }
+    if (sf < s1) { /* the last, partial step: zeros past K */
+        const int k = sf * 32;
+#pragma unroll
+        for (int i = 0; i < RA; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) av[i][e] = k + ao + koff(e) < K ? ap[i][k + koff(e)] : 0.f;
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int kk = k + koff(e) + (BNK ? ao : 4 * bo);
+                bv[i][e] = kk < K ? (BNK ? ldw(bp[i], k + koff(e)) : ldw(bp[0], (size_t)kk * N + i)) : 0.f;
+            }
+        __syncthreads();
+        store();
+        __syncthreads();
+        multiply();
+    }
+
+    /* output (row, column) of accumulator value (i, j, q) */
+    auto om = [&](int i, int q) { return m0 + wm * (BM / 2) + i * 16 + 4 * (lane >> 4) + q; };
+    auto on = [&](int j) {
+        return PAIR ? n0 + 2 * (wn * (BN / 4) + (j & (JB / 2 - 1)) * 16 + (lane & 15)) + j / (JB / 2)
+                    : n0 + wn * (BN / 2) + j * 16 + (lane & 15);
+    };
+    unsigned long long odd = 0;
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int j = 0; j < JB; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (odd_value(acc[i][j][q])) odd |= 1ull << ((i * JB + j) * 4 + q);
+    while (odd) {
+        const int c = __ffsll(odd) - 1;
+        odd &= odd - 1;
+        const int m = om(c / (4 * JB), c & 3), n = on((c >> 2) % JB);
+        const float v = m < M && n < N ? again<BT, BNK>(a.A, B, N, K, m, n, s0 * 32, min(s1 * 32, K)) : 0.f;
+#pragma unroll
+        for (int i = 0; i < IB; ++i)
+#pragma unroll
+            for (int j = 0; j < JB; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (c == (i * JB + j) * 4 + q) acc[i][j][q] = v;
+    }
+
+    float *C = EPI == GEPI_PARTIAL ? a.part + (size_t)blockIdx.y * M * N : a.C;
+    if constexpr (EPI != GEPI_PARTIAL) {
+        if (a.bias) {
+#pragma unroll
+            for (int j = 0; j < JB; ++j) {
+                const float b = a.bias[min(on(j), N - 1)];
+#pragma unroll
+                for (int i = 0; i < IB; ++i) acc[i][j] += b;
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int m = om(i, q);
+            if (m >= M) continue;
+            if constexpr (PAIR) {
+#pragma unroll
+                for (int j = 0; j < JB / 2; ++j) {
+                    const int n = on(j);
+                    float *c = C + (size_t)m * N + n;
+                    if (n + 1 < N) *(f32x2u *)c = (f32x2){acc[i][j][q], acc[i][j + JB / 2][q]};
+                    else if (n < N) *c = acc[i][j][q];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < JB; ++j)
+                    if (on(j) < N) C[(size_t)m * N + on(j)] = acc[i][j][q];
+            }
+        }
+}
+
+#define G2_XGEMM(name, BT, BNK, EPI, BM, BN, OCC) \
+    extern "C" __global__ __launch_bounds__(256, OCC) void name(const g2_gemm_args a) { xgemm_impl<BT, BNK, EPI, BM, BN>(a); }
+G2_XGEMM(g2k_xgemm128_f32, float, false, GEPI_STORE, 128, 128, 2)
+G2_XGEMM(g2k_xgemm128_f16, _Float16, false, GEPI_STORE, 128, 128, 2)
+G2_XGEMM(g2k_xgemm64_f32, float, false, GEPI_STORE, 64, 64, 3)
+G2_XGEMM(g2k_xgemm64_f16, _Float16, false, GEPI_STORE, 64, 64, 3)
+G2_XGEMM(g2k_xgemm64_part_f32, float, false, GEPI_PARTIAL, 64, 64, 3)
+G2_XGEMM(g2k_xgemm64_part_f16, _Float16, false, GEPI_PARTIAL, 64, 64, 3)
+
+/* C = (part[0] + ... + part[ks-1]) + bias, the splits in order; four
+ * elements of the M x N matrix per thread, ks <= G2_XG_MAXKS. */
+G2K void g2k_xgemm_sum(const g2_gemm_args a)
+{
+    const size_t MN = (size_t)a.M * a.N;
+    for (size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4; i < MN; i += (size_t)gridDim.x * 1024) {
+        if (i + 4 <= MN) {
+            f32x4 p[G2_XG_MAXKS];
+#pragma unroll
+            for (int z = 0; z < G2_XG_MAXKS; ++z)
+                if (z < a.ksplit) p[z] = *(const xg::f32x4u *)(a.part + z * MN + i);
+            f32x4 v = p[0];
+#pragma unroll
+            for (int z = 1; z < G2_XG_MAXKS; ++z)
+                if (z < a.ksplit) v += p[z];
+            if (a.bias) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] += a.bias[(i + e) % (size_t)a.N];
+            }
+            *(xg::f32x4u *)(a.C + i) = v;
+        } else {
+            for (size_t j = i; j < MN; ++j) {
+                float v = a.part[j];
+                for (int z = 1; z < a.ksplit; ++z) v += a.part[z * MN + j];
+                a.C[j] = a.bias ? v + a.bias[j % (size_t)a.N] : v;
+            }
+        }
+    }
+}
+
+/* Few tiles: a work-group of 8 waves takes one 16 RB x 32 tile, the K steps
+ * dealt to the waves in turn, their sums added in wave order through LDS.  No
+ * staging: a lane loads its own fragments (8 k of a row of A; 8 rows of a
+ * column pair of B) straight from memory, and the loads of the next step are
+ * issued before the products of this one.  Bounded by load latency, one wait
+ * per step: 64 x 2304 x 768 takes 8 us (the fp32-instruction kernel before:
+ * 57), 96 x 768 x 3072 14 us (218).  16 waves, and 64-row tiles, were no
+ * faster.  N >= 2. */
+template <typename BT, int RB>
+__device__ void xskinny_impl(const g2_gemm_args &a)
+{
+    using namespace xg;
+    constexpr int PB = sizeof(BT) == 4 ? 3 : 2, NW = 8;
+    __shared__ float red[NW][RB * 2][256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int M = a.M, N = a.N, K = a.K;
+    const int nmb = (M + 16 * RB - 1) / (16 * RB);
+    const int tile = tile_of(blockIdx.x, gridDim.x);
+    const int m0 = (tile % nmb) * 16 * RB, n0 = (tile / nmb) * 32;
+    const BT *B = (const BT *)a.B;
+    const int fr = lane & 15, fk = 4 * (lane >> 4);
+    /* column pair; the pair that the last column begins is loaded one
+     * column early */
+    const bool late = n0 + 2 * fr + 1 == N;
+    const float *ap[RB];
+#pragma unroll
+    for (int i = 0; i < RB; ++i) ap[i] = a.A + (size_t)min(m0 + 16 * i + fr, M - 1) * K + fk;
+    const BT *bp = B + min(n0 + 2 * fr, N - 2);
+    const int nkt = (K + 31) >> 5;
+
+    float av[RB][8], bv[2][8];
+    auto load = [&](int t) {
+        const int k = t * 32;
+        if (k + 32 <= K) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const size_t o = (size_t)(k + fk + koff(e)) * N;
+                if constexpr (sizeof(BT) == 4) {
+                    const f32x2 w = *(const f32x2u *)((const float *)bp + o);
+                    bv[0][e] = w.x;
+                    bv[1][e] = w.y;
+                } else {
+                    const f16x2u w = *(const f16x2u *)((const _Float16 *)bp + o);
+                    bv[0][e] = (float)w.x;
+                    bv[1][e] = (float)w.y;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < RB; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *(f32x4 *)(av[i] + 4 * h) = *(const f32x4u *)(ap[i] + k + 16 * h);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int kk = k + fk + koff(e);
+                bv[0][e] = kk < K ? ldw(bp, (size_t)kk * N) : 0.f;
+                bv[1][e] = kk < K ? ldw(bp, (size_t)kk * N + 1) : 0.f;
+#pragma unroll
+                for (int i = 0; i < RB; ++i) av[i][e] = kk < K ? ap[i][k + koff(e)] : 0.f;
+            }
+        }
+    };
+    f32x4 acc[RB][2];
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (wave < nkt) load(wave);
+    for (int t = wave; t < nkt; t += NW) {
+        u32x4 b[2][PB], f[RB][3];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bv[0][e] = late ? bv[1][e] : bv[0][e];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) parts8<PB>(bv[j], b[j]);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) parts8<3>(av[i], f[i]);
+        if (t + NW < nkt) load(t + NW);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) mma_parts<PB, 2>(acc[i], f[i], b);
+    }
+    /* [block][row 4 (l/16) + q][column l % 16] */
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) red[wave][2 * i + j][(4 * (lane >> 4) + q) * 16 + fr] = acc[i][j][q];
+    __syncthreads();
+    for (int o = tid; o < RB * 512; o += NW * 64) {
+        const int i = o >> 9, r = (o >> 5) & 15, c = o & 31;
+        const int m = m0 + 16 * i + r, n = n0 + c;
+        if (m >= M || n >= N) continue;
+        float v = red[0][2 * i + (c & 1)][r * 16 + (c >> 1)];
+        bool odd = odd_value(v);
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            const float x = red[w][2 * i + (c & 1)][r * 16 + (c >> 1)];
+            odd |= odd_value(x);
+            v += x;
+        }
+        if (odd) v = again<BT, false>(a.A, B, N, K, m, n, 0, K);
+        if (a.bias) v += a.bias[n];
+        a.C[(size_t)m * N + n] = v;
+    }
+}
+#define G2_XSKINNY(name, BT, RB) \
+    extern "C" __global__ __launch_bounds__(512) void name(const g2_gemm_args a) { xskinny_impl<BT, RB>(a); }
+G2_XSKINNY(g2k_xskinny1_f32, float, 1)
+G2_XSKINNY(g2k_xskinny1_f16, _Float16, 1)
+G2_XSKINNY(g2k_xskinny2_f32, float, 2)
+G2_XSKINNY(g2k_xskinny2_f16, _Float16, 2)

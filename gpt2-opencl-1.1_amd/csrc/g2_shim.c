@@ -10,6 +10,7 @@
  * main.c:537).  Every entry point validates shapes and pointers on the host
  * and returns a G2_E_* code instead of launching an out-of-range kernel.
  */
+#include <pthread.h>
 #include <stdarg.h>
 #include <stdio.h>
 #include <stdlib.h>
@@ -25,7 +26,8 @@ static const char *const g2_kernel_names[G2F_COUNT] = { G2_KERNEL_LIST(G2_NAME_E
 #undef G2_NAME_ENTRY
 
 /* Library scratch: split-K partials of g2_matvec (at most 64 splits of
- * G2_MAX_VOCAB columns) and the attention chunk partials of g2_attn_1q. */
+ * G2_MAX_VOCAB columns) and of g2_matmul (as many as fit), and the attention
+ * chunk partials of g2_attn_1q. */
 #define G2_MV_MAX_SPLITS 64
 #define G2_SCRATCH_FLOATS ((size_t)G2_MV_MAX_SPLITS * 65536)
 #define G2_ATTN_PART_FLOATS ((size_t)64 * G2_ATTN_MAX_CHUNKS * 66)
@@ -321,7 +323,58 @@ int g2_sync(void)
 static unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
 static int aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
 
-static int gemm_kn(int fid, const float *A, const void *B, const float *bias, float *C,
+/* The launches that write and read G.scratch are enqueued without another
+ * thread's between them; the stream then keeps their order. */
+static pthread_mutex_t g_scratch = PTHREAD_MUTEX_INITIALIZER;
+static void scratch_lock(void) { pthread_mutex_lock(&g_scratch); }
+static void scratch_unlock(void) { pthread_mutex_unlock(&g_scratch); }
+
+/* The GEMM kernel for M x N x K, by the estimated time (us) of each form
+ * (g2_matmul.hip): the direct form on 16- or 32-row tiles of 32 columns (K
+ * steps of 32 dealt to 8 waves), 64 x 64 tiles with K in ks splits added by a
+ * second launch, and 128 x 128 tiles.  A form's step costs its latency while
+ * the CUs hold at most one work-group each, and its throughput times the
+ * work-groups per CU beyond; up to nearly two, some CUs hold two and decide.
+ * The constants are fitted to MI355X times of 45 shapes (8..1024 rows, 258 to
+ * 50257 columns, K 267..6400, both weight types): the pick is the fastest
+ * form or within 10% of it on 41.  Examples, us of direct 16 / direct 32 / 64
+ * x 64 / its best split / 128 x 128: 96 x 768 x 3072: 14 / 20 / 69 / 16 / -;
+ * 512 x 1024 x 1024: 19 / 15 / 25 / 19 / 60; 256 x 1280 x 5120: 61 / 58 / 113
+ * / 34 / 276; 333 x 6400 x 1600: 117 / 97 / 74 / - / 94; 1024 x 50257 x 1600:
+ * - / - / 1200 / - / 880. */
+enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128 };
+
+static double xg_load(double per_cu) { return per_cu <= 1 ? per_cu : per_cu < 1.7 ? 1.7 : per_cu; }
+
+static int xg_pick(long M, long N, long K, int *splits)
+{
+    const double cus = g2i_cus(), steps = (double)((K + 31) / 32);
+    double best = 1e300;
+    int pick = XG_64;
+    *splits = 1;
+    for (int r = 1; r <= 2 && N >= 2; ++r) {
+        const double per_cu = xg_load((double)((N + 31) / 32) * (double)((M + 16 * r - 1) / (16 * r)) / cus);
+        const double t = r == 1 ? per_cu : 1.6 * per_cu, latency = r == 1 ? 1.0 : 1.4;
+        const double us = 3 + (double)(long)((steps + 7) / 8) * (t > latency ? t : latency);
+        if (us < best) { best = us; pick = r == 1 ? XG_DIRECT16 : XG_DIRECT32; }
+    }
+    const double tiles = (double)((N + 63) / 64) * (double)((M + 63) / 64), mn = (double)M * (double)N;
+    for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
+        if (ks > 1 && (ks * mn > (double)G2_SCRATCH_FLOATS || 2 * ks > steps)) break;
+        const double t = 0.3 + 0.42 * xg_load(tiles * ks / cus);
+        double us = 3 + steps / ks * (t > 0.7 ? t : 0.7);
+        if (ks > 1) us += 5 + (2 * ks + 1) * mn * sizeof(float) / 6e6;
+        if (us < best) { best = us; pick = XG_64; *splits = ks; }
+    }
+    if (N >= 2) {
+        const double t = 0.5 + 1.25 * ((double)((N + 127) / 128) * (double)((M + 127) / 128) / cus);
+        const double us = 3 + steps * (t > 1.85 ? t : 1.85);
+        if (us < best) { pick = XG_128; *splits = 1; }
+    }
+    return pick;
+}
+
+static int gemm_kn(int f16, const float *A, const void *B, const float *bias, float *C,
                    int M, int N, int K)
 {
     NEED_READY();
@@ -330,18 +383,34 @@ static int gemm_kn(int fid, const float *A, const void *B, const float *bias, fl
     g2_gemm_args a;
     memset(&a, 0, sizeof a);
     a.A = A; a.B = B; a.bias = bias; a.C = C; a.M = M; a.N = N; a.K = K;
-    return g2i_launch(fid, cdiv(N, 64), cdiv(M, 64), 256, &a);
+    switch (xg_pick(M, N, K, &a.ksplit)) {
+    case XG_DIRECT16:
+        return g2i_launch(f16 ? G2F_XSKINNY1_F16 : G2F_XSKINNY1_F32, cdiv(N, 32) * cdiv(M, 16), 1, 512, &a);
+    case XG_DIRECT32:
+        return g2i_launch(f16 ? G2F_XSKINNY2_F16 : G2F_XSKINNY2_F32, cdiv(N, 32) * cdiv(M, 32), 1, 512, &a);
+    case XG_128:
+        return g2i_launch(f16 ? G2F_XGEMM128_F16 : G2F_XGEMM128_F32, cdiv(N, 128) * cdiv(M, 128), 1, 256, &a);
+    }
+    const unsigned tiles = cdiv(N, 64) * cdiv(M, 64);
+    if (a.ksplit == 1) return g2i_launch(f16 ? G2F_XGEMM64_F16 : G2F_XGEMM64_F32, tiles, 1, 256, &a);
+    a.part = G.scratch;
+    const unsigned sum = cdiv((long)M * N, 1024);
+    scratch_lock();
+    int rc = g2i_launch(f16 ? G2F_XGEMM64_PART_F16 : G2F_XGEMM64_PART_F32, tiles, (unsigned)a.ksplit, 256, &a);
+    if (!rc) rc = g2i_launch(G2F_XGEMM_SUM, sum < 2048 ? sum : 2048, 1, 256, &a);
+    scratch_unlock();
+    return rc;
 }
 
 int g2_matmul(const float *A, const float *B, const float *bias, float *C, int M, int N, int K)
 {
-    return gemm_kn(G2F_GEMM_KN_F32, A, B, bias, C, M, N, K);
+    return gemm_kn(0, A, B, bias, C, M, N, K);
 }
 
 int g2_matmul_f16(const float *A, const uint16_t *B, const float *bias, float *C,
                   int M, int N, int K)
 {
-    return gemm_kn(G2F_GEMM_KN_F16, A, B, bias, C, M, N, K);
+    return gemm_kn(1, A, B, bias, C, M, N, K);
 }
 
 /* Split count for g2_matvec: about 2048 work-groups over the column tiles,

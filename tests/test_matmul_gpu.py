@@ -1,0 +1,71 @@
+"""g2_matmul's forms at the sizes where they can go wrong, and the values
+that bf16 parts cannot carry, against the CPU oracle's fp32 product.
+
+The sizes put each form (direct 16- and 32-row tiles, 64x64 tiles whole and
+in K splits, 128x128 tiles) on ragged edges: one row or column past a tile,
+odd column counts (a column pair that the last column begins), K below one
+step of 32, one past it, and splits that end in a partial step.
+"""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from parity import assert_close_bound, dot_bound
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(M, N, K, f16, seed):
+    r = np.random.default_rng(seed)
+    A = r.standard_normal((M, K)).astype(np.float32)
+    B = (0.02 * r.standard_normal((K, N))).astype(np.float32)
+    if f16:
+        B = B.astype(np.float16).astype(np.float32)
+    return A, B, r.standard_normal(N).astype(np.float32)
+
+
+def product(g2, A, B, bias, f16):
+    (M, K), N = A.shape, B.shape[1]
+    dC = g2.to_device(np.full(M * N + 64, 7.0, np.float32))
+    dB = g2.to_device(g2.convert_f16(B) if f16 else B)
+    g2.matmul(g2.to_device(A), dB, None if bias is None else g2.to_device(bias), dC, M, N, K, f16=f16)
+    got = dC.download(np.float32, M * N + 64)
+    assert (got[M * N:] == 7.0).all()  # nothing past the matrix
+    return got[:M * N].reshape(M, N)
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 1), (1, 1, 40), (17, 1, 65), (3, 2, 31),            # one column: no pairs
+    (16, 31, 32), (17, 33, 33), (15, 65, 257), (33, 97, 300),  # direct
+    (65, 129, 1000), (40, 300, 5007), (130, 257, 2049),        # direct or splits
+    (333, 1601, 96), (470, 2305, 70), (257, 5121, 1281),       # 64 x 64
+    (700, 8321, 70), (641, 12801, 32),                         # 128 x 128
+])
+def test_matmul_edges(g2, M, N, K, f16):
+    A, B, bias = operands(M, N, K, f16, M + N + K)
+    bound = dot_bound(np.abs(A).astype(np.float64), np.abs(B).astype(np.float64), K)
+    assert_close_bound(product(g2, A, B, bias, f16), oracle.matmul(A, B, bias, M, N, K), bound, what="matmul")
+    assert_close_bound(product(g2, A, B, None, f16), oracle.matmul(A, B, None, M, N, K), bound, what="no bias")
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("M,N,K", [(20, 70, 100), (70, 200, 4100), (470, 2305, 70), (700, 8321, 70)])
+def test_matmul_special_values(g2, M, N, K, f16):
+    """Rows with an infinity, a NaN, a value that rounds past bf16's largest,
+    and rows of magnitudes whose low parts bf16 cannot hold."""
+    A, B, _ = operands(M, N, K, f16, 5)
+    A[1, 7], A[2, 9], A[3, 11], A[M - 1, K - 1] = np.inf, np.nan, -np.inf, np.inf
+    A[4] *= np.float32(2.0) ** -112
+    A[5] = 0
+    A[6], A[7] = 0, 0
+    A[6, 3], A[7, K - 1] = 3.4e38, -3.4e38
+    B[:, 2] = 0.5
+    with np.errstate(all="ignore"):
+        ref = oracle.matmul(A, B, None, M, N, K)
+        got = product(g2, A, B, None, f16)
+        bound = dot_bound(np.abs(A).astype(np.float64), np.abs(B).astype(np.float64), K)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    fin = np.isfinite(ref)
+    np.testing.assert_array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
+    assert (np.abs(got[fin].astype(np.float64) - ref[fin]) <= bound[fin] + 1e-45).all()
