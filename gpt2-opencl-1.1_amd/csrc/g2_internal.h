@@ -51,6 +51,13 @@ extern "C" {
     X(XGEMM64_PART_F32, "g2k_xgemm64_part_f32")                               \
     X(XGEMM64_PART_F16, "g2k_xgemm64_part_f16")                               \
     X(XGEMM_SUM, "g2k_xgemm_sum")                                             \
+    X(XDUO_F32, "g2k_xduo_f32") X(XDUO_F16, "g2k_xduo_f16")                   \
+    X(XDUO_PART_F32, "g2k_xduo_part_f32")                                     \
+    X(XDUO_PART_F16, "g2k_xduo_part_f16")                                     \
+    X(XDUO_NK_PART, "g2k_xduo_nk_part")                                       \
+    X(XDUO_NK_PART64, "g2k_xduo_nk_part64")                                   \
+    X(XDUO_NK_GELU, "g2k_xduo_nk_gelu") X(XDUO_NK_RESID, "g2k_xduo_nk_resid") \
+    X(XDUO_NK_QKV, "g2k_xduo_nk_qkv")                                         \
     X(XSKINNY1_F32, "g2k_xskinny1_f32") X(XSKINNY1_F16, "g2k_xskinny1_f16")   \
     X(XSKINNY2_F32, "g2k_xskinny2_f32") X(XSKINNY2_F16, "g2k_xskinny2_f16")   \
     X(GEMM_NK_F32_STORE, "g2k_gemm_nk_f32_store")                             \
@@ -112,9 +119,9 @@ int g2i_launch3(int fid, unsigned gx, unsigned gy, unsigned gz, unsigned bx, voi
  * many as the buffer holds) */
 #define G2_PF_MAXSPLIT 5
 #define G2_PF_BIGSPLIT 8
-/* the fp32-weight prefill GEMM's split-K slices (floats; 8 MiB) and its
- * epilogue codes (g2k_sgemm_*, g2k_splitk_epi) */
-#define G2_SG_PART_FLOATS ((size_t)512 * 4096)
+/* the fp32-weight prefill GEMM's split-K slices (floats; 16 MiB) and its
+ * epilogue codes (g2k_sgemm_*, g2k_xduo_nk_*, g2k_splitk_epi) */
+#define G2_SG_PART_FLOATS ((size_t)256 * 128 * 128)
 #define G2_SG_GELU 1
 #define G2_SG_RESID 2
 #define G2_SG_QKV 3

@@ -89,7 +89,7 @@ typedef struct {
 } g2_skred_args;
 #define G2_SKLN_MAXN 2048
 #define G2_SKLN_MAXKS 8     /* slices g2k_splitk_resid_ln reads (ks <= this) */
-#define G2_SKLN_F32_MAXKS 8 /* slices g2k_splitk_resid_ln_f32 reads */
+#define G2_SKLN_F32_MAXKS 12 /* slices g2k_splitk_resid_ln_f32 reads */
 
 /* The split-K epilogue of the prefill GEMMs (g2k_splitk_epi): v[m,n] =
  * (sum over z < ks in order of part[z][m][n]) + bias[n], then epi 1 gelu
@@ -107,7 +107,7 @@ typedef struct {
     uint16_t *kh, *kl, *vth, *vtl; /* as in g2_gemm_args */
     uint16_t *Ch, *Cl;
 } g2_skepi_args;
-#define G2_SKEPI_MAXKS 8 /* slices g2k_splitk_epi reads */
+#define G2_SKEPI_MAXKS 12 /* slices g2k_splitk_epi reads */
 
 /* Reference-layout matvec, first pass: partial[split*N + n] = sum over the
  * split's contiguous k-range of A[k] B[k*N + n]; grid (column tiles, splits). */

@@ -129,11 +129,10 @@ __device__ __forceinline__ int tile_of(int w, int T)
  * Measured on MI355X (N(0,1) by N(0,0.02)): 1024 x 50257 x 1600 in 0.80 ms
  * with fp32 B (1.24 PFLOP/s of bf16 products, above the 1.14 that a library
  * bf16 product of 8192^3 reaches; the fp32-instruction kernel before: 3.35
- * ms), 0.66 ms with fp16 B (3.05).  Taken back: two steps in flight, two LDS
- * buffers, all fragments read ahead, raised wave priority (each within 5%),
- * and two groups of four waves that alternate between splitting and
- * multiplying on one tile (up to 30% faster at one tile per CU, 10% slower
- * with many). */
+ * ms), 0.66 ms with fp16 B (3.05).  With one work-group per CU a step takes
+ * 1.85 us, its conversions, LDS traffic and products one after the other
+ * (xduo_impl is for that).  Taken back: two steps in flight, two LDS buffers,
+ * all fragments read ahead, raised wave priority (each within 5%). */
 template <typename BT, bool BNK, int EPI, int BM, int BN>
 __device__ void xgemm_impl(const g2_gemm_args &a)
 {
@@ -375,6 +374,315 @@ G2K void g2k_xgemm_sum(const g2_gemm_args a)
         }
     }
 }
+
+/* One tile per CU: BM x 128 outputs per work-group of two groups of 2 x 2
+ * waves, each with an LDS buffer and every other K step of 32.  The groups
+ * alternate: while one multiplies, the other splits its next step's values
+ * into their parts and stores them, so a SIMD holds one wave of each and its
+ * matrix core works through the other's conversions; the groups' sums are
+ * added at the end.  Staging as in xgemm_impl.  Epilogues as g2_gemm_args
+ * describes them; GEPI_PARTIAL: gridDim.y splits of whole steps.  A step
+ * takes 1.02 us (0.75 at BM 64; 1.85 in xgemm_impl at one work-group per CU),
+ * of which the products alone 0.79 and the reads in front of them 0.2; W
+ * [N,K] of n_embd 1280 by 256 rows: fc 24 us in three splits (the fp32
+ * instruction, whole: 47), fc2 25 in twelve (34), qkv 20 in four (30). */
+template <typename BT, bool BNK, int EPI, int BM>
+__device__ void xduo_impl(const g2_gemm_args &a)
+{
+    using namespace xg;
+    constexpr int BN = 128, RA = BM / 64, IB = BM / 32, HB = IB / 2;
+    constexpr int PB = sizeof(BT) == 4 ? 3 : 2;
+    constexpr int SA = BM * 16 + 64, SB = BN * 16 + (BNK ? 64 : 0); /* octet plane strides, bytes */
+    constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
+    __shared__ __attribute__((aligned(16))) unsigned char lds[2 * ST];
+    const int tid = threadIdx.x & 255, lane = tid & 63;
+    const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = w8 >> 2, wave = w8 & 3, wm = wave >> 1, wn = wave & 1;
+    const int M = a.M, N = a.N, K = a.K;
+    const int nmb = (M + BM - 1) / BM;
+    const int tile = tile_of(blockIdx.x, gridDim.x);
+    const int m0 = (tile % nmb) * BM, n0 = (tile / nmb) * BN;
+    const int nkt = (K + 31) >> 5, ks = gridDim.y;
+    const int s0 = (int)(((long)nkt * blockIdx.y) / ks), s1 = (int)(((long)nkt * (blockIdx.y + 1)) / ks);
+    const int sf = min(s1, K >> 5); /* steps s0 .. sf - 1 are whole */
+    const BT *B = (const BT *)a.B;
+    unsigned char *st = lds + g * ST;
+
+    const int ar = tid >> 2, ao = (tid & 3) * 4;
+    const float *ap[RA];
+#pragma unroll
+    for (int i = 0; i < RA; ++i) ap[i] = a.A + (size_t)min(m0 + ar + 64 * i, M - 1) * K + ao;
+    const int bc = tid & 63, bo = wave;
+    const bool late = !BNK && n0 + bc * 2 + 1 == N;
+    const BT *bp[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        bp[i] = BNK ? B + (size_t)min(n0 + ar + 64 * i, N - 1) * K + ao : B + min(n0 + bc * 2, N - 2) + i;
+
+    float av[RA][8], bv[2][8];
+    /* whole step t (past the last one: that one again, unused) */
+    auto load = [&](int t) {
+        const int k = min(t, sf - 1) * 32;
+#pragma unroll
+        for (int i = 0; i < RA; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) *(f32x4 *)(av[i] + 4 * h) = *(const f32x4u *)(ap[i] + k + 16 * h);
+        if constexpr (BNK) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) *(f32x4 *)(bv[i] + 4 * h) = *(const f32x4u *)((const float *)bp[i] + k + 16 * h);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const size_t o = (size_t)(k + 4 * bo + koff(e)) * N;
+                if constexpr (sizeof(BT) == 4) {
+                    const f32x2 w = *(const f32x2u *)((const float *)bp[0] + o);
+                    bv[0][e] = w.x;
+                    bv[1][e] = w.y;
+                } else { /* both columns' bits; widened in store() */
+                    bv[0][e] = __builtin_bit_cast(float, *(const f16x2u *)((const _Float16 *)bp[0] + o));
+                }
+            }
+        }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int i = 0; i < RA; ++i) {
+            u32x4 p[3];
+            parts8<3>(av[i], p);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *(u32x4 *)(st + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
+        }
+        float b[2][8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if constexpr (!BNK && sizeof(BT) == 2) {
+                const f16x2u w = __builtin_bit_cast(f16x2u, bv[0][e]);
+                b[0][e] = (float)w.x;
+                b[1][e] = (float)w.y;
+            } else {
+                b[0][e] = bv[0][e];
+                b[1][e] = bv[1][e];
+            }
+            if constexpr (!BNK) b[0][e] = late ? b[1][e] : b[0][e];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            u32x4 p[PB];
+            parts8<PB>(b[i], p);
+#pragma unroll
+            for (int q = 0; q < PB; ++q)
+                *(u32x4 *)(st + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
+        }
+    };
+
+    f32x4 acc[IB][4];
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    /* column block j of the wave: positions 16 j of its half (BNK), or blocks
+     * 0, 1 of the even columns and 2, 3 of the odd ones */
+    const unsigned char *arow = st + (lane >> 4) * SA + (wm * (BM / 2) + (lane & 15)) * 16;
+    const unsigned char *brow = st + 12 * SA + (lane >> 4) * SB + (wn * (BNK ? 64 : 32) + (lane & 15)) * 16;
+    auto multiply = [&]() {
+        u32x4 f[IB][3], b[4][PB];
+        auto read_a = [&](int q) {
+#pragma unroll
+            for (int i = 0; i < IB; ++i) f[i][q] = *(const u32x4 *)(arow + 4 * q * SA + i * 256);
+        };
+        auto read_b = [&](int q) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                b[j][q] = *(const u32x4 *)(brow + 4 * q * SB + (BNK ? j * 256 : (j & 1) * 256 + (j >> 1) * 1024));
+        };
+        auto products = [&](int p, int q) {
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = mma(f[i][p], b[j][q], acc[i][j]);
+        };
+        /* a part's reads are issued one or two products ahead of its use */
+#define XG_KEEP_ORDER __builtin_amdgcn_sched_barrier(0)
+        read_b(0);
+        read_a(2);
+        read_a(1);
+        XG_KEEP_ORDER;
+        __builtin_amdgcn_s_setprio(1);
+        products(2, 0);
+        XG_KEEP_ORDER;
+        read_a(0);
+        XG_KEEP_ORDER;
+        products(1, 0);
+        XG_KEEP_ORDER;
+        read_b(1);
+        XG_KEEP_ORDER;
+        products(0, 0);
+        XG_KEEP_ORDER;
+        if constexpr (PB == 3) read_b(PB - 1);
+        XG_KEEP_ORDER;
+        products(1, 1);
+        products(0, 1);
+        if constexpr (PB == 3) {
+            XG_KEEP_ORDER;
+            products(0, PB - 1);
+        }
+        XG_KEEP_ORDER;
+        __builtin_amdgcn_s_setprio(0);
+#undef XG_KEEP_ORDER
+    };
+
+    /* group g takes whole steps s0 + g, s0 + g + 2, ...; both groups pass the
+     * same number of barriers */
+    if (sf > s0) {
+        const int n = (sf - s0 + 1) >> 1;
+        load(s0 + g);
+        if (g) __syncthreads();
+        for (int i = 0; i < n; ++i) {
+            const int t = s0 + g + 2 * i;
+            store();
+            load(t + 2);
+            __syncthreads();
+            if (t < sf) multiply();
+            __syncthreads();
+        }
+        if (!g) __syncthreads();
+    }
+    if (sf < s1 && !g) { /* the last, partial step: zeros past K */
+        const int k = sf * 32;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+#pragma unroll
+            for (int i = 0; i < RA; ++i) av[i][e] = k + ao + koff(e) < K ? ap[i][k + koff(e)] : 0.f;
+            const int kk = k + koff(e) + (BNK ? ao : 4 * bo);
+            const size_t o = BNK ? (size_t)(k + koff(e)) : (size_t)kk * N;
+            if constexpr (BNK || sizeof(BT) == 4) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) bv[i][e] = kk < K ? ldw(bp[i], o) : 0.f;
+            } else {
+                bv[0][e] = kk < K ? __builtin_bit_cast(float, *(const f16x2u *)((const _Float16 *)bp[0] + o)) : 0.f;
+            }
+        }
+        store();
+    }
+    __syncthreads();
+    if (sf < s1 && !g) multiply();
+    __syncthreads();
+
+    /* each group hands half of its row blocks to the other and finishes the
+     * other half: group 0 blocks 0 .. HB - 1, group 1 the rest */
+    f32x4 sum[HB][4];
+    {
+        f32x4 *x = (f32x4 *)lds + (g * 4 + wave) * (HB * 256) + lane;
+        const f32x4 *y = (const f32x4 *)lds + ((1 - g) * 4 + wave) * (HB * 256) + lane;
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 lo = acc[i][j], hi = acc[i + HB][j];
+                f32x4 give;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    give[q] = g ? lo[q] : hi[q];
+                    sum[i][j][q] = g ? hi[q] : lo[q];
+                }
+                x[(i * 4 + j) * 64] = give;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[i][j] += y[(i * 4 + j) * 64];
+    }
+
+    /* output (row, column) of value (i, j, q) */
+    auto om = [&](int i, int q) { return m0 + wm * (BM / 2) + (g * HB + i) * 16 + 4 * (lane >> 4) + q; };
+    auto on = [&](int j) {
+        return BNK ? n0 + wn * 64 + j * 16 + (lane & 15) : n0 + 2 * (wn * 32 + (j & 1) * 16 + (lane & 15)) + (j >> 1);
+    };
+    unsigned odd = 0;
+#pragma unroll
+    for (int c = 0; c < 16 * HB; ++c)
+        if (odd_value(sum[c >> 4][(c >> 2) & 3][c & 3])) odd |= 1u << c;
+    while (odd) {
+        const int c = __ffs(odd) - 1;
+        odd &= odd - 1;
+        const int m = om(c >> 4, c & 3), n = on((c >> 2) & 3);
+        const float v = m < M && n < N ? again<BT, BNK>(a.A, B, N, K, m, n, s0 * 32, min(s1 * 32, K)) : 0.f;
+#pragma unroll
+        for (int d = 0; d < 16 * HB; ++d)
+            if (c == d) sum[d >> 4][(d >> 2) & 3][d & 3] = v;
+    }
+
+    /* every load of the epilogue before its first store */
+    if constexpr (EPI != GEPI_PARTIAL) {
+        float bias[4], rv[HB][4][4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bias[j] = a.bias ? a.bias[min(on(j), N - 1)] : 0.f;
+        if constexpr (EPI == GEPI_RESID) {
+#pragma unroll
+            for (int i = 0; i < HB; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        rv[i][j][q] = a.C[(size_t)min(om(i, q), M - 1) * N + min(on(j), N - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (a.bias) sum[i][j][q] += bias[j];
+                    if constexpr (EPI == GEPI_RESID) sum[i][j][q] += rv[i][j][q];
+                    if constexpr (EPI == GEPI_GELU) sum[i][j][q] = gelu_f(sum[i][j][q]);
+                }
+    }
+    if constexpr (EPI == GEPI_QKV) {
+        const qkv_dst d = qkv_of(a);
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (on(j) < N) qkv_store4(d, om(i, 0), M, on(j), sum[i][j]);
+        return;
+    }
+    float *C = EPI == GEPI_PARTIAL ? a.part + (size_t)blockIdx.y * M * N : a.C;
+#pragma unroll
+    for (int i = 0; i < HB; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int m = om(i, q);
+            if (m >= M) continue;
+            if constexpr (!BNK) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int n = on(j);
+                    float *c = C + (size_t)m * N + n;
+                    if (n + 1 < N) *(f32x2u *)c = (f32x2){sum[i][j][q], sum[i][j + 2][q]};
+                    else if (n < N) *c = sum[i][j][q];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (on(j) < N) C[(size_t)m * N + on(j)] = sum[i][j][q];
+            }
+        }
+}
+
+#define G2_XDUO(name, BT, BNK, EPI, BM) \
+    extern "C" __global__ __launch_bounds__(512, 2) void name(const g2_gemm_args a) { xduo_impl<BT, BNK, EPI, BM>(a); }
+G2_XDUO(g2k_xduo_nk_part, float, true, GEPI_PARTIAL, 128)
+G2_XDUO(g2k_xduo_nk_part64, float, true, GEPI_PARTIAL, 64)
+G2_XDUO(g2k_xduo_nk_gelu, float, true, GEPI_GELU, 128)
+G2_XDUO(g2k_xduo_nk_resid, float, true, GEPI_RESID, 128)
+G2_XDUO(g2k_xduo_nk_qkv, float, true, GEPI_QKV, 128)
+G2_XDUO(g2k_xduo_f32, float, false, GEPI_STORE, 128)
+G2_XDUO(g2k_xduo_f16, _Float16, false, GEPI_STORE, 128)
+G2_XDUO(g2k_xduo_part_f32, float, false, GEPI_PARTIAL, 128)
+G2_XDUO(g2k_xduo_part_f16, _Float16, false, GEPI_PARTIAL, 128)
 
 /* Few tiles: a work-group of 8 waves takes one 16 RB x 32 tile, the K steps
  * dealt to the waves in turn, their sums added in wave order through LDS.  No

@@ -1005,34 +1005,72 @@ static int prefill_resid(g2_model *m, const float *A, const uint16_t *Ah, const 
     return rc;
 }
 
-/* The fp32-weight prefill GEMM (g2k_sgemm_*, K % 32 == 0) with epilogue
- * epi (G2_SG_GELU, _RESID or _QKV as g2_gemm_args describes them).  A
- * prompt too short to fill the machine with 64x64 tiles gets split-K
- * slices (at most 8, each at least two K steps of 32), summed in order with
- * the bias and the epilogue by g2k_splitk_epi: as many as keep the
- * work-groups within 256, or within 512 for a K of 64 steps or more (fc2).
- * Measured at 64..512 rows and n_embd 768..1280, this picks the best or
- * within 10% of the best of 1..8 slices for every GEMM.  ks slices of at
- * most 64 ceil(M/64) x 64 ceil(N/64) floats each fit G2_SG_PART_FLOATS:
- * ks * tiles <= 512.  With ln_g (a residual epilogue followed by a
- * LayerNorm: proj -> ln_2, fc2 -> the next ln_1) the slice sum is fused
- * with that LayerNorm (g2k_splitk_resid_ln_f32, writing m->ln_out) and
- * *ln_done is set; otherwise the caller runs it. */
+/* The form of the fp32-weight prefill GEMM and its K splits, by estimated
+ * time (us): 64 x 64 tiles on the fp32 matrix instruction (g2k_sgemm_*), or,
+ * for more than 64 rows, 64 x 128 or 128 x 128 tiles in bf16 parts
+ * (g2k_xduo_nk_*, one work-group per CU; the 64-row form with splits only).
+ * A split writes its partial tile and a second launch adds them with the
+ * epilogue.  Up to 64 rows the weights' bytes bound all forms and sgemm is
+ * the fastest or equal; us of the GEMM alone as sgemm / 64 x 128 / 128 x 128
+ * with their splits, n_embd 1280: fc 100 rows 28.8 / 17.2 / 17.3, 256 rows
+ * 47.5 / 32.4 / 24.0, 512 rows 72.3 / 55.3 / 46.7; fc2 26.3 / 18.0 / 22.6,
+ * 33.5 / 28.1 / 24.8, 60.4 / 47.8 / 38.9; proj 256 rows 12.0 / 11.2 / 12.6. */
+enum { SG_FORM_F32, SG_FORM_DUO64, SG_FORM_DUO128 };
+
+static int sg_pick(int M, int N, int K, int *splits)
+{
+    const int nk = K / 32;
+    const double cus = g2i_cus(), slice = (double)M * N * sizeof(float);
+    const unsigned t64 = cdivu(N, 64) * cdivu(M, 64);
+    /* as many splits as keep sgemm's work-groups within 256, or within 512
+     * for a K of 64 steps or more (fc2), each of at least two steps */
+    const unsigned target = nk >= 64 ? 512 : 256;
+    int ks = t64 >= target ? 1 : (int)(target / t64);
+    if (ks > 8) ks = 8;
+    if (ks > nk / 2) ks = nk / 2 > 1 ? nk / 2 : 1;
+    *splits = ks;
+    if (M <= 64) return SG_FORM_F32;
+    const double write = 1 / 2.6e6, read = 1 / 5e6; /* us per byte of a slice */
+    const double load = 0.6 * t64 * ks / cus;
+    double best = 3 + (double)nk / ks * (load > 0.68 ? load : 0.68) + (ks > 1 ? 3 + ks * slice * (write + read) : 0);
+    int pick = SG_FORM_F32;
+    for (int form = SG_FORM_DUO64; form <= SG_FORM_DUO128; ++form) {
+        const int rows = form == SG_FORM_DUO64 ? 64 : 128;
+        const unsigned tiles = cdivu(N, 128) * cdivu(M, (unsigned)rows);
+        for (int k = form == SG_FORM_DUO64 ? 2 : 1; k <= G2_SKEPI_MAXKS && 2 * k <= nk; ++k) {
+            if (k > 1 && tiles * (unsigned)k > cus) break;
+            const double us = 4 + (double)nk / k * (rows == 64 ? 0.75 : 1.02) * ceil(tiles * k / cus) +
+                              (k > 1 ? 3 + k * slice * (write + read) : 0);
+            if (us < best) { best = us; pick = form; *splits = k; }
+        }
+    }
+    return pick;
+}
+
+/* The fp32-weight prefill GEMM (K % 32 == 0) with epilogue epi (G2_SG_GELU,
+ * _RESID or _QKV as g2_gemm_args describes them), in sg_pick's form.  Splits
+ * are summed in order with the bias and the epilogue by g2k_splitk_epi; with
+ * ln_g (a residual epilogue followed by a LayerNorm: proj -> ln_2, fc2 -> the
+ * next ln_1) the sum is fused with that LayerNorm (g2k_splitk_resid_ln_f32,
+ * writing m->ln_out) and *ln_done is set; otherwise the caller runs it. */
 static int prefill_sgemm(g2_model *m, int epi, g2_gemm_args *g, const float *ln_g, const float *ln_b, int *ln_done)
 {
     *ln_done = 0;
-    const unsigned gx = cdivu(g->N, 64), gy = cdivu(g->M, 64), tiles = gx * gy;
-    const int nk = g->K / 32;
-    const unsigned target = nk >= 64 ? 512 : 256;
-    int ks = tiles >= target ? 1 : (int)(target / tiles);
-    if (ks > 8) ks = 8;
-    if (ks > nk / 2) ks = nk / 2 > 1 ? nk / 2 : 1;
-    if ((size_t)ks * g->M * g->N > G2_SG_PART_FLOATS) return g2i_err(G2_E_LIMIT, "split-K slices exceed the buffer");
+    int ks;
+    const int form = sg_pick(g->M, g->N, g->K, &ks), duo = form != SG_FORM_F32;
+    const unsigned gx = cdivu(g->N, 64), gy = cdivu(g->M, 64);
+    const unsigned tiles = cdivu(g->N, 128) * cdivu(g->M, form == SG_FORM_DUO64 ? 64 : 128);
+    if ((size_t)ks * g->M * g->N > G2_SG_PART_FLOATS && ks > 1)
+        return g2i_err(G2_E_LIMIT, "split-K slices exceed the buffer");
+    if (ks == 1 && duo)
+        return g2i_launch(epi == G2_SG_GELU ? G2F_XDUO_NK_GELU : epi == G2_SG_RESID ? G2F_XDUO_NK_RESID : G2F_XDUO_NK_QKV,
+                          tiles, 1, 512, g);
     if (ks == 1)
         return g2i_launch(epi == G2_SG_GELU ? G2F_SGEMM_GELU : epi == G2_SG_RESID ? G2F_SGEMM_RESID : G2F_SGEMM_QKV,
                           gx, gy, 256, g);
     g->part = m->pf_part;
-    int rc = g2i_launch3(G2F_SGEMM_PARTIAL, gx, gy, (unsigned)ks, 256, g);
+    int rc = duo ? g2i_launch(form == SG_FORM_DUO64 ? G2F_XDUO_NK_PART64 : G2F_XDUO_NK_PART, tiles, (unsigned)ks, 512, g)
+                 : g2i_launch3(G2F_SGEMM_PARTIAL, gx, gy, (unsigned)ks, 256, g);
     if (!rc && epi == G2_SG_RESID && ln_g && g->N <= G2_SKLN_MAXN && g->N % 4 == 0 && ks <= G2_SKLN_F32_MAXKS) {
         g2_skred_args r = { m->pf_part, g->bias, g->C, g->M, g->N, ks, ln_g, ln_b, NULL, NULL, m->ln_out };
         *ln_done = 1;

@@ -10,6 +10,7 @@
  * main.c:537).  Every entry point validates shapes and pointers on the host
  * and returns a G2_E_* code instead of launching an out-of-range kernel.
  */
+#include <math.h>
 #include <pthread.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -331,8 +332,9 @@ static void scratch_unlock(void) { pthread_mutex_unlock(&g_scratch); }
 
 /* The GEMM kernel for M x N x K, by the estimated time (us) of each form
  * (g2_matmul.hip): the direct form on 16- or 32-row tiles of 32 columns (K
- * steps of 32 dealt to 8 waves), 64 x 64 tiles with K in ks splits added by a
- * second launch, and 128 x 128 tiles.  A form's step costs its latency while
+ * steps of 32 dealt to 8 waves), 64 x 64 tiles and 128 x 128 tiles of two
+ * alternating wave groups, both with K in ks splits added by a second launch,
+ * and 128 x 128 tiles of two and more work-groups per CU.  A form's step costs its latency while
  * the CUs hold at most one work-group each, and its throughput times the
  * work-groups per CU beyond; up to nearly two, some CUs hold two and decide.
  * The constants are fitted to MI355X times of 45 shapes (8..1024 rows, 258 to
@@ -342,7 +344,7 @@ static void scratch_unlock(void) { pthread_mutex_unlock(&g_scratch); }
  * 512 x 1024 x 1024: 19 / 15 / 25 / 19 / 60; 256 x 1280 x 5120: 61 / 58 / 113
  * / 34 / 276; 333 x 6400 x 1600: 117 / 97 / 74 / - / 94; 1024 x 50257 x 1600:
  * - / - / 1200 / - / 880. */
-enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128 };
+enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128, XG_DUO };
 
 static double xg_load(double per_cu) { return per_cu <= 1 ? per_cu : per_cu < 1.7 ? 1.7 : per_cu; }
 
@@ -369,7 +371,14 @@ static int xg_pick(long M, long N, long K, int *splits)
     if (N >= 2) {
         const double t = 0.5 + 1.25 * ((double)((N + 127) / 128) * (double)((M + 127) / 128) / cus);
         const double us = 3 + steps * (t > 1.85 ? t : 1.85);
-        if (us < best) { pick = XG_128; *splits = 1; }
+        if (us < best) { best = us; pick = XG_128; *splits = 1; }
+        const double tiles = (double)((N + 127) / 128) * (double)((M + 127) / 128);
+        for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
+            if (ks > 1 && (ks * mn > (double)G2_SCRATCH_FLOATS || 2 * ks > steps || tiles * ks > cus)) break;
+            double duo = 4 + steps / ks * 1.05 * ceil(tiles * ks / cus);
+            if (ks > 1) duo += 5 + ks * mn * sizeof(float) * (1 / 2.6e6 + 1 / 6e6);
+            if (duo < best) { best = duo; pick = XG_DUO; *splits = ks; }
+        }
     }
     return pick;
 }
@@ -383,7 +392,8 @@ static int gemm_kn(int f16, const float *A, const void *B, const float *bias, fl
     g2_gemm_args a;
     memset(&a, 0, sizeof a);
     a.A = A; a.B = B; a.bias = bias; a.C = C; a.M = M; a.N = N; a.K = K;
-    switch (xg_pick(M, N, K, &a.ksplit)) {
+    const int pick = xg_pick(M, N, K, &a.ksplit), duo = pick == XG_DUO;
+    switch (pick) {
     case XG_DIRECT16:
         return g2i_launch(f16 ? G2F_XSKINNY1_F16 : G2F_XSKINNY1_F32, cdiv(N, 32) * cdiv(M, 16), 1, 512, &a);
     case XG_DIRECT32:
@@ -391,12 +401,15 @@ static int gemm_kn(int f16, const float *A, const void *B, const float *bias, fl
     case XG_128:
         return g2i_launch(f16 ? G2F_XGEMM128_F16 : G2F_XGEMM128_F32, cdiv(N, 128) * cdiv(M, 128), 1, 256, &a);
     }
-    const unsigned tiles = cdiv(N, 64) * cdiv(M, 64);
-    if (a.ksplit == 1) return g2i_launch(f16 ? G2F_XGEMM64_F16 : G2F_XGEMM64_F32, tiles, 1, 256, &a);
+    const unsigned tile = duo ? 128 : 64, tiles = cdiv(N, tile) * cdiv(M, tile), threads = duo ? 512 : 256;
+    const int whole = duo ? (f16 ? G2F_XDUO_F16 : G2F_XDUO_F32) : (f16 ? G2F_XGEMM64_F16 : G2F_XGEMM64_F32);
+    const int part = duo ? (f16 ? G2F_XDUO_PART_F16 : G2F_XDUO_PART_F32)
+                         : (f16 ? G2F_XGEMM64_PART_F16 : G2F_XGEMM64_PART_F32);
+    if (a.ksplit == 1) return g2i_launch(whole, tiles, 1, threads, &a);
     a.part = G.scratch;
     const unsigned sum = cdiv((long)M * N, 1024);
     scratch_lock();
-    int rc = g2i_launch(f16 ? G2F_XGEMM64_PART_F16 : G2F_XGEMM64_PART_F32, tiles, (unsigned)a.ksplit, 256, &a);
+    int rc = g2i_launch(part, tiles, (unsigned)a.ksplit, threads, &a);
     if (!rc) rc = g2i_launch(G2F_XGEMM_SUM, sum < 2048 ? sum : 2048, 1, 256, &a);
     scratch_unlock();
     return rc;

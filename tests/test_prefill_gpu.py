@@ -127,3 +127,20 @@ def test_prefill_attention_helpers(g2, monkeypatch, E, NH, P):
     m.free()
     np.testing.assert_allclose(lg_h, lg_n, rtol=1e-5, atol=1e-5)
     assert np.array_equal(lg_h2, lg_f2), "second prompt differs from a fresh model's"
+
+
+@pytest.mark.parametrize("E,NH,P", [(768, 12, 65), (768, 12, 129), (1280, 20, 100), (1280, 20, 257), (768, 12, 1000)])
+def test_prefill_f32_forms(g2, E, NH, P):
+    """fp32 weights at prompts where the GEMM's forms and K splits change
+    (64 x 128 and 128 x 128 tiles in bf16 parts, with and without splits,
+    one row past a tile, 1000 rows: whole, above the slice buffer) against
+    the oracle: every logit within 2e-4 (measured below 1e-5)."""
+    cfg = g2.make_config(2, E, NH, vocab_size=2048)
+    w = g2.synth_weights(cfg, SEED, affine=True)
+    prompt = random_prompt(P, cfg.vocab_size, 400 + P)
+    ref = oracle.Model(cfg, w).generate(prompt, 1, logit_steps=1)[2][0]
+    m = g2.Model.from_host(cfg, w, g2.F32, g2.PATH_FUSED)
+    m.prefill(prompt)
+    got = m.logits().copy()
+    m.free()
+    np.testing.assert_allclose(got, ref, rtol=2e-4, atol=2e-4)
