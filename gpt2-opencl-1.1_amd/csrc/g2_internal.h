@@ -33,9 +33,9 @@ extern "C" {
 
 /* Kernel table: index -> symbol name in the gfx950 code object. */
 #define G2_KERNEL_LIST(X)                                                     \
-    X(MVKN_F32, "g2k_mvkn_f32") X(MVKN_F32_S, "g2k_mvkn_f32_s")               \
-    X(MVKN_F16, "g2k_mvkn_f16") X(MVKN_F16_S, "g2k_mvkn_f16_s")               \
-    X(MVSK_F32, "g2k_mvsk_f32") X(MVSK_F16, "g2k_mvsk_f16")                   \
+    X(MATVEC4_F32, "g2k_matvec4_f32") X(MATVEC4_F16, "g2k_matvec4_f16")       \
+    X(MATVEC8_F32, "g2k_matvec8_f32") X(MATVEC8_F16, "g2k_matvec8_f16")       \
+    X(MATVEC16_F32, "g2k_matvec16_f32") X(MATVEC16_F16, "g2k_matvec16_f16")   \
     X(REDUCE, "g2k_reduce") X(LAYERNORM, "g2k_layernorm")                     \
     X(ADD, "g2k_add") X(GELU, "g2k_gelu")                                     \
     X(EMBED_F32, "g2k_embed_f32") X(EMBED_F16, "g2k_embed_f16")               \

@@ -109,24 +109,19 @@ typedef struct {
 } g2_skepi_args;
 #define G2_SKEPI_MAXKS 12 /* slices g2k_splitk_epi reads */
 
-/* Reference-layout matvec, first pass: partial[split*N + n] = sum over the
- * split's contiguous k-range of A[k] B[k*N + n]; grid (column tiles, splits). */
+/* Reference-layout matvec B[K,N]: slice s of nslice sums k = s, s + nslice,
+ * ... (math.cl:229-246) to out[s*N + n], then + bias, + residual, GELU (each
+ * optional; NULL, NULL, 0 with slices).  Grid (column groups, nslice). */
 typedef struct {
     const float *A;
     const void *B;
-    float *partial;
-    int N, K, rows_per_split;
-} g2_mvkn_args;
+    float *out;
+    const float *bias;
+    const float *residual;
+    int N, K, nslice, apply_gelu;
+} g2_matvec_args;
 
-/* Split-K partials with the reference's strided slices (math.cl:229-246). */
-typedef struct {
-    const float *A;
-    const void *B;
-    float *partial;
-    int N, K, kslice;
-} g2_mvsk_args;
-
-/* reduce_partial (math.cl:249-280), also the second pass of g2_matvec. */
+/* reduce_partial (math.cl:249-280). */
 typedef struct {
     const float *partial;
     const float *bias;

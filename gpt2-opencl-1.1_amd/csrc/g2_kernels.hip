@@ -93,106 +93,109 @@ template <> __device__ __forceinline__ float ldw<_Float16>(const _Float16 *p, si
  * Reference operators
  * ==================================================================== */
 
-/* ---- matvec, reference layout B[K,N] (launch_matvec, main.c:1554-1576) ---
- * Pass 1: grid (ceil(N/256), splits).  Each work-group owns 256 columns (4 per
- * lane) and a contiguous k-range of rows_per_split rows; wave w takes rows
- * k0+w, k0+w+4, ...; the four wave sums are added in wave order into
- * partial[split][n].  Pass 2 is g2k_reduce. */
-template <typename WT, bool VEC>
-__device__ void mvkn_impl(const g2_mvkn_args &a)
+/* ---- matvec, reference layout B[K,N] (launch_matvec, main.c:1554-1576), and
+ * matvec4_sk (math.cl:229-246): slice s = blockIdx.y of nslice sums k = s, s +
+ * nslice, ... into out[s][N]; without slices (nslice 1) bias, residual and
+ * GELU follow, in the same launch.
+ *
+ * A work-group of 1024 threads takes CL * V columns over all of its k: CL
+ * lanes of V columns (16 bytes, at any alignment) side by side, 1024 / CL k
+ * rows at a time, so that even a small matrix is one burst of loads per CU
+ * and no sum crosses work-groups.  A thread's sums are added over the lanes
+ * of its wave that share its columns, then over the 16 waves in order.  The
+ * last lane of a ragged N takes the last V columns (loads stay inside the
+ * row; it writes only those that no other lane has).  Bounded by the launch
+ * and a few load latencies for small matrices, by HBM for large ones: 50257 x
+ * 768 takes 37 us with fp32 weights (4.2 TB/s; 70 in two launches before),
+ * 20 with fp16 (47); 768 x 3072 in four slices 7 (85: one lane per four
+ * columns walked its slice alone).  Eight rows ahead instead of four: 39 and
+ * 23 us for 50257 x 768, no gain elsewhere. */
+template <typename WT, int CL>
+__device__ void matvec_impl(const g2_matvec_args &a)
 {
-    __shared__ float red[4][256];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int col = blockIdx.x * 256 + lane * 4;
-    const int k0 = blockIdx.y * a.rows_per_split;
-    const int k1 = min(a.K, k0 + a.rows_per_split);
-    const WT *B = (const WT *)a.B;
-    float acc0 = 0.f, acc1 = 0.f, acc2 = 0.f, acc3 = 0.f;
-    if (VEC && col + 3 < a.N) {
-        int k = k0 + wave;
-        for (; k + 12 < k1; k += 16) {
-            float av[4];
-            float bv[4][4];
+    constexpr int V = 16 / sizeof(WT), RG = 1024 / CL;
+    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    typedef _Float16 f16x8u __attribute__((ext_vector_type(8), aligned(2)));
+    __shared__ float red[16][CL * V];
+    const int tid = threadIdx.x, cl = tid & (CL - 1), rg = tid / CL;
+    const int N = a.N, K = a.K, ns = a.nslice;
+    const int col = (blockIdx.x * CL + cl) * V, base = min(col, max(N - V, 0));
+    const WT *B = (const WT *)a.B + base;
+    float acc[V];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const size_t base = (size_t)(k + 4 * u) * a.N + col;
-                av[u] = a.A[k + 4 * u];
-                if constexpr (sizeof(WT) == 4) {
-                    const f32x4 w = *(const f32x4 *)((const float *)B + base);
-                    bv[u][0] = w.x; bv[u][1] = w.y; bv[u][2] = w.z; bv[u][3] = w.w;
-                } else {
-                    const f16x4 w = *(const f16x4 *)((const _Float16 *)B + base);
-                    bv[u][0] = (float)w.x; bv[u][1] = (float)w.y;
-                    bv[u][2] = (float)w.z; bv[u][3] = (float)w.w;
-                }
-            }
+    for (int e = 0; e < V; ++e) acc[e] = 0.f;
+    auto row = [&](int k, float (&w)[V]) {
+        const WT *p = B + (size_t)k * N;
+        if (N < V) { /* one vector would leave the row */
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                acc0 = fmaf(av[u], bv[u][0], acc0);
-                acc1 = fmaf(av[u], bv[u][1], acc1);
-                acc2 = fmaf(av[u], bv[u][2], acc2);
-                acc3 = fmaf(av[u], bv[u][3], acc3);
-            }
+            for (int e = 0; e < V; ++e) w[e] = e < N ? (float)p[e] : 0.f;
+        } else if constexpr (sizeof(WT) == 4) {
+            const f32x4 v = *(const f32x4u *)p;
+#pragma unroll
+            for (int e = 0; e < V; ++e) w[e] = v[e];
+        } else {
+            const f16x8 v = *(const f16x8u *)p;
+#pragma unroll
+            for (int e = 0; e < V; ++e) w[e] = (float)v[e];
         }
-        for (; k < k1; k += 4) {
-            const size_t base = (size_t)k * a.N + col;
-            const float av = a.A[k];
-            acc0 = fmaf(av, ldw(B, base + 0), acc0);
-            acc1 = fmaf(av, ldw(B, base + 1), acc1);
-            acc2 = fmaf(av, ldw(B, base + 2), acc2);
-            acc3 = fmaf(av, ldw(B, base + 3), acc3);
+    };
+    constexpr int U = 4;
+    const long step = (long)RG * ns;
+    long k = blockIdx.y + (long)rg * ns;
+    for (; k + (U - 1) * step < K; k += U * step) {
+        float x[U], w[U][V];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            x[u] = a.A[k + u * step];
+            row((int)(k + u * step), w[u]);
         }
-    } else {
-        for (int k = k0 + wave; k < k1; k += 4) {
-            const size_t base = (size_t)k * a.N;
-            const float av = a.A[k];
-            if (col + 0 < a.N) acc0 = fmaf(av, ldw(B, base + col + 0), acc0);
-            if (col + 1 < a.N) acc1 = fmaf(av, ldw(B, base + col + 1), acc1);
-            if (col + 2 < a.N) acc2 = fmaf(av, ldw(B, base + col + 2), acc2);
-            if (col + 3 < a.N) acc3 = fmaf(av, ldw(B, base + col + 3), acc3);
-        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < V; ++e) acc[e] = fmaf(x[u], w[u][e], acc[e]);
     }
-    red[wave][lane * 4 + 0] = acc0;
-    red[wave][lane * 4 + 1] = acc1;
-    red[wave][lane * 4 + 2] = acc2;
-    red[wave][lane * 4 + 3] = acc3;
+    {
+        float x[U - 1], w[U - 1][V];
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (k + u * step < K) {
+                x[u] = a.A[k + u * step];
+                row((int)(k + u * step), w[u]);
+            }
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (k + u * step < K)
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[e] = fmaf(x[u], w[u][e], acc[e]);
+    }
+#pragma unroll
+    for (int o = CL; o < 64; o <<= 1)
+#pragma unroll
+        for (int e = 0; e < V; ++e) acc[e] += __shfl_xor(acc[e], o);
+    if ((tid & 63) < CL)
+#pragma unroll
+        for (int e = 0; e < V; ++e) red[tid >> 6][cl * V + e] = acc[e];
     __syncthreads();
-    const int t = threadIdx.x, n = blockIdx.x * 256 + t;
-    if (n < a.N)
-        a.partial[(size_t)blockIdx.y * a.N + n] =
-            ((red[0][t] + red[1][t]) + red[2][t]) + red[3][t];
+    if (tid >= CL * V) return;
+    /* thread -> lane tid / V, element tid % V */
+    const int c0 = (blockIdx.x * CL + tid / V) * V, n = min(c0, max(N - V, 0)) + tid % V;
+    if (n < c0 || n >= N) return;
+    float v = red[0][tid];
+#pragma unroll
+    for (int w = 1; w < 16; ++w) v += red[w][tid];
+    if (a.bias) v += a.bias[n];
+    if (a.residual) v += a.residual[n];
+    if (a.apply_gelu) v = gelu_f(v);
+    a.out[(size_t)blockIdx.y * N + n] = v;
 }
-
-G2K void g2k_mvkn_f32(const g2_mvkn_args a) { mvkn_impl<float, true>(a); }
-G2K void g2k_mvkn_f32_s(const g2_mvkn_args a) { mvkn_impl<float, false>(a); }
-G2K void g2k_mvkn_f16(const g2_mvkn_args a) { mvkn_impl<_Float16, true>(a); }
-G2K void g2k_mvkn_f16_s(const g2_mvkn_args a) { mvkn_impl<_Float16, false>(a); }
-
-/* ---- matvec4_sk (math.cl:229-246): slice s sums k = s, s+kslice, ... ------
- * grid (ceil(N/4 / 256), kslice); one thread per (4 columns, slice). */
-template <typename WT>
-__device__ void mvsk_impl(const g2_mvsk_args &a)
-{
-    const int c4 = blockIdx.x * 256 + threadIdx.x;
-    const int s = blockIdx.y;
-    const int N4 = a.N >> 2;
-    if (c4 >= N4 || s >= a.kslice) return;
-    const WT *B = (const WT *)a.B;
-    float acc0 = 0.f, acc1 = 0.f, acc2 = 0.f, acc3 = 0.f;
-    for (int k = s; k < a.K; k += a.kslice) {
-        const size_t base = (size_t)k * a.N + (size_t)c4 * 4;
-        const float av = a.A[k];
-        acc0 = fmaf(av, ldw(B, base + 0), acc0);
-        acc1 = fmaf(av, ldw(B, base + 1), acc1);
-        acc2 = fmaf(av, ldw(B, base + 2), acc2);
-        acc3 = fmaf(av, ldw(B, base + 3), acc3);
-    }
-    float *p = a.partial + (size_t)s * a.N + (size_t)c4 * 4;
-    p[0] = acc0; p[1] = acc1; p[2] = acc2; p[3] = acc3;
-}
-
-G2K void g2k_mvsk_f32(const g2_mvsk_args a) { mvsk_impl<float>(a); }
-G2K void g2k_mvsk_f16(const g2_mvsk_args a) { mvsk_impl<_Float16>(a); }
+#define G2_MATVEC(name, WT, CL) \
+    extern "C" __global__ __launch_bounds__(1024) void name(const g2_matvec_args a) { matvec_impl<WT, CL>(a); }
+G2_MATVEC(g2k_matvec4_f32, float, 4)
+G2_MATVEC(g2k_matvec8_f32, float, 8)
+G2_MATVEC(g2k_matvec16_f32, float, 16)
+G2_MATVEC(g2k_matvec4_f16, _Float16, 4)
+G2_MATVEC(g2k_matvec8_f16, _Float16, 8)
+G2_MATVEC(g2k_matvec16_f16, _Float16, 16)
 
 /* ---- reduce_partial (math.cl:249-280): slices added in order, then bias,
  * residual, GELU.  residual may alias C (each n is read then written by the

@@ -26,11 +26,10 @@ extern const unsigned char g2_hsaco_end[];
 static const char *const g2_kernel_names[G2F_COUNT] = { G2_KERNEL_LIST(G2_NAME_ENTRY) };
 #undef G2_NAME_ENTRY
 
-/* Library scratch: split-K partials of g2_matvec (at most 64 splits of
- * G2_MAX_VOCAB columns) and of g2_matmul (as many as fit), and the attention
- * chunk partials of g2_attn_1q. */
-#define G2_MV_MAX_SPLITS 64
-#define G2_SCRATCH_FLOATS ((size_t)G2_MV_MAX_SPLITS * 65536)
+/* Library scratch: K slices of g2_matvec (at most 8 of 65536 columns) and of
+ * g2_matmul (as many as fit), and the attention chunk partials of
+ * g2_attn_1q. */
+#define G2_SCRATCH_FLOATS ((size_t)64 * 65536)
 #define G2_ATTN_PART_FLOATS ((size_t)64 * G2_ATTN_MAX_CHUNKS * 66)
 
 static struct {
@@ -426,20 +425,30 @@ int g2_matmul_f16(const float *A, const uint16_t *B, const float *bias, float *C
     return gemm_kn(1, A, B, bias, C, M, N, K);
 }
 
-/* Split count for g2_matvec: about 2048 work-groups over the column tiles,
- * at least 8 rows per split, at most G2_MV_MAX_SPLITS. */
-static int mv_splits(int N, int K, int *rows_per_split)
+/* Column lanes of a matvec work-group (CL lanes of 16 bytes): 16 (256 bytes of
+ * a row per work-group, the best of HBM's rate), fewer where that leaves under
+ * 160 work-groups for the chip; four at least (64 bytes; two were slower).
+ * us with 4 / 8 / 16: 6400 x 1600 fp32 (400 / 200 / 100 work-groups) 17.6 /
+ * 11.0 / 13.6, fp16 (200 / 100 / 50) 9.1 / 10.7 / 17.6; 50257 x 768 fp32 63 /
+ * 44 / 37. */
+static int matvec_launch(int f16, g2_matvec_args *a)
 {
-    const int tiles = (int)cdiv(N, 256);
-    int s = (int)cdiv(2048, tiles);
-    if (s > G2_MV_MAX_SPLITS) s = G2_MV_MAX_SPLITS;
-    if (s > (K + 7) / 8) s = (K + 7) / 8;
-    if (s < 1) s = 1;
-    int rps = (int)cdiv(K, s);
-    *rows_per_split = rps;
-    return (int)cdiv(K, rps);
+    const unsigned v = f16 ? 8 : 4;
+    int shape = 2; /* CL = 4 << shape */
+    while (shape > 0 && cdiv(a->N, (4u << shape) * v) * (unsigned)a->nslice < 160) --shape;
+    const int fid = (f16 ? G2F_MATVEC4_F16 : G2F_MATVEC4_F32) + 2 * shape;
+    return g2i_launch(fid, cdiv(a->N, (4u << shape) * v), (unsigned)a->nslice, 1024, a);
 }
 
+static int overlap(const void *p, size_t np, const void *q, size_t nq)
+{
+    return (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
+}
+
+/* One launch, except: a tall narrow matrix (its few work-groups would walk
+ * over 128 KB each) goes in slices to the scratch, added by a second launch
+ * (1600 x 6400 fp32 11 us + the launch against 20, 768 x 3072 7 against 13);
+ * so does a product into memory that holds its operands. */
 static int matvec_any(int f16, const float *A, const void *B, const float *bias,
                       const float *res, float *C, int N, int K, int gelu)
 {
@@ -447,16 +456,22 @@ static int matvec_any(int f16, const float *A, const void *B, const float *bias,
     if (!A || !B || !C) return g2i_err(G2_E_ARG, "g2_matvec: NULL buffer");
     if (N <= 0 || K <= 0) return g2i_err(G2_E_ARG, "g2_matvec: N and K must be positive");
     if (N > 65536) return g2i_err(G2_E_LIMIT, "g2_matvec: N=%d above 65536", N);
-    int rps;
-    const int splits = mv_splits(N, K, &rps);
-    const int vec = (N % 4) == 0 && aligned(B, f16 ? 8 : 16);
-    const int fid = f16 ? (vec ? G2F_MVKN_F16 : G2F_MVKN_F16_S)
-                        : (vec ? G2F_MVKN_F32 : G2F_MVKN_F32_S);
-    g2_mvkn_args a = { A, B, G.scratch, N, K, rps };
-    int rc = g2i_launch(fid, cdiv(N, 256), (unsigned)splits, 256, &a);
-    if (rc) return rc;
-    g2_reduce_args r = { G.scratch, bias, res, C, N, splits, gelu ? 1 : 0 };
-    return g2i_launch(G2F_REDUCE, cdiv(N, 256), 1, 256, &r);
+    const unsigned narrow = cdiv(N, f16 ? 32 : 16);
+    unsigned slices = 1;
+    if (K > 2048 && narrow < 160) slices = cdiv(256, narrow) < 8 ? cdiv(256, narrow) : 8;
+    const size_t nc = (size_t)N * sizeof(float);
+    if (slices == 1 && !overlap(C, nc, A, (size_t)K * sizeof(float)) &&
+        !overlap(C, nc, B, (size_t)N * K * (f16 ? 2 : 4))) {
+        g2_matvec_args a = { A, B, C, bias, res, N, K, 1, gelu ? 1 : 0 };
+        return matvec_launch(f16, &a);
+    }
+    g2_matvec_args a = { A, B, G.scratch, NULL, NULL, N, K, (int)slices, 0 };
+    g2_reduce_args r = { G.scratch, bias, res, C, N, (int)slices, gelu ? 1 : 0 };
+    scratch_lock();
+    int rc = matvec_launch(f16, &a);
+    if (!rc) rc = g2i_launch(G2F_REDUCE, cdiv(N, 256), 1, 256, &r);
+    scratch_unlock();
+    return rc;
 }
 
 int g2_matvec(const float *A, const float *B, const float *bias, const float *residual,
@@ -478,8 +493,8 @@ static int matvec_sk_any(int f16, const float *A, const void *B, float *partial,
     if (!A || !B || !partial) return g2i_err(G2_E_ARG, "g2_matvec_sk: NULL buffer");
     if (N <= 0 || K <= 0 || (N & 3)) return g2i_err(G2_E_ARG, "g2_matvec_sk: N must be a positive multiple of 4");
     if (kslice < 1 || kslice > 8) return g2i_err(G2_E_ARG, "g2_matvec_sk: kslice %d not in 1..8", kslice);
-    g2_mvsk_args a = { A, B, partial, N, K, kslice };
-    return g2i_launch(f16 ? G2F_MVSK_F16 : G2F_MVSK_F32, cdiv(N / 4, 256), (unsigned)kslice, 256, &a);
+    g2_matvec_args a = { A, B, partial, NULL, NULL, N, K, kslice, 0 };
+    return matvec_launch(f16, &a);
 }
 
 int g2_matvec_sk(const float *A, const float *B, float *partial, int N, int K, int kslice)

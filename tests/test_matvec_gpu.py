@@ -1,0 +1,63 @@
+"""g2_matvec and g2_matvec_sk at the sizes where their launches can go wrong:
+rows shorter than one 16-byte vector, columns past the last whole vector or
+column group, K below and above the rows that a work-group takes at once, the
+column-lane choices, the sliced form of tall narrow matrices, operands at odd
+addresses and results that overlap an operand; against the CPU oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle
+from parity import assert_close_bound, dot_bound
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(N, K, f16, seed):
+    r = np.random.default_rng(seed)
+    A, B = r.standard_normal(K).astype(np.float32), (0.02 * r.standard_normal((K, N))).astype(np.float32)
+    B = B.astype(np.float16).astype(np.float32) if f16 else B
+    return A, B, r.standard_normal(N).astype(np.float32), r.standard_normal(N).astype(np.float32)
+
+
+def exact(A, B, bias, res):
+    return A.astype(np.float64) @ B.astype(np.float64) + bias + res
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("N,K", [(1, 1), (3, 300), (7, 257), (9, 1023), (33, 64), (17, 2049), (515, 6400), (1601, 3000),
+                                 (2563, 100), (10243, 65), (20487, 33)])
+def test_matvec_edges(g2, N, K, f16):
+    A, B, bias, res = operands(N, K, f16, N + K)
+    dA, dbias = g2.to_device(A), g2.to_device(bias)
+    raw = g2.convert_f16(B) if f16 else B
+    bound = dot_bound(np.abs(A), np.abs(B), K)
+    for shift in (0, raw.itemsize):  # B at a vector's address, then one element past it
+        dB = g2.to_device(np.concatenate([np.zeros(shift // raw.itemsize, raw.dtype), raw.ravel()]))
+        dC = g2.to_device(np.concatenate([res, np.full(8, 7.0, np.float32)]))
+        g2.matvec(dA, dB.offset(shift), dbias, dC, dC, N, K, f16=f16)
+        got = dC.download(np.float32, N + 8)
+        assert (got[N:] == 7.0).all()  # nothing past the vector
+        assert_close_bound(got[:N], exact(A, B, bias, res), bound, what="matvec")
+
+
+@pytest.mark.parametrize("N,K", [(768, 768), (100, 2500)])
+def test_matvec_in_place(g2, N, K):
+    """C in A's memory: the product reads all of A first."""
+    A, B, bias, res = operands(N, K, False, 9)
+    dA = g2.to_device(A)
+    g2.matvec(dA, g2.to_device(B), g2.to_device(bias), g2.to_device(res), dA, N, K)
+    assert_close_bound(dA.download(np.float32, N), exact(A, B, bias, res), dot_bound(np.abs(A), np.abs(B), K), what="in place")
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("N,K,ks", [(4, 3, 8), (12, 2, 5), (36, 1025, 3), (1028, 700, 7), (2564, 6400, 8)])
+def test_matvec_sk_edges(g2, N, K, ks, f16):
+    A, B, _, _ = operands(N, K, f16, N + K + ks)
+    dP = g2.to_device(np.full(ks * N + 8, 7.0, np.float32))
+    g2.matvec_sk(g2.to_device(A), g2.to_device(g2.convert_f16(B) if f16 else B), dP, N, K, ks, f16=f16)
+    got = dP.download(np.float32, ks * N + 8)
+    assert (got[ks * N:] == 7.0).all()
+    ref = oracle.matvec4_sk(A, B, N, K, ks)
+    for s in range(ks):
+        bound = dot_bound(np.abs(A[s::ks]), np.abs(B[s::ks]), max(len(A[s::ks]), 1))
+        assert_close_bound(got[s * N:(s + 1) * N], ref[s], bound, what=f"slice {s}")
