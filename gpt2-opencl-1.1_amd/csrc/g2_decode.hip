@@ -156,6 +156,112 @@ extern "C" __global__ __launch_bounds__(64) void g2k_attn_merge(const g2_attn1q_
     a.out[h * 64 + d] = acc / L;
 }
 
+/* Up to 256 positions (G2_ATTN_GROUP chunks) in one launch: grid NH, 256
+ * threads per chunk, each as g2k_attn_part but with every load (queries, keys,
+ * values) issued at the start, the chunks merged through LDS.  Bounded by the
+ * launch and one memory latency: 12 or 25 heads of 64 positions 3.9 us a call,
+ * of 256 5.0, against 6.5 in two launches.  Beyond 256 positions two launches
+ * stay: one work-group reads 64 KB of keys and values per chunk, and four
+ * chunks to a work-group with a merge behind were slower (25 heads of 1024: 8.9
+ * us a call against 8.5), as was merging in the same launch by the work-group
+ * that counts a head's last chunk in (an agent-scope store, atomic and load,
+ * three memory round trips: 9.7). */
+template <bool VEC>
+__device__ void attn_short_impl(const g2_attn1q_args &a)
+{
+    __shared__ float reds[G2_ATTN_GROUP][16][65];
+    __shared__ float prs[G2_ATTN_GROUP][64];
+    __shared__ float stat[G2_ATTN_GROUP][2];
+    const int grp = threadIdx.x >> 8, tid = threadIdx.x & 255, h = blockIdx.x;
+    const int T = attn_T(a), nch = (T + 63) >> 6;
+    if (h >= a.NH || nch > (int)(blockDim.x >> 8)) return;
+    const int j0 = grp * 64, S = a.S, D = a.D;
+    float (&red)[16][65] = reds[grp];
+    float *pr = prs[grp];
+    const int q4 = tid & 15, g4 = tid >> 4; /* scores: position quad, dim group; values: dim quad, position group */
+    float q[4], k[4][4], v[4][4];
+    {
+        const int j = j0 + 4 * q4;
+        const float *kb = a.k_cache + (size_t)(h * 64 + 4 * g4) * S;
+        const float *vb = a.v_cache + h * 64 + 4 * q4;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            if (VEC && j + 3 < S) {
+                const f32x4 x = j < T ? *(const f32x4 *)(kb + (size_t)d * S + j) : (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) k[d][e] = x[e];
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) k[d][e] = j + e < T ? kb[(size_t)d * S + j + e] : 0.f;
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) q[d] = a.q[h * 64 + 4 * g4 + d];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int jv = j0 + 4 * g4 + e;
+            if (VEC) {
+                const f32x4 x = jv < T ? *(const f32x4 *)(vb + (size_t)jv * D) : (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int f = 0; f < 4; ++f) v[e][f] = x[f];
+            } else {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) v[e][f] = jv < T ? vb[(size_t)jv * D + f] : 0.f;
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float s = 0.f;
+#pragma unroll
+        for (int d = 0; d < 4; ++d) s = fmaf(q[d], k[d][e], s);
+        red[g4][4 * q4 + e] = s;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        const bool ok = j0 + tid < T;
+        float s = 0.f;
+#pragma unroll
+        for (int g = 0; g < 16; ++g) s += red[g][tid];
+        s *= a.scale;
+        const float mx = wave_max(ok ? s : -INFINITY);
+        const float p = ok ? expf(s - mx) : 0.f;
+        const float sum = wave_sum(p);
+        pr[tid] = p;
+        if (tid == 0) {
+            stat[grp][0] = mx;
+            stat[grp][1] = sum;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {
+        float o = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (j0 + 4 * g4 + e < T) o = fmaf(pr[4 * g4 + e], v[e][f], o);
+        red[g4][4 * q4 + f] = o;
+    }
+    __syncthreads();
+    /* wave 0: the chunks in order, dim tid */
+    if (threadIdx.x >= 64) return;
+    float M = stat[0][0], L = 0.f, acc = 0.f;
+    for (int g = 1; g < nch; ++g) M = fmaxf(M, stat[g][0]);
+    for (int g = 0; g < nch; ++g) {
+        float o = 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o += reds[g][i][tid];
+        const float w = expf(stat[g][0] - M);
+        L = fmaf(stat[g][1], w, L);
+        acc = fmaf(o, w, acc);
+    }
+    a.out[h * 64 + tid] = acc / L;
+}
+#define G2_ATTN_SHORT(name, VEC) \
+    extern "C" __global__ __launch_bounds__(256 * G2_ATTN_GROUP) void name(const g2_attn1q_args a) { attn_short_impl<VEC>(a); }
+G2_ATTN_SHORT(g2k_attn_short, true)
+G2_ATTN_SHORT(g2k_attn_short_s, false)
+
 /* ======================================================================
  * Packed matvec rows
  * ==================================================================== */

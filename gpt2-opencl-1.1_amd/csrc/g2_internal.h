@@ -33,9 +33,9 @@ extern "C" {
 
 /* Kernel table: index -> symbol name in the gfx950 code object. */
 #define G2_KERNEL_LIST(X)                                                     \
-    X(MATVEC4_F32, "g2k_matvec4_f32") X(MATVEC4_F16, "g2k_matvec4_f16")       \
-    X(MATVEC8_F32, "g2k_matvec8_f32") X(MATVEC8_F16, "g2k_matvec8_f16")       \
-    X(MATVEC16_F32, "g2k_matvec16_f32") X(MATVEC16_F16, "g2k_matvec16_f16")   \
+    X(MVSK4_F32, "g2k_mvsk_f32_4") X(MVSK4_F16, "g2k_mvsk_f16_4")       \
+    X(MVSK8_F32, "g2k_mvsk_f32_8") X(MVSK8_F16, "g2k_mvsk_f16_8")       \
+    X(MVSK16_F32, "g2k_mvsk_f32_16") X(MVSK16_F16, "g2k_mvsk_f16_16")   \
     X(REDUCE, "g2k_reduce") X(LAYERNORM, "g2k_layernorm")                     \
     X(ADD, "g2k_add") X(GELU, "g2k_gelu")                                     \
     X(EMBED_F32, "g2k_embed_f32") X(EMBED_F16, "g2k_embed_f16")               \
@@ -43,6 +43,7 @@ extern "C" {
     X(ATTN_SOFTMAX, "g2k_attn_softmax") X(ATTN_OUT, "g2k_attn_out")           \
     X(ATTN_PART, "g2k_attn_part") X(ATTN_PART_S, "g2k_attn_part_s")           \
     X(ATTN_MERGE, "g2k_attn_merge") X(ARGMAX_MERGE, "g2k_argmax_merge")       \
+    X(ATTN_SHORT, "g2k_attn_short") X(ATTN_SHORT_S, "g2k_attn_short_s")       \
     G2_ROWS_LIST(X, STORE, "store") G2_ROWS_LIST(X, LN_QKV, "ln_qkv")         \
     G2_ROWS_LIST(X, RESID, "resid") G2_ROWS_LIST(X, LN_GELU, "ln_gelu")       \
     G2_ROWS_LIST(X, LN_ARGMAX, "ln_argmax")                                   \
@@ -140,7 +141,8 @@ int g2i_device_alloc(void **p, size_t bytes);
 int g2i_rows_launch(int fid_f32_64, int f16, g2_rows_args *a);
 /* Work-groups g2i_rows_launch uses for N rows of K (0 if K is invalid). */
 unsigned g2i_rows_grid(int N, int K, int f16);
-/* Single-query attention: partials over `chunks` key chunks, then merge. */
+/* Single-query attention over `chunks` key chunks: one launch up to
+ * G2_ATTN_GROUP (a length given by the caller), else partials, then merge. */
 int g2i_attn_launch(g2_attn1q_args *a, unsigned chunks);
 
 /* host helpers (g2_host.c) */

@@ -193,8 +193,10 @@ typedef struct {
 } g2_attnout_args;
 
 /* Single-query attention, head dim 64, split over 64-position key chunks
- * (partials kernel) and merged by a second kernel.  T = T_fixed if > 0,
- * else state[G2S_POS] + 1.  part: [NH][max_chunks][2 + 64] floats. */
+ * (partials kernel) and merged by a second kernel, or (g2k_attn_short) up to
+ * G2_ATTN_GROUP chunks in one work-group per head.  T = T_fixed if > 0, else
+ * state[G2S_POS] + 1.  part: [NH][max_chunks][2 + 64] floats. */
+#define G2_ATTN_GROUP 4
 typedef struct {
     const float *q;
     const float *k_cache;

@@ -190,12 +190,12 @@ __device__ void matvec_impl(const g2_matvec_args &a)
 }
 #define G2_MATVEC(name, WT, CL) \
     extern "C" __global__ __launch_bounds__(1024) void name(const g2_matvec_args a) { matvec_impl<WT, CL>(a); }
-G2_MATVEC(g2k_matvec4_f32, float, 4)
-G2_MATVEC(g2k_matvec8_f32, float, 8)
-G2_MATVEC(g2k_matvec16_f32, float, 16)
-G2_MATVEC(g2k_matvec4_f16, _Float16, 4)
-G2_MATVEC(g2k_matvec8_f16, _Float16, 8)
-G2_MATVEC(g2k_matvec16_f16, _Float16, 16)
+G2_MATVEC(g2k_mvsk_f32_4, float, 4)
+G2_MATVEC(g2k_mvsk_f32_8, float, 8)
+G2_MATVEC(g2k_mvsk_f32_16, float, 16)
+G2_MATVEC(g2k_mvsk_f16_4, _Float16, 4)
+G2_MATVEC(g2k_mvsk_f16_8, _Float16, 8)
+G2_MATVEC(g2k_mvsk_f16_16, _Float16, 16)
 
 /* ---- reduce_partial (math.cl:249-280): slices added in order, then bias,
  * residual, GELU.  residual may alias C (each n is read then written by the
@@ -399,62 +399,100 @@ G2K void g2k_split_kv(const g2_splitkv_args a)
     a.v_cache[(size_t)pos * a.D + d] = a.qkv[(size_t)i * 3 * a.D + 2 * a.D + d];
 }
 
-/* ---- attn_scores_1q (math.cl:388-412); grid (NH, ceil(T/256)) ---------- */
+/* ---- attn_scores_1q (math.cl:388-412); grid (NH, ceil(T/64)): a thread has
+ * one position and every fourth dim, 16 loads in flight; the four dim groups
+ * (waves) are added in order. */
 G2K void g2k_attn_scores(const g2_scores_args a)
 {
-    const int h = blockIdx.x, j = blockIdx.y * 256 + threadIdx.x;
-    if (h >= a.NH || j >= a.T) return;
+    __shared__ float red[4][64];
+    const int h = blockIdx.x, lane = threadIdx.x & 63, g = threadIdx.x >> 6;
+    const int j = blockIdx.y * 64 + lane, jc = min(j, a.T - 1);
     const float *q = a.qkv + a.q_base + (size_t)h * a.DH;
-    const float *kc = a.k_cache + (size_t)h * a.DH * a.S + j;
+    const float *kc = a.k_cache + (size_t)h * a.DH * a.S + jc;
     float s = 0.f;
-    for (int k = 0; k < a.DH; ++k) s = fmaf(q[k], kc[(size_t)k * a.S], s);
-    a.scores[(size_t)h * a.S + j] = s * a.scale;
+    for (int k0 = g; k0 < a.DH; k0 += 64) {
+        float x[16], y[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int k = k0 + 4 * u;
+            x[u] = k < a.DH ? q[k] : 0.f;
+            y[u] = k < a.DH ? kc[(size_t)k * a.S] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 16; ++u) s = fmaf(x[u], y[u], s);
+    }
+    red[g][lane] = s;
+    __syncthreads();
+    if (g == 0 && j < a.T)
+        a.scores[(size_t)h * a.S + j] = (((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]) * a.scale;
 }
 
 /* ---- attn_softmax_1q (math.cl:415-456): one work-group per head, in place,
- * row stride G2_MAX_SEQ. */
+ * row stride G2_MAX_SEQ; the row stays in registers between its one read and
+ * its one write. */
 G2K void g2k_attn_softmax(const g2_softmax_args a)
 {
+    constexpr int V = G2_KV_MAX_SEQ / 256;
     __shared__ float red4[4];
     const int h = blockIdx.x;
     if (h >= a.NH) return;
     float *row = a.scores + (size_t)h * G2_KV_MAX_SEQ;
-    float mx = -1e30f;
-    for (int j = threadIdx.x; j < a.T; j += 256) mx = fmaxf(mx, row[j]);
+    float x[V], mx = -1e30f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int j = threadIdx.x + 256 * i;
+        x[i] = j < a.T ? row[j] : -1e30f;
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) mx = fmaxf(mx, x[i]);
     mx = wave_max(mx);
     if ((threadIdx.x & 63) == 0) red4[threadIdx.x >> 6] = mx;
     __syncthreads();
     const float m = fmaxf(fmaxf(red4[0], red4[1]), fmaxf(red4[2], red4[3]));
     __syncthreads();
     float s = 0.f;
-    for (int j = threadIdx.x; j < a.T; j += 256) {
-        const float e = expf(row[j] - m);
-        row[j] = e;
-        s += e;
-    }
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+        if ((int)threadIdx.x + 256 * i < a.T) {
+            x[i] = expf(x[i] - m);
+            s += x[i];
+        }
     const float inv = 1.0f / block_sum(s, red4);
-    for (int j = threadIdx.x; j < a.T; j += 256) row[j] *= inv;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        const int j = threadIdx.x + 256 * i;
+        if (j < a.T) row[j] = x[i] * inv;
+    }
 }
 
-/* ---- attn_out_1q (math.cl:459-476): grid ceil(D/64), block 1024: lane d of
- * the block's 64 dims, 16 waves split j (j = wave, wave+16, ...). */
+/* ---- attn_out_1q (math.cl:459-476): grid ceil(D/16), block 1024: 16 dims x
+ * 64 positions at a time (j = row, row + 64, ...), four ahead; the 64 sums of
+ * a dim are added over a wave's four rows, then over the 16 waves in order. */
 extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout_args a)
 {
-    __shared__ float red[16][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int d = blockIdx.x * 64 + lane;
+    __shared__ float red[16][16];
+    const int tid = threadIdx.x, d = blockIdx.x * 16 + (tid & 15), dc = min(d, a.D - 1);
+    const float *srow = a.scores + (size_t)(dc / a.DH) * G2_KV_MAX_SEQ;
     float o = 0.f;
-    if (d < a.D) {
-        const float *srow = a.scores + (size_t)(d / a.DH) * G2_KV_MAX_SEQ;
-        for (int j = wave; j < a.T; j += 16)
-            o = fmaf(srow[j], a.v_cache[(size_t)j * a.D + d], o);
+    for (int j0 = tid >> 4; j0 < a.T; j0 += 256) {
+        float p[4], v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int j = j0 + 64 * u;
+            p[u] = j < a.T ? srow[j] : 0.f;
+            v[u] = j < a.T ? a.v_cache[(size_t)j * a.D + dc] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) o = fmaf(p[u], v[u], o);
     }
-    red[wave][lane] = o;
+    o += __shfl_xor(o, 16);
+    o += __shfl_xor(o, 32);
+    if ((tid & 63) < 16) red[tid >> 6][tid & 15] = o;
     __syncthreads();
-    if (wave == 0 && d < a.D) {
+    if (tid < 16 && d < a.D) {
         float s = 0.f;
 #pragma unroll
-        for (int w = 0; w < 16; ++w) s += red[w][lane];
+        for (int w = 0; w < 16; ++w) s += red[w][tid];
         a.out[a.out_base + d] = s;
     }
 }

@@ -436,7 +436,7 @@ static int matvec_launch(int f16, g2_matvec_args *a)
     const unsigned v = f16 ? 8 : 4;
     int shape = 2; /* CL = 4 << shape */
     while (shape > 0 && cdiv(a->N, (4u << shape) * v) * (unsigned)a->nslice < 160) --shape;
-    const int fid = (f16 ? G2F_MATVEC4_F16 : G2F_MATVEC4_F32) + 2 * shape;
+    const int fid = (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + 2 * shape;
     return g2i_launch(fid, cdiv(a->N, (4u << shape) * v), (unsigned)a->nslice, 1024, a);
 }
 
@@ -583,7 +583,7 @@ int g2_attn_scores_1q(const float *qkv, const float *k_cache, float *scores, int
         NH * DH > D || q_base < 0)
         return g2i_err(G2_E_ARG, "g2_attn_scores_1q: bad sizes");
     g2_scores_args a = { qkv, k_cache, scores, q_base, T_kv, D, DH, NH, max_seq, scale };
-    return g2i_launch(G2F_ATTN_SCORES, (unsigned)NH, cdiv(T_kv, 256), 256, &a);
+    return g2i_launch(G2F_ATTN_SCORES, (unsigned)NH, cdiv(T_kv, 64), 256, &a);
 }
 
 int g2_attn_softmax_1q(float *scores, int T_kv, int NH)
@@ -603,7 +603,7 @@ int g2_attn_out_1q(const float *scores, const float *v_cache, float *out, int T_
     if (T_kv <= 0 || T_kv > G2_MAX_SEQ || D <= 0 || DH <= 0 || out_base < 0)
         return g2i_err(G2_E_ARG, "g2_attn_out_1q: bad sizes");
     g2_attnout_args a = { scores, v_cache, out, T_kv, D, DH, out_base };
-    return g2i_launch(G2F_ATTN_OUT, cdiv(D, 64), 1, 1024, &a);
+    return g2i_launch(G2F_ATTN_OUT, cdiv(D, 16), 1, 1024, &a);
 }
 
 int g2_attn_1q(const float *qkv, const float *k_cache, const float *v_cache, float *out,
@@ -655,8 +655,12 @@ int g2_attn_1q_noalloc(const float *qkv, const float *k_cache, const float *v_ca
 int g2i_attn_launch(g2_attn1q_args *a, unsigned chunks)
 {
     const int vec = a->S % 4 == 0 && a->D % 4 == 0 && aligned(a->k_cache, 16) && aligned(a->v_cache, 16);
+    if (chunks <= G2_ATTN_GROUP && a->T_fixed > 0)
+        return g2i_launch(vec ? G2F_ATTN_SHORT : G2F_ATTN_SHORT_S, (unsigned)a->NH, 1, 256 * chunks, a);
+    scratch_lock();
     int rc = g2i_launch(vec ? G2F_ATTN_PART : G2F_ATTN_PART_S, (unsigned)a->NH, chunks, 256, a);
     if (!rc) rc = g2i_launch(G2F_ATTN_MERGE, (unsigned)a->NH, 1, 64, a);
+    scratch_unlock();
     return rc;
 }
 

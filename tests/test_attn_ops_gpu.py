@@ -1,0 +1,59 @@
+"""The single-query attention operators away from the GPT-2 shapes: head dims
+that no block of 16 loads divides, lengths on both sides of a block of
+positions, caches whose stride or address rules out 16-byte loads, and fused
+calls on both sides of one, two and four chunks, in a row, so that the shared
+partials hold an earlier call's; against a 64-bit softmax attention."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(q, kc, vc, T, NH, DH, scale):
+    s = (q.astype(np.float64).reshape(NH, DH, 1) * kc.reshape(NH, DH, -1)[:, :, :T]).sum(1) * scale
+    p = np.exp(s - s.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    return s, p, np.einsum("ht,thd->hd", p, vc[:T].astype(np.float64).reshape(T, NH, DH)).ravel()
+
+
+@pytest.mark.parametrize("NH,DH,S,T", [(3, 5, 70, 64), (2, 17, 65, 65), (1, 64, 1024, 1), (5, 80, 257, 257), (4, 130, 1000, 999),
+                                       (12, 64, 1024, 1024)])
+def test_reference_operators(g2, NH, DH, S, T):
+    D = NH * DH
+    r = np.random.default_rng(NH * DH + T)
+    q, kc, vc = (r.standard_normal(n).astype(np.float32) for n in (D, D * S, S * D))
+    scale = float(np.float32(1 / np.sqrt(DH)))
+    s, p, o = reference(q, kc, vc.reshape(S, D), T, NH, DH, scale)
+    dk, dv, dO = g2.to_device(kc), g2.to_device(vc), g2.to_device(np.full(D + 1, 7.0, np.float32))
+    # scores are written with stride S and read by the softmax with stride 1024
+    dS = g2.to_device(np.zeros(NH * 1024, np.float32))
+    g2.attn_scores_1q(g2.to_device(q), dk, dS, 0, T, D, DH, NH, S, scale)
+    got = dS.download(np.float32, NH * S).reshape(NH, S)[:, :T]
+    np.testing.assert_allclose(got, s, rtol=1e-5, atol=2e-6 * np.sqrt(DH))
+    rows = np.zeros((NH, 1024), np.float32)
+    rows[:, :T] = s
+    dS = g2.to_device(rows)
+    g2.attn_softmax_1q(dS, T, NH)
+    got = dS.download(np.float32, NH * 1024).reshape(NH, 1024)
+    np.testing.assert_allclose(got[:, :T], p, rtol=2e-5, atol=1e-7)
+    assert (got[:, T:] == 0).all()  # nothing past the row
+    g2.attn_out_1q(dS, dv, dO, T, D, DH, 0)
+    got = dO.download(np.float32, D + 1)
+    np.testing.assert_allclose(got[:D], o, rtol=1e-4, atol=2e-5)
+    assert got[D] == 7.0
+
+
+@pytest.mark.parametrize("NH,S,shift", [(1, 1024, 0), (25, 1024, 0), (7, 1023, 0), (12, 1024, 1), (64, 1000, 0)])
+def test_fused_lengths_in_a_row(g2, NH, S, shift):
+    D = NH * 64
+    r = np.random.default_rng(NH + S)
+    q, kc, vc = (r.standard_normal(n).astype(np.float32) for n in (D, D * S, S * D))
+    pad = np.zeros(shift, np.float32)
+    dq, dk, dv = g2.to_device(q), g2.to_device(np.concatenate([pad, kc])), g2.to_device(np.concatenate([pad, vc]))
+    for fn in (g2.attn_1q, g2.attn_1q_noalloc):
+        for T in (S, 64, 65, 1, 128, 129, 256, 257, 63, S - 1):
+            dO = g2.DevBuf(D * 4)
+            for _ in range(2):
+                fn(dq, dk.offset(4 * shift), dv.offset(4 * shift), dO, 0, T, D, NH, S, 0, 0.125)
+            o = reference(q, kc, vc.reshape(S, D), T, NH, 64, 0.125)[2]
+            np.testing.assert_allclose(dO.download(np.float32, D), o, rtol=1e-4, atol=2e-5, err_msg=f"T {T}")
