@@ -44,6 +44,7 @@ extern "C" {
     X(ATTN_PART, "g2k_attn_part") X(ATTN_PART_S, "g2k_attn_part_s")           \
     X(ATTN_MERGE, "g2k_attn_merge") X(ARGMAX_MERGE, "g2k_argmax_merge")       \
     X(ATTN_SHORT, "g2k_attn_short") X(ATTN_SHORT_S, "g2k_attn_short_s")       \
+    X(ATTN_ROWS, "g2k_attn_rows")                                             \
     G2_ROWS_LIST(X, STORE, "store") G2_ROWS_LIST(X, LN_QKV, "ln_qkv")         \
     G2_ROWS_LIST(X, RESID, "resid") G2_ROWS_LIST(X, LN_GELU, "ln_gelu")       \
     G2_ROWS_LIST(X, LN_ARGMAX, "ln_argmax")                                   \

@@ -192,6 +192,17 @@ typedef struct {
     int T, D, DH, out_base;
 } g2_attnout_args;
 
+/* A prompt's causal attention by rows (g2k_attn_rows): out[P][D] from the
+ * queries in qkv[P][3D] and the caches. */
+typedef struct {
+    const float *qkv;
+    const float *k_cache;
+    const float *v_cache;
+    float *out;
+    int D, DH, S;
+    float scale;
+} g2_attnrows_args;
+
 /* Single-query attention, head dim 64, split over 64-position key chunks
  * (partials kernel) and merged by a second kernel, or (g2k_attn_short) up to
  * G2_ATTN_GROUP chunks in one work-group per head.  T = T_fixed if > 0, else

@@ -497,6 +497,83 @@ extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout
     }
 }
 
+/* ---- a prompt's attention on the reference path: the three operators above
+ * for every row i of qkv [P][3D] over positions 0..i, scores kept in LDS; grid
+ * (NH, P), 256 threads.  The reference runs its three launches per row
+ * (prefill(), main.c:1739-1790), 36 P launches for 12 layers: a 96-token
+ * prompt of the 124M model took 22 ms with the former operators and takes
+ * 0.97 in one launch a layer, 500 tokens 2.3 ms (96).  Bounded
+ * by load latency, a work-group's T / 64 blocks one after the other; long
+ * rows start first, so that the last ones running are short. */
+G2K void g2k_attn_rows(const g2_attnrows_args a)
+{
+    __shared__ float sc[G2_KV_MAX_SEQ];
+    __shared__ float red[4][64];
+    __shared__ float red4[4];
+    const int h = blockIdx.x, i = gridDim.y - 1 - blockIdx.y, T = i + 1;
+    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6, DH = a.DH;
+    const float *q = a.qkv + (size_t)i * 3 * a.D + (size_t)h * DH;
+    const float *kc = a.k_cache + (size_t)h * DH * a.S;
+    /* scores: wave g takes 64-position blocks g, g + 4, ... */
+    for (int j0 = 64 * g; j0 < T; j0 += 256) {
+        const float *kj = kc + min(j0 + lane, i);
+        float s = 0.f;
+        for (int k0 = 0; k0 < DH; k0 += 16) {
+            float x[16], y[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const bool in = k0 + u < DH;
+                x[u] = in ? q[k0 + u] : 0.f;
+                y[u] = in ? kj[(size_t)(k0 + u) * a.S] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s = fmaf(x[u], y[u], s);
+        }
+        if (j0 + lane < T) sc[j0 + lane] = s * a.scale;
+    }
+    __syncthreads();
+    /* softmax, as g2k_attn_softmax */
+    float mx = -1e30f;
+    for (int j = threadIdx.x; j < T; j += 256) mx = fmaxf(mx, sc[j]);
+    mx = wave_max(mx);
+    if (lane == 0) red4[g] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red4[0], red4[1]), fmaxf(red4[2], red4[3]));
+    __syncthreads();
+    float sum = 0.f;
+    for (int j = threadIdx.x; j < T; j += 256) {
+        const float e = expf(sc[j] - mx);
+        sc[j] = e;
+        sum += e;
+    }
+    const float inv = 1.0f / block_sum(sum, red4);
+    for (int j = threadIdx.x; j < T; j += 256) sc[j] *= inv;
+    __syncthreads();
+    /* weighted sum: wave g takes positions g, g + 4, ..., eight ahead */
+    const float *v = a.v_cache + (size_t)h * DH;
+    for (int d0 = 0; d0 < DH; d0 += 64) {
+        const int d = min(d0 + lane, DH - 1);
+        float o = 0.f;
+        for (int j0 = g; j0 < T; j0 += 32) {
+            float p[8], y[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const bool in = j0 + 4 * u < T;
+                p[u] = in ? sc[j0 + 4 * u] : 0.f;
+                y[u] = in ? v[(size_t)(j0 + 4 * u) * a.D + d] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) o = fmaf(p[u], y[u], o);
+        }
+        red[g][lane] = o;
+        __syncthreads();
+        if (g == 0 && d0 + lane < DH)
+            a.out[(size_t)i * a.D + (size_t)h * DH + d0 + lane] =
+                ((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane];
+        __syncthreads();
+    }
+}
+
 /* ======================================================================
  * MFMA GEMM (the fused prefill where the forms below do not apply; the
  * reference matmul is in g2_matmul.hip)

@@ -689,15 +689,14 @@ static int ref_matvec_splitk(g2_model *m, const float *A, const float *B, const 
     return rc;
 }
 
-static int ref_attention(g2_model *m, const float *qkv, int l, int q_base, int T_kv, float *out,
-                         int out_base)
+/* A decode step's attention by the three operators. */
+static int ref_attention(g2_model *m, const float *qkv, int l, int T_kv, float *out)
 {
     const int E = m->cfg.n_embd, NH = m->cfg.n_head, DH = E / NH;
     const float scale = 1.0f / sqrtf((float)DH); /* main.c:1692 */
-    int rc = g2_attn_scores_1q(qkv, m->L[l].k_cache, m->scores, q_base, T_kv, E, DH, NH,
-                               G2_KV_MAX_SEQ, scale);
+    int rc = g2_attn_scores_1q(qkv, m->L[l].k_cache, m->scores, 0, T_kv, E, DH, NH, G2_KV_MAX_SEQ, scale);
     if (!rc) rc = g2_attn_softmax_1q(m->scores, T_kv, NH);
-    if (!rc) rc = g2_attn_out_1q(m->scores, m->L[l].v_cache, out, T_kv, E, DH, out_base);
+    if (!rc) rc = g2_attn_out_1q(m->scores, m->L[l].v_cache, out, T_kv, E, DH, 0);
     return rc;
 }
 
@@ -710,8 +709,12 @@ static int ref_prefill(g2_model *m, int P)
         rc = g2_layernorm(m->hidden, m->ln_out, y->ln1_w, y->ln1_b, E, P);
         if (!rc) rc = g2_matmul(m->ln_out, y->qkv_w, y->qkv_b, m->qkv_full, P, T, E);
         if (!rc) rc = g2_split_kv(m->qkv_full, y->k_cache, y->v_cache, 0, P, E, G2_KV_MAX_SEQ);
-        for (int i = 0; i < P && !rc; ++i)
-            rc = ref_attention(m, m->qkv_full, l, i * 3 * E, i + 1, m->attn, i * E);
+        if (!rc) {
+            const int DH = E / m->cfg.n_head;
+            g2_attnrows_args t = { m->qkv_full, y->k_cache, y->v_cache, m->attn, E, DH, G2_KV_MAX_SEQ,
+                                   1.0f / sqrtf((float)DH) };
+            rc = g2i_launch(G2F_ATTN_ROWS, (unsigned)m->cfg.n_head, (unsigned)P, 256, &t);
+        }
         if (!rc) rc = g2_matmul(m->attn, y->proj_w, y->proj_b, m->attn_proj, P, E, E);
         if (!rc) rc = g2_add(m->hidden, m->attn_proj, P * E);
         if (!rc) rc = g2_layernorm(m->hidden, m->ln_out, y->ln2_w, y->ln2_b, E, P);
@@ -735,7 +738,7 @@ static int ref_decode(g2_model *m, int pos)
         rc = g2_layernorm(m->hidden, m->ln_out, y->ln1_w, y->ln1_b, E, 1);
         if (!rc) rc = g2_matvec(m->ln_out, y->qkv_w, y->qkv_b, NULL, m->qkv_new, T, E, 0);
         if (!rc) rc = g2_split_kv(m->qkv_new, y->k_cache, y->v_cache, pos, 1, E, G2_KV_MAX_SEQ);
-        if (!rc) rc = ref_attention(m, m->qkv_new, l, 0, pos + 1, m->attn, 0);
+        if (!rc) rc = ref_attention(m, m->qkv_new, l, pos + 1, m->attn);
         if (!rc) rc = ref_matvec_splitk(m, m->attn, y->proj_w, y->proj_b, m->hidden, m->hidden, E, E);
         if (!rc) rc = g2_layernorm(m->hidden, m->ln_out, y->ln2_w, y->ln2_b, E, 1);
         if (!rc) rc = g2_matvec(m->ln_out, y->fc_w, y->fc_b, NULL, m->ffn1, F, E, 1);
