@@ -1115,10 +1115,13 @@ static int fused_prefill(g2_model *m, int P)
      * fp32-MFMA GEMM for comparison */
     const char *pe = getenv("G2_PREFILL_F32MFMA");
     const int h = f16 && E % 64 == 0 && F % 64 == 0 && !(pe && pe[0] == '1');
-    /* prompts of more than 64 rows: the 128x128 tiles (G2_PREFILL_GEMM64=1
-     * keeps the 64x64 ones, whose results are identical) */
+    /* the 128x128 tiles for every prompt: short ones leave most of a tile's
+     * rows unused, but their K splits stream the weights from all CUs, which
+     * is what bounds them (8 tokens: 774M 2.2 ms against 4.0 on the 64x64
+     * tiles, 1.5B 3.3 against 6.3).  G2_PREFILL_GEMM64=1 keeps the 64x64 ones,
+     * whose results agree to fp32 rounding */
     const char *p64 = getenv("G2_PREFILL_GEMM64");
-    const int big = h && P > 64 && !(p64 && p64[0] == '1');
+    const int big = h && !(p64 && p64[0] == '1');
     /* fp32 weights: the 64x64 fp32-MFMA GEMM with K steps of 32 streamed
      * through LDS, split-K for short prompts */
     const int sg = !f16 && E % 32 == 0 && F % 32 == 0;
