@@ -24,7 +24,6 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 /* vectors at any element's address */
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef _Float16 f16x2u __attribute__((ext_vector_type(2), aligned(2)));
 
@@ -355,16 +354,17 @@ G2K void g2k_xgemm_sum(const g2_gemm_args a)
             f32x4 p[G2_XG_MAXKS];
 #pragma unroll
             for (int z = 0; z < G2_XG_MAXKS; ++z)
-                if (z < a.ksplit) p[z] = *(const xg::f32x4u *)(a.part + z * MN + i);
+                if (z < a.ksplit) p[z] = *(const f32x4u *)(a.part + z * MN + i);
             f32x4 v = p[0];
 #pragma unroll
             for (int z = 1; z < G2_XG_MAXKS; ++z)
                 if (z < a.ksplit) v += p[z];
             if (a.bias) {
+                unsigned n = MN >> 32 ? (unsigned)(i % (size_t)a.N) : (unsigned)i % (unsigned)a.N;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] += a.bias[(i + e) % (size_t)a.N];
+                for (int e = 0; e < 4; ++e, n = n + 1 < (unsigned)a.N ? n + 1 : 0) v[e] += a.bias[n];
             }
-            *(xg::f32x4u *)(a.C + i) = v;
+            *(f32x4u *)(a.C + i) = v;
         } else {
             for (size_t j = i; j < MN; ++j) {
                 float v = a.part[j];

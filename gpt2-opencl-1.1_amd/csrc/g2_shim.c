@@ -529,7 +529,7 @@ int g2_layernorm(const float *x, float *out, const float *gamma, const float *be
 
 static unsigned ew_grid(int n)
 {
-    unsigned g = cdiv(n, 256);
+    unsigned g = cdiv(n, 1024);
     return g > 4096 ? 4096 : g;
 }
 

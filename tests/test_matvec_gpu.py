@@ -2,7 +2,8 @@
 rows shorter than one 16-byte vector, columns past the last whole vector or
 column group, K below and above the rows that a work-group takes at once, the
 column-lane choices, the sliced form of tall narrow matrices, operands at odd
-addresses and results that overlap an operand; against the CPU oracle."""
+addresses and results that overlap an operand; and the elementwise operators'
+and the LayerNorm's remainders; against the CPU oracle."""
 import numpy as np
 import pytest
 
@@ -61,3 +62,30 @@ def test_matvec_sk_edges(g2, N, K, ks, f16):
     for s in range(ks):
         bound = dot_bound(np.abs(A[s::ks]), np.abs(B[s::ks]), max(len(A[s::ks]), 1))
         assert_close_bound(got[s * N:(s + 1) * N], ref[s], bound, what=f"slice {s}")
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1025, 4097])
+def test_elementwise_tails(g2, n):
+    """add and gelu, four elements to a thread: every remainder, one element
+    past an aligned address, nothing past the end."""
+    r = np.random.default_rng(n)
+    a, b = (r.standard_normal(n + 2).astype(np.float32) for _ in range(2))
+    da, db = g2.to_device(a), g2.to_device(b)
+    g2.add(da.offset(4), db.offset(4), n)
+    np.testing.assert_array_equal(da.download(np.float32, n + 2), np.concatenate([a[:1], a[1:-1] + b[1:-1], a[-1:]]))
+    g2.gelu(db.offset(4), n)
+    got = db.download(np.float32, n + 2)
+    np.testing.assert_allclose(got[1:-1], oracle.gelu(b[1:-1].copy()), rtol=4e-6, atol=1e-6)
+    assert got[0] == b[0] and got[-1] == b[-1]
+
+
+@pytest.mark.parametrize("E", [1, 255, 257, 2047, 2048, 2049, 5000])
+def test_layernorm_widths(g2, E):
+    """Rows kept in registers (up to 2048) and rows read three times."""
+    r = np.random.default_rng(E)
+    x, g, b = r.standard_normal((3, E)).astype(np.float32) * 3 + 0.5, *r.standard_normal((2, E)).astype(np.float32)
+    dO = g2.to_device(np.full(3 * E + 4, 7.0, np.float32))
+    g2.layernorm(g2.to_device(x), dO, g2.to_device(g), g2.to_device(b), E, 3)
+    got = dO.download(np.float32, 3 * E + 4)
+    np.testing.assert_allclose(got[:3 * E].reshape(3, E), oracle.layernorm(x, g, b, E, 3), rtol=2e-5, atol=2e-5)
+    assert (got[3 * E:] == 7.0).all()
