@@ -1042,7 +1042,8 @@ static int sg_pick(int M, int N, int K, int *splits)
         const unsigned tiles = cdivu(N, 128) * cdivu(M, (unsigned)rows);
         for (int k = form == SG_FORM_DUO64 ? 2 : 1; k <= G2_SKEPI_MAXKS && 2 * k <= nk; ++k) {
             if (k > 1 && tiles * (unsigned)k > cus) break;
-            const double us = 4 + (double)nk / k * (rows == 64 ? 0.75 : 1.02) * ceil(tiles * k / cus) +
+            const double rounds = ceil(tiles * k / cus); /* several, all CUs at it: a third slower */
+            const double us = 4 + (double)nk / k * (rows == 64 ? 0.75 : rounds > 1 ? 1.4 : 1.02) * rounds +
                               (k > 1 ? 3 + k * slice * (write + read) : 0);
             if (us < best) { best = us; pick = form; *splits = k; }
         }
