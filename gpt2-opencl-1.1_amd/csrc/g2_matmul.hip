@@ -12,12 +12,21 @@
  * rate of the fp32 instruction (4 k): a sixth of 32 k against 4 k leaves
  * 2.7 times the fp32 peak and fewer roundings of the running sum.
  *
- * What the parts cannot carry shows in the accumulator: infinities, NaN and
- * magnitudes that round past bf16's largest make it not finite; factors so
- * small (all of a row or column below 2^-109) that their low parts are
- * subnormal bf16 leave it below 2^-60, unless the other factors exceed 2^40.
- * Such an output, not zero, is computed again in fp32 (again()), so an
- * infinity or NaN comes out as fp32 arithmetic has it.
+ * The conversion and both matrix instructions keep subnormals, so the parts
+ * carry every value whose last bit, 2^-23 of its power of two, is a multiple
+ * of bf16's smallest, 2^-133.  A work-group that reads a smaller one (not
+ * zero, below 2^-110) computes its tile, or its split's part of it, again on
+ * the fp32 matrix instruction (again_tile()): a factor of 2^-120 can meet one
+ * of 2^80, and the sum shows nothing of it.  The test is on the values that a
+ * thread converts, three operations beside the eleven of a pair's parts (a
+ * test for large factors and small sums instead, with a second look at the
+ * operands where it says so, was slower: the prefill of 256 tokens at 774M
+ * 4.58 ms against 4.37).  Such a tile takes about what the fp32 instruction
+ * alone takes: 1024 x 8192 x 1600 of nothing but small values 0.58 ms (0.15).
+ * Infinities, NaN and magnitudes that round past bf16's largest make the sum
+ * not finite; such an output, and one below 2^-60 that is not zero, is
+ * computed again in fp32 (again()), so an infinity or NaN comes out as fp32
+ * arithmetic has it.
  */
 namespace xg {
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -27,13 +36,20 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef _Float16 f16x2u __attribute__((ext_vector_type(2), aligned(2)));
 
-/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts. */
+/* The smallest magnitude but zero among the values a thread has converted, as
+ * its bits doubled (the sign shifted out) less one: zero wraps to the top. */
+constexpr unsigned LEAST0 = ~0u, LEAST_WHOLE = ((127u - 110u) << 24) - 1; /* none yet; 2^-110 */
+
+/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts; three
+ * parts, of fp32 values, go into `least`, two parts carry any fp16 value. */
 template <int P>
-__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P])
+__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], unsigned &least)
 {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         f32x2 r = {v[2 * e], v[2 * e + 1]};
+        if constexpr (P == 3)
+            least = min(min(least, 2 * __float_as_uint(v[2 * e]) - 1), 2 * __float_as_uint(v[2 * e + 1]) - 1);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
             const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
@@ -97,6 +113,61 @@ __device__ __noinline__ float again(const float *A, const BT *B, int N, int K, i
     return s;
 }
 
+/* Whether a wave of the work-group has read a value that the parts do not
+ * carry: one word of LDS per wave, a barrier for all. */
+template <int WAVES>
+__device__ __forceinline__ bool any_small(unsigned (&words)[WAVES], unsigned least)
+{
+    const bool wave_has = __ballot(least < LEAST_WHOLE) != 0;
+    if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = wave_has;
+    __syncthreads();
+    unsigned any = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) any |= words[w];
+    return any != 0;
+}
+
+/* A wave's IB x JB blocks of 16 x 16, rows m + 16 i and column n[j] of the
+ * lane, over k0 <= k < k1, added to acc by the fp32 matrix instruction: a lane
+ * takes four consecutive k of 16, straight from memory. */
+template <typename BT, bool BNK, int IB, int JB>
+__device__ __forceinline__ void again_tile(const float *A, const BT *B, int M, int N, int K, int m, const int (&n)[JB],
+                                           int k0, int k1, f32x4 (&acc)[IB][JB])
+{
+    const int lane = threadIdx.x & 63, fk = 4 * (lane >> 4);
+#pragma unroll 1
+    for (int k = k0 + fk; k - fk < k1; k += 16) {
+        const bool whole = k - fk + 16 <= k1;
+        float x[IB][4], y[JB][4];
+        auto four = [&](float (&v)[4], const float *p) {
+            if (whole) {
+                *(f32x4 *)v = *(const f32x4u *)p;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = k + e < k1 ? p[e] : 0.f;
+            }
+        };
+#pragma unroll
+        for (int i = 0; i < IB; ++i) four(x[i], A + (size_t)min(m + 16 * i + (lane & 15), M - 1) * K + k);
+#pragma unroll
+        for (int j = 0; j < JB; ++j) {
+            const size_t c = min(n[j], N - 1);
+            if constexpr (BNK) {
+                four(y[j], B + c * K + k);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[j][e] = whole || k + e < k1 ? ldw(B, (size_t)(k + e) * N + c) : 0.f;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int i = 0; i < IB; ++i)
+#pragma unroll
+                for (int j = 0; j < JB; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[i][e], y[j][e], acc[i][j], 0, 0, 0);
+    }
+}
+
 /* The k, within a step of 32, of element e of octet o is 4 o + koff(e), for
  * both factors: the four lanes of a row then load 64 consecutive bytes. */
 __device__ __forceinline__ constexpr int koff(int e) { return e < 4 ? e : 12 + e; }
@@ -142,6 +213,8 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     constexpr int IB = BM / 32, JB = BN / 32;                       /* 16-blocks of a wave */
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[ST];
+    __shared__ unsigned small[4];
+    unsigned least = LEAST0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int M = a.M, N = a.N, K = a.K;
@@ -201,7 +274,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RA; ++i) {
             u32x4 p[3];
-            parts8<3>(av[i], p);
+            parts8<3>(av[i], p, least);
 #pragma unroll
             for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
         }
@@ -212,7 +285,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             u32x4 p[PB];
-            parts8<PB>(bv[i], p);
+            parts8<PB>(bv[i], p, least);
 #pragma unroll
             for (int q = 0; q < PB; ++q)
                 *(u32x4 *)(lds + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
@@ -280,6 +353,16 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
         return PAIR ? n0 + 2 * (wn * (BN / 4) + (j & (JB / 2 - 1)) * 16 + (lane & 15)) + j / (JB / 2)
                     : n0 + wn * (BN / 2) + j * 16 + (lane & 15);
     };
+    if (__builtin_expect(any_small(small, least), 0)) {
+        int n[JB];
+#pragma unroll
+        for (int j = 0; j < JB; ++j) n[j] = on(j);
+#pragma unroll
+        for (int i = 0; i < IB; ++i)
+#pragma unroll
+            for (int j = 0; j < JB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        again_tile<BT, BNK>(a.A, B, M, N, K, m0 + wm * (BM / 2), n, s0 * 32, min(s1 * 32, K), acc);
+    }
     unsigned long long odd = 0;
 #pragma unroll
     for (int i = 0; i < IB; ++i)
@@ -395,6 +478,8 @@ __device__ void xduo_impl(const g2_gemm_args &a)
     constexpr int SA = BM * 16 + 64, SB = BN * 16 + (BNK ? 64 : 0); /* octet plane strides, bytes */
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * ST];
+    __shared__ unsigned small[8];
+    unsigned least = LEAST0;
     const int tid = threadIdx.x & 255, lane = tid & 63;
     const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = w8 >> 2, wave = w8 & 3, wm = wave >> 1, wn = wave & 1;
@@ -450,7 +535,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RA; ++i) {
             u32x4 p[3];
-            parts8<3>(av[i], p);
+            parts8<3>(av[i], p, least);
 #pragma unroll
             for (int q = 0; q < 3; ++q) *(u32x4 *)(st + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
         }
@@ -470,7 +555,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             u32x4 p[PB];
-            parts8<PB>(b[i], p);
+            parts8<PB>(b[i], p, least);
 #pragma unroll
             for (int q = 0; q < PB; ++q)
                 *(u32x4 *)(st + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
@@ -601,6 +686,14 @@ __device__ void xduo_impl(const g2_gemm_args &a)
     auto on = [&](int j) {
         return BNK ? n0 + wn * 64 + j * 16 + (lane & 15) : n0 + 2 * (wn * 32 + (j & 1) * 16 + (lane & 15)) + (j >> 1);
     };
+    if (__builtin_expect(any_small(small, least), 0)) {
+        const int n[4] = {on(0), on(1), on(2), on(3)};
+#pragma unroll
+        for (int i = 0; i < HB; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) sum[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        again_tile<BT, BNK>(a.A, B, M, N, K, m0 + wm * (BM / 2) + g * HB * 16, n, s0 * 32, min(s1 * 32, K), sum);
+    }
     unsigned odd = 0;
 #pragma unroll
     for (int c = 0; c < 16 * HB; ++c)
@@ -698,6 +791,8 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
     using namespace xg;
     constexpr int PB = sizeof(BT) == 4 ? 3 : 2, NW = 8;
     __shared__ float red[NW][RB * 2][256];
+    __shared__ unsigned small[NW];
+    unsigned least = LEAST0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = a.M, N = a.N, K = a.K;
     const int nmb = (M + 16 * RB - 1) / (16 * RB);
@@ -757,21 +852,33 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int e = 0; e < 8; ++e) bv[0][e] = late ? bv[1][e] : bv[0][e];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) parts8<PB>(bv[j], b[j]);
+        for (int j = 0; j < 2; ++j) parts8<PB>(bv[j], b[j], least);
 #pragma unroll
-        for (int i = 0; i < RB; ++i) parts8<3>(av[i], f[i]);
+        for (int i = 0; i < RB; ++i) parts8<3>(av[i], f[i], least);
         if (t + NW < nkt) load(t + NW);
 #pragma unroll
         for (int i = 0; i < RB; ++i) mma_parts<PB, 2>(acc[i], f[i], b);
     }
     /* [block][row 4 (l/16) + q][column l % 16] */
+    auto hand_in = [&]() {
 #pragma unroll
-    for (int i = 0; i < RB; ++i)
+        for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) red[wave][2 * i + j][(4 * (lane >> 4) + q) * 16 + fr] = acc[i][j][q];
-    __syncthreads();
+                for (int q = 0; q < 4; ++q) red[wave][2 * i + j][(4 * (lane >> 4) + q) * 16 + fr] = acc[i][j][q];
+    };
+    hand_in();
+    if (__builtin_expect(any_small(small, least), 0)) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        const int n[2] = {n0 + 2 * fr, n0 + 2 * fr + 1};
+        for (int t = wave; t < nkt; t += NW) again_tile<BT, false>(a.A, B, M, N, K, m0, n, 32 * t, min(32 * t + 32, K), acc);
+        hand_in(); /* its own words, which no other wave has read yet */
+        __syncthreads();
+    }
     for (int o = tid; o < RB * 512; o += NW * 64) {
         const int i = o >> 9, r = (o >> 5) & 15, c = o & 31;
         const int m = m0 + 16 * i + r, n = n0 + c;

@@ -69,3 +69,67 @@ def test_matmul_special_values(g2, M, N, K, f16):
     fin = np.isfinite(ref)
     np.testing.assert_array_equal(got[~fin & ~np.isnan(ref)], ref[~fin & ~np.isnan(ref)])
     assert (np.abs(got[fin].astype(np.float64) - ref[fin]) <= bound[fin] + 1e-45).all()
+
+
+# one size per form: direct 16 and 32 rows, 64x64 whole and split, 128x128 of
+# several work-groups per CU, of alternating wave groups whole and split
+FORM_SIZES = [(20, 70, 100), (18, 5755, 1389), (470, 2305, 70), (70, 200, 4100), (700, 8321, 70), (118, 20173, 1191),
+              (257, 5121, 1281)]
+
+
+def sized(r, shape, e):
+    """Values of magnitude 2^e to 2^(e+1), all 24 bits random."""
+    return np.ldexp(np.float32(1) + r.random(shape, np.float32), e).astype(np.float32) * r.choice(np.float32([-1, 1]), shape)
+
+
+@pytest.mark.parametrize("f16,ea,eb", [(False, -115, 70), (False, 70, -120), (False, -126, 100), (False, -140, 100),
+                                       (True, -120, 10), (True, -140, 12)])
+@pytest.mark.parametrize("M,N,K", FORM_SIZES)
+def test_matmul_small_by_large(g2, M, N, K, f16, ea, eb):
+    """Operands whose low bits bf16 parts do not hold, against ones that lift
+    the product back among ordinary values: fp32 products all the same.  A sum
+    of K random terms takes roundings of 2^-24 of a partial sum that grows to
+    its own size, sqrt(K) / 3 of them in the norm; a result in fp32's
+    subnormals is off by half their step besides."""
+    r = np.random.default_rng(K)
+    A, B = sized(r, (M, K), ea), sized(r, (K, N), eb)
+    if f16:
+        B = B.astype(np.float16).astype(np.float32)
+    got, ref = product(g2, A, B, None, f16).astype(np.float64), A.astype(np.float64) @ B.astype(np.float64)
+    err = np.linalg.norm(got - ref) - 2.0 ** -150 * np.sqrt(M * N)
+    assert err <= 2.0 ** -24 * (2 + np.sqrt(K) / 2) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("M,N,K", FORM_SIZES)
+def test_matmul_one_small_value(g2, M, N, K):
+    """One subnormal value in each operand, alone with a large factor: in a row
+    and a column that the tile's other values do not share."""
+    A, B, _ = operands(M, N, K, False, 3)
+    A[M - 1], B[:, N - 1] = 0, 0
+    A[M - 1, K - 1], B[K - 1, 0] = 2.0 ** -140, 2.0 ** 120
+    A[0, 0], B[0, N - 1] = -(2.0 ** 120), 2.0 ** -145
+    got = product(g2, A, B, None, False)
+    assert got[M - 1, 0] == 2.0 ** -20 and got[0, N - 1] == -(2.0 ** -25)
+
+
+@pytest.mark.parametrize("P", [70, 300, 1000])
+def test_prefill_small_weights_large_gain(g2, P):
+    """The fp32 prefill's GEMMs (more than 64 rows: bf16 parts, split and whole)
+    with q/k/v and MLP weights of 2^-128 behind LayerNorm gains of 2^122."""
+    cfg = g2.make_config(2, 768, 12, vocab_size=1000)
+    w = g2.synth_weights(cfg, 77)
+    gain, part = np.float32(2.0 ** 122), np.float32(2.0 ** -122)
+    for i, layer in enumerate(w["layers"]):
+        layer = list(layer)
+        for norm, mat in ((0, 2), (6, 8)):
+            layer[norm] = (layer[norm] * gain).astype(np.float32)
+            layer[mat] = (layer[mat] * part).astype(np.float32)
+        w["layers"][i] = tuple(layer)
+    ids = np.random.default_rng(P).integers(0, cfg.vocab_size, P).astype(np.int32)
+    m = g2.Model.from_host(cfg, w, g2.F32, g2.PATH_FUSED)
+    m.prefill(ids)
+    om = oracle.Model(cfg, w)
+    om.prefill(ids)
+    np.testing.assert_allclose(m.logits(), om.logits(), rtol=0, atol=1e-4)
+    om.close()
+    m.free()
