@@ -23,10 +23,9 @@
  * operands where it says so, was slower: the prefill of 256 tokens at 774M
  * 4.58 ms against 4.37).  Such a tile takes about what the fp32 instruction
  * alone takes: 1024 x 8192 x 1600 of nothing but small values 0.58 ms (0.15).
- * Infinities, NaN and magnitudes that round past bf16's largest make the sum
- * not finite; such an output, and one below 2^-60 that is not zero, is
- * computed again in fp32 (again()), so an infinity or NaN comes out as fp32
- * arithmetic has it.
+ * Infinities, NaN and magnitudes that round past bf16's largest make a sum not
+ * finite; the tile is then computed again in the same way, so they come out as
+ * fp32 arithmetic has them.
  */
 namespace xg {
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -82,43 +81,26 @@ __device__ __forceinline__ void mma_parts(f32x4 (&acc)[J], const u32x4 (&a)[3], 
             if (pb[p] < PB) acc[j] = mma(a[pa[p]], b[j][pb[p] < PB ? pb[p] : 0], acc[j]);
 }
 
-/* The bit of an accumulator value that has to be computed again. */
-__device__ __forceinline__ bool odd_value(float v)
+/* Adds a NaN to z (zeros at first) for a sum that is not finite, else zero. */
+__device__ __forceinline__ void finite(f32x4 &z, const f32x4 &v)
 {
-    const unsigned b = __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
-    return b >= 0x7f800000u || (b != 0 && b < (67u << 23));
+#pragma unroll
+    for (int q = 0; q < 4; ++q) z[q] = fmaf(v[q], 0.f, z[q]);
 }
 
-/* Output (m, n) over k0 <= k < k1 in fp32, in order; a sum that has become
- * NaN stays NaN. */
-template <typename BT, bool BNK>
-__device__ __noinline__ float again(const float *A, const BT *B, int N, int K, int m, int n, int k0, int k1)
+/* Whether what a thread has seen calls for the fp32 instruction. */
+__device__ __forceinline__ bool not_carried(unsigned least, const f32x4 &z)
 {
-    const float *a = A + (size_t)m * K;
-    const BT *b = B + (BNK ? (size_t)n * K : (size_t)n);
-    const size_t sb = BNK ? 1 : (size_t)N;
-    float s = 0.f;
-    int k = k0;
-    for (; k + 16 <= k1 && s == s; k += 16) {
-        float x[16], y[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            x[e] = a[k + e];
-            y[e] = ldw(b, (size_t)(k + e) * sb);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s = fmaf(x[e], y[e], s);
-    }
-    for (; k < k1 && s == s; ++k) s = fmaf(a[k], ldw(b, (size_t)k * sb), s);
-    return s;
+    const float s = (z[0] + z[1]) + (z[2] + z[3]);
+    return least < LEAST_WHOLE || s != s;
 }
 
-/* Whether a wave of the work-group has read a value that the parts do not
- * carry: one word of LDS per wave, a barrier for all. */
+/* Whether any thread of the work-group says so: one word of LDS per wave, a
+ * barrier for all. */
 template <int WAVES>
-__device__ __forceinline__ bool any_small(unsigned (&words)[WAVES], unsigned least)
+__device__ __forceinline__ bool any_thread(unsigned (&words)[WAVES], bool mine)
 {
-    const bool wave_has = __ballot(least < LEAST_WHOLE) != 0;
+    const bool wave_has = __ballot(mine) != 0;
     if ((threadIdx.x & 63) == 0) words[threadIdx.x >> 6] = wave_has;
     __syncthreads();
     unsigned any = 0;
@@ -213,7 +195,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     constexpr int IB = BM / 32, JB = BN / 32;                       /* 16-blocks of a wave */
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[ST];
-    __shared__ unsigned small[4];
+    __shared__ unsigned words[4];
     unsigned least = LEAST0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
@@ -353,7 +335,12 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
         return PAIR ? n0 + 2 * (wn * (BN / 4) + (j & (JB / 2 - 1)) * 16 + (lane & 15)) + j / (JB / 2)
                     : n0 + wn * (BN / 2) + j * 16 + (lane & 15);
     };
-    if (__builtin_expect(any_small(small, least), 0)) {
+    f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < IB; ++i)
+#pragma unroll
+        for (int j = 0; j < JB; ++j) finite(z, acc[i][j]);
+    if (__builtin_expect(any_thread(words, not_carried(least, z)), 0)) {
         int n[JB];
 #pragma unroll
         for (int j = 0; j < JB; ++j) n[j] = on(j);
@@ -362,27 +349,6 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
             for (int j = 0; j < JB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         again_tile<BT, BNK>(a.A, B, M, N, K, m0 + wm * (BM / 2), n, s0 * 32, min(s1 * 32, K), acc);
-    }
-    unsigned long long odd = 0;
-#pragma unroll
-    for (int i = 0; i < IB; ++i)
-#pragma unroll
-        for (int j = 0; j < JB; ++j)
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-                if (odd_value(acc[i][j][q])) odd |= 1ull << ((i * JB + j) * 4 + q);
-    while (odd) {
-        const int c = __ffsll(odd) - 1;
-        odd &= odd - 1;
-        const int m = om(c / (4 * JB), c & 3), n = on((c >> 2) % JB);
-        const float v = m < M && n < N ? again<BT, BNK>(a.A, B, N, K, m, n, s0 * 32, min(s1 * 32, K)) : 0.f;
-#pragma unroll
-        for (int i = 0; i < IB; ++i)
-#pragma unroll
-            for (int j = 0; j < JB; ++j)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    if (c == (i * JB + j) * 4 + q) acc[i][j][q] = v;
     }
 
     float *C = EPI == GEPI_PARTIAL ? a.part + (size_t)blockIdx.y * M * N : a.C;
@@ -478,7 +444,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
     constexpr int SA = BM * 16 + 64, SB = BN * 16 + (BNK ? 64 : 0); /* octet plane strides, bytes */
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * ST];
-    __shared__ unsigned small[8];
+    __shared__ unsigned words[8];
     unsigned least = LEAST0;
     const int tid = threadIdx.x & 255, lane = tid & 63;
     const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -686,26 +652,18 @@ __device__ void xduo_impl(const g2_gemm_args &a)
     auto on = [&](int j) {
         return BNK ? n0 + wn * 64 + j * 16 + (lane & 15) : n0 + 2 * (wn * 32 + (j & 1) * 16 + (lane & 15)) + (j >> 1);
     };
-    if (__builtin_expect(any_small(small, least), 0)) {
+    f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < HB; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) finite(z, sum[i][j]);
+    if (__builtin_expect(any_thread(words, not_carried(least, z)), 0)) {
         const int n[4] = {on(0), on(1), on(2), on(3)};
 #pragma unroll
         for (int i = 0; i < HB; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) sum[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         again_tile<BT, BNK>(a.A, B, M, N, K, m0 + wm * (BM / 2) + g * HB * 16, n, s0 * 32, min(s1 * 32, K), sum);
-    }
-    unsigned odd = 0;
-#pragma unroll
-    for (int c = 0; c < 16 * HB; ++c)
-        if (odd_value(sum[c >> 4][(c >> 2) & 3][c & 3])) odd |= 1u << c;
-    while (odd) {
-        const int c = __ffs(odd) - 1;
-        odd &= odd - 1;
-        const int m = om(c >> 4, c & 3), n = on((c >> 2) & 3);
-        const float v = m < M && n < N ? again<BT, BNK>(a.A, B, N, K, m, n, s0 * 32, min(s1 * 32, K)) : 0.f;
-#pragma unroll
-        for (int d = 0; d < 16 * HB; ++d)
-            if (c == d) sum[d >> 4][(d >> 2) & 3][d & 3] = v;
     }
 
     /* every load of the epilogue before its first store */
@@ -791,7 +749,6 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
     using namespace xg;
     constexpr int PB = sizeof(BT) == 4 ? 3 : 2, NW = 8;
     __shared__ float red[NW][RB * 2][256];
-    __shared__ unsigned small[NW];
     unsigned least = LEAST0;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = a.M, N = a.N, K = a.K;
@@ -868,32 +825,49 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) red[wave][2 * i + j][(4 * (lane >> 4) + q) * 16 + fr] = acc[i][j][q];
     };
+    /* a wave with something that the parts do not carry hands in NaN, which
+     * shows in every thread's sum; finite sums never add up to one */
+    f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) finite(z, acc[i][j]);
+    if (__builtin_expect(__ballot(not_carried(least, z)) != 0, 0))
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){NAN, NAN, NAN, NAN};
     hand_in();
-    if (__builtin_expect(any_small(small, least), 0)) {
+    __syncthreads();
+    /* output o of the tile: its sum over the waves, in order */
+    auto total = [&](int o) {
+        const int i = o >> 9, r = (o >> 5) & 15, c = o & 31;
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float x = red[w][2 * i + (c & 1)][r * 16 + (c >> 1)];
+            v = w ? v + x : x;
+        }
+        return v;
+    };
+    float v = total(tid);
+    if (__builtin_expect(v != v, 0)) { /* of all threads or none */
+        __syncthreads();
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         const int n[2] = {n0 + 2 * fr, n0 + 2 * fr + 1};
         for (int t = wave; t < nkt; t += NW) again_tile<BT, false>(a.A, B, M, N, K, m0, n, 32 * t, min(32 * t + 32, K), acc);
-        hand_in(); /* its own words, which no other wave has read yet */
+        hand_in();
         __syncthreads();
+        v = total(tid);
     }
-    for (int o = tid; o < RB * 512; o += NW * 64) {
-        const int i = o >> 9, r = (o >> 5) & 15, c = o & 31;
-        const int m = m0 + 16 * i + r, n = n0 + c;
-        if (m >= M || n >= N) continue;
-        float v = red[0][2 * i + (c & 1)][r * 16 + (c >> 1)];
-        bool odd = odd_value(v);
 #pragma unroll
-        for (int w = 1; w < NW; ++w) {
-            const float x = red[w][2 * i + (c & 1)][r * 16 + (c >> 1)];
-            odd |= odd_value(x);
-            v += x;
-        }
-        if (odd) v = again<BT, false>(a.A, B, N, K, m, n, 0, K);
-        if (a.bias) v += a.bias[n];
-        a.C[(size_t)m * N + n] = v;
+    for (int o = tid; o < RB * 512; o += NW * 64) {
+        const int m = m0 + (o >> 5), n = n0 + (o & 31);
+        if (o >= 512) v = total(o);
+        if (m < M && n < N) a.C[(size_t)m * N + n] = a.bias ? v + a.bias[n] : v;
     }
 }
 #define G2_XSKINNY(name, BT, RB) \

@@ -6,6 +6,8 @@ in K splits, 128x128 tiles) on ragged edges: one row or column past a tile,
 odd column counts (a column pair that the last column begins), K below one
 step of 32, one past it, and splits that end in a partial step.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -110,6 +112,37 @@ def test_matmul_one_small_value(g2, M, N, K):
     A[0, 0], B[0, N - 1] = -(2.0 ** 120), 2.0 ** -145
     got = product(g2, A, B, None, False)
     assert got[M - 1, 0] == 2.0 ** -20 and got[0, N - 1] == -(2.0 ** -25)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 200, 4100), (256, 1280, 1280), (512, 4000, 640), (1024, 8192, 1600)])
+def test_matmul_time_by_values(g2, M, N, K):
+    """Products of small size (1e-10 by 1e-10) take the ordinary time, and an
+    infinity in every row or operands that only fp32 holds about the fp32
+    instruction's: direct, 64x64 split, 128x128 (measured 1.0 and up to 5 times
+    the ordinary time; 10 to 60 when each such output was summed by itself)."""
+    A, B, _ = operands(M, N, K, False, 4)
+    dA, dB, dC = g2.DevBuf(A.nbytes), g2.DevBuf(B.nbytes), g2.DevBuf(4 * M * N)
+
+    def seconds(a, b):
+        dA.upload(a)
+        dB.upload(b)
+        best = 1.0
+        for _ in range(5):
+            g2.matmul(dA, dB, None, dC, M, N, K)
+            g2.sync()
+            t = time.perf_counter()
+            for _ in range(10):
+                g2.matmul(dA, dB, None, dC, M, N, K)
+            g2.sync()
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    plain = seconds(A, B)
+    assert seconds(A * np.float32(1e-10), B * np.float32(5e-9)) < 2 * plain
+    rows = A.copy()
+    rows[:, K // 2] = np.inf
+    assert seconds(rows, B) < 8 * plain
+    assert seconds(A * np.float32(2.0 ** -125), B) < 8 * plain
 
 
 @pytest.mark.parametrize("P", [70, 300, 1000])
