@@ -14,15 +14,17 @@
  *
  * The conversion and both matrix instructions keep subnormals, so the parts
  * carry every value whose last bit, 2^-23 of its power of two, is a multiple
- * of bf16's smallest, 2^-133.  A work-group that reads a smaller one (not
- * zero, below 2^-110) computes its tile, or its split's part of it, again on
- * the fp32 matrix instruction (again_tile()): a factor of 2^-120 can meet one
- * of 2^80, and the sum shows nothing of it.  The test is on the values that a
- * thread converts, three operations beside the eleven of a pair's parts (a
- * test for large factors and small sums instead, with a second look at the
- * operands where it says so, was slower: the prefill of 256 tokens at 774M
- * 4.58 ms against 4.37).  Such a tile takes about what the fp32 instruction
- * alone takes: 1024 x 8192 x 1600 of nothing but small values 0.58 ms (0.15).
+ * of bf16's smallest, 2^-133.  A work-group that reads a smaller one computes
+ * its tile, or its split's part of it, again on the fp32 matrix instruction
+ * (again_tile()): a factor of 2^-120 can meet one of 2^80, and the sum shows
+ * nothing of it.  The test is whether what is left for the third part is
+ * subnormal in fp32, one operation per value beside the 5.5 of its parts: it
+ * is for every value that the parts do not carry and never for one of 2^-103
+ * or more.  (A running minimum of the values took 1.5: 333 x 6400 x 1600 fp16
+ * 54.5 us against 49.9; a test for large factors and small sums, with a second
+ * look at the operands where it says so, was slower still.)  Such a tile takes
+ * about what the fp32 instruction alone takes: 1024 x 8192 x 1600 of nothing
+ * but small values 0.54 ms (0.14).
  * Infinities, NaN and magnitudes that round past bf16's largest make a sum not
  * finite; the tile is then computed again in the same way, so they come out as
  * fp32 arithmetic has them.
@@ -35,22 +37,17 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef _Float16 f16x2u __attribute__((ext_vector_type(2), aligned(2)));
 
-/* The smallest magnitude but zero among the values a thread has converted, as
- * its bits doubled (the sign shifted out) less one: zero wraps to the top. */
-constexpr unsigned LEAST0 = ~0u, LEAST_WHOLE = ((127u - 110u) << 24) - 1; /* none yet; 2^-110 */
-
-/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts; three
- * parts, of fp32 values, go into `least`, two parts carry any fp16 value. */
+/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts; `lossy`
+ * is set where three may not be all of a value.  Two are, of any fp16 value. */
 template <int P>
-__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], unsigned &least)
+__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], bool &lossy)
 {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         f32x2 r = {v[2 * e], v[2 * e + 1]};
-        if constexpr (P == 3)
-            least = min(min(least, 2 * __float_as_uint(v[2 * e]) - 1), 2 * __float_as_uint(v[2 * e + 1]) - 1);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
+            if (P == 3 && p == 2) lossy |= __builtin_amdgcn_classf(r.x, 0x90) | __builtin_amdgcn_classf(r.y, 0x90);
             const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
             o[p][e] = w;
             if (p + 1 < P) {
@@ -89,10 +86,10 @@ __device__ __forceinline__ void finite(f32x4 &z, const f32x4 &v)
 }
 
 /* Whether what a thread has seen calls for the fp32 instruction. */
-__device__ __forceinline__ bool not_carried(unsigned least, const f32x4 &z)
+__device__ __forceinline__ bool not_carried(bool lossy, const f32x4 &z)
 {
     const float s = (z[0] + z[1]) + (z[2] + z[3]);
-    return least < LEAST_WHOLE || s != s;
+    return lossy || s != s;
 }
 
 /* Whether any thread of the work-group says so: one word of LDS per wave, a
@@ -196,7 +193,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[ST];
     __shared__ unsigned words[4];
-    unsigned least = LEAST0;
+    bool lossy = false;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int M = a.M, N = a.N, K = a.K;
@@ -256,7 +253,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RA; ++i) {
             u32x4 p[3];
-            parts8<3>(av[i], p, least);
+            parts8<3>(av[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
         }
@@ -267,7 +264,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             u32x4 p[PB];
-            parts8<PB>(bv[i], p, least);
+            parts8<PB>(bv[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < PB; ++q)
                 *(u32x4 *)(lds + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
@@ -340,7 +337,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     for (int i = 0; i < IB; ++i)
 #pragma unroll
         for (int j = 0; j < JB; ++j) finite(z, acc[i][j]);
-    if (__builtin_expect(any_thread(words, not_carried(least, z)), 0)) {
+    if (__builtin_expect(any_thread(words, not_carried(lossy, z)), 0)) {
         int n[JB];
 #pragma unroll
         for (int j = 0; j < JB; ++j) n[j] = on(j);
@@ -445,7 +442,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[2 * ST];
     __shared__ unsigned words[8];
-    unsigned least = LEAST0;
+    bool lossy = false;
     const int tid = threadIdx.x & 255, lane = tid & 63;
     const int w8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = w8 >> 2, wave = w8 & 3, wm = wave >> 1, wn = wave & 1;
@@ -501,7 +498,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RA; ++i) {
             u32x4 p[3];
-            parts8<3>(av[i], p, least);
+            parts8<3>(av[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < 3; ++q) *(u32x4 *)(st + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
         }
@@ -521,7 +518,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
             u32x4 p[PB];
-            parts8<PB>(b[i], p, least);
+            parts8<PB>(b[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < PB; ++q)
                 *(u32x4 *)(st + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
@@ -657,7 +654,7 @@ __device__ void xduo_impl(const g2_gemm_args &a)
     for (int i = 0; i < HB; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) finite(z, sum[i][j]);
-    if (__builtin_expect(any_thread(words, not_carried(least, z)), 0)) {
+    if (__builtin_expect(any_thread(words, not_carried(lossy, z)), 0)) {
         const int n[4] = {on(0), on(1), on(2), on(3)};
 #pragma unroll
         for (int i = 0; i < HB; ++i)
@@ -749,7 +746,7 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
     using namespace xg;
     constexpr int PB = sizeof(BT) == 4 ? 3 : 2, NW = 8;
     __shared__ float red[NW][RB * 2][256];
-    unsigned least = LEAST0;
+    bool lossy = false;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = a.M, N = a.N, K = a.K;
     const int nmb = (M + 16 * RB - 1) / (16 * RB);
@@ -809,9 +806,9 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int e = 0; e < 8; ++e) bv[0][e] = late ? bv[1][e] : bv[0][e];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) parts8<PB>(bv[j], b[j], least);
+        for (int j = 0; j < 2; ++j) parts8<PB>(bv[j], b[j], lossy);
 #pragma unroll
-        for (int i = 0; i < RB; ++i) parts8<3>(av[i], f[i], least);
+        for (int i = 0; i < RB; ++i) parts8<3>(av[i], f[i], lossy);
         if (t + NW < nkt) load(t + NW);
 #pragma unroll
         for (int i = 0; i < RB; ++i) mma_parts<PB, 2>(acc[i], f[i], b);
@@ -832,7 +829,7 @@ __device__ void xskinny_impl(const g2_gemm_args &a)
     for (int i = 0; i < RB; ++i)
 #pragma unroll
         for (int j = 0; j < 2; ++j) finite(z, acc[i][j]);
-    if (__builtin_expect(__ballot(not_carried(least, z)) != 0, 0))
+    if (__builtin_expect(__ballot(not_carried(lossy, z)) != 0, 0))
 #pragma unroll
         for (int i = 0; i < RB; ++i)
 #pragma unroll
