@@ -142,8 +142,10 @@ int g2i_device_alloc(void **p, size_t bytes);
 int g2i_rows_launch(int fid_f32_64, int f16, g2_rows_args *a);
 /* Work-groups g2i_rows_launch uses for N rows of K (0 if K is invalid). */
 unsigned g2i_rows_grid(int N, int K, int f16);
-/* Single-query attention over `chunks` key chunks: one launch up to
- * G2_ATTN_GROUP (a length given by the caller), else partials, then merge. */
+/* Single-query attention over `chunks` key chunks: one launch where
+ * g2i_attn_one_launch allows it (lengths given by the caller, 0 otherwise),
+ * else partials, then merge. */
+int g2i_attn_one_launch(const float *q, const float *k_cache, const float *v_cache, const float *out, int T, int D, int S);
 int g2i_attn_launch(g2_attn1q_args *a, unsigned chunks);
 
 /* host helpers (g2_host.c) */

@@ -322,6 +322,10 @@ int g2_sync(void)
 
 static unsigned cdiv(long a, long b) { return (unsigned)((a + b - 1) / b); }
 static int aligned(const void *p, size_t a) { return ((uintptr_t)p % a) == 0; }
+static int overlap(const void *p, size_t np, const void *q, size_t nq)
+{
+    return (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
+}
 
 /* The launches that write and read G.scratch are enqueued without another
  * thread's between them; the stream then keeps their order. */
@@ -441,11 +445,6 @@ static int matvec_launch(int f16, g2_matvec_args *a)
     while (shape > 0 && cdiv(a->N, (4u << shape) * v) * (unsigned)a->nslice < 160) --shape;
     const int fid = (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + 2 * shape;
     return g2i_launch(fid, cdiv(a->N, (4u << shape) * v), (unsigned)a->nslice, 1024, a);
-}
-
-static int overlap(const void *p, size_t np, const void *q, size_t nq)
-{
-    return (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
 }
 
 /* One launch, except: a tall narrow matrix (its few work-groups would walk
@@ -655,10 +654,22 @@ int g2_attn_1q_noalloc(const float *qkv, const float *k_cache, const float *v_ca
     return g2i_attn_launch(&a, cdiv(T_kv, G2_ATTN_CHUNK));
 }
 
+/* Whether a call fits one launch: a work-group per head takes up to
+ * G2_ATTN_GROUP chunks and writes its head while others may still read, so the
+ * output must not lie in what they read (the queries in place are its own
+ * head's).  Two launches read everything before they write. */
+int g2i_attn_one_launch(const float *q, const float *k_cache, const float *v_cache, const float *out, int T, int D, int S)
+{
+    const size_t f = sizeof(float), n = (size_t)D * f;
+    if (T <= 0 || T > G2_ATTN_GROUP * G2_ATTN_CHUNK) return 0;
+    return (out == q || !overlap(out, n, q, n)) && !overlap(out, n, k_cache, ((size_t)(D - 1) * S + T) * f) &&
+           !overlap(out, n, v_cache, (size_t)T * n);
+}
+
 int g2i_attn_launch(g2_attn1q_args *a, unsigned chunks)
 {
     const int vec = a->S % 4 == 0 && a->D % 4 == 0 && aligned(a->k_cache, 16) && aligned(a->v_cache, 16);
-    if (chunks <= G2_ATTN_GROUP && a->T_fixed > 0)
+    if (g2i_attn_one_launch(a->q, a->k_cache, a->v_cache, a->out, a->T_fixed, a->D, a->S))
         return g2i_launch(vec ? G2F_ATTN_SHORT : G2F_ATTN_SHORT_S, (unsigned)a->NH, 1, 256 * chunks, a);
     scratch_lock();
     int rc = g2i_launch(vec ? G2F_ATTN_PART : G2F_ATTN_PART_S, (unsigned)a->NH, chunks, 256, a);

@@ -61,6 +61,23 @@ def test_fused_lengths_in_a_row(g2, NH, S, shift):
             np.testing.assert_allclose(dO.download(np.float32, D), o, rtol=1e-4, atol=2e-5, err_msg=f"T {T}")
 
 
+@pytest.mark.parametrize("T", [1, 64, 200, 256, 300])
+def test_fused_output_in_its_operands(g2, T):
+    """An output over the queries (in place, and a head further), over keys
+    and over values in use: everything is read before it is written."""
+    NH, S = 20, 512
+    D = NH * 64
+    r = np.random.default_rng(T)
+    q, kc, vc = (r.standard_normal(n).astype(np.float32) for n in (2 * D, D * S, S * D))
+    o = reference(q[:D], kc, vc.reshape(S, D), T, NH, 64, 0.125)[2]
+    for fn in (g2.attn_1q, g2.attn_1q_noalloc):
+        for which, at in ((0, 0), (0, 64), (1, 0), (1, 5 * S + 3), (2, 0), (2, (T - 1) * D)):
+            bufs = [g2.to_device(x) for x in (q, kc, vc)]
+            fn(*bufs, bufs[which], 0, T, D, NH, S, at, 0.125)
+            got = bufs[which].download(np.float32, at + D)[at:]
+            np.testing.assert_allclose(got, o, rtol=1e-4, atol=2e-5, err_msg=f"operand {which} + {at}")
+
+
 @pytest.mark.parametrize("E,NH,P", [(128, 2, 1), (96, 6, 64), (160, 2, 65), (30, 2, 257), (256, 4, 1000)])
 def test_reference_prefill_attention(g2, E, NH, P):
     """The reference path's prompt attention (all rows in one launch) at head

@@ -1,0 +1,30 @@
+"""The operators' choice of kernel, on the CPU: which forms a call may take
+where its result lies in the memory of its operands.  A work-group of a
+one-launch form writes while others still read, so these calls take forms
+that read everything first; no GPU is involved, the addresses are numbers."""
+import ctypes as C
+
+import pytest
+
+import g2hip
+
+lib = C.CDLL(g2hip.LIB_PATH)
+F = 4
+
+
+@pytest.mark.parametrize("NH,S,T", [(1, 256, 256), (2, 1024, 1), (12, 1024, 200), (25, 700, 256)])
+def test_attention_in_one_launch_reads_what_it_does_not_write(NH, S, T):
+    fn = lib.g2i_attn_one_launch
+    fn.argtypes = [C.c_void_p] * 4 + [C.c_int] * 3
+    D = 64 * NH
+    q, k, v, out = 1 << 20, 1 << 24, 1 << 28, 1 << 30
+    kend, vend = k + ((D - 1) * S + T) * F, v + T * D * F
+    assert fn(q, k, v, out, T, D, S) == 1
+    assert fn(q, k, v, out, 257, D, S) == 0 and fn(q, k, v, out, 0, D, S) == 0  # too long; a length on the device
+    assert fn(q, k, v, q, T, D, S) == 1  # each head's queries, by the work-group that has read them
+    for o in (q + F, q - F, q + 64 * F, q + (D - 1) * F, q - (D - 1) * F):
+        assert fn(q, k, v, o, T, D, S) == (1 if D == 64 and abs(o - q) >= 64 * F else 0)
+    for o in (q + D * F, q - D * F, k - D * F, kend, v - D * F, vend):  # beside them
+        assert fn(q, k, v, o, T, D, S) == 1
+    for o in (k, k - (D - 1) * F, kend - F, v, v - (D - 1) * F, vend - F):
+        assert fn(q, k, v, o, T, D, S) == 0
