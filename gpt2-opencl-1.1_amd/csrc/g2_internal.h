@@ -142,6 +142,9 @@ int g2i_device_alloc(void **p, size_t bytes);
 int g2i_rows_launch(int fid_f32_64, int f16, g2_rows_args *a);
 /* Work-groups g2i_rows_launch uses for N rows of K (0 if K is invalid). */
 unsigned g2i_rows_grid(int N, int K, int f16);
+/* g2_matmul's form for M x N x K on num_cus CUs and its K splits (1 if whole). */
+enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128, XG_DUO };
+int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits);
 /* Single-query attention over `chunks` key chunks: one launch where
  * g2i_attn_one_launch allows it (lengths given by the caller, 0 otherwise),
  * else partials, then merge. */

@@ -26,10 +26,12 @@ extern const unsigned char g2_hsaco_end[];
 static const char *const g2_kernel_names[G2F_COUNT] = { G2_KERNEL_LIST(G2_NAME_ENTRY) };
 #undef G2_NAME_ENTRY
 
-/* Library scratch: K slices of g2_matvec (at most 8 of 65536 columns) and of
- * g2_matmul (as many as fit), and the attention chunk partials of
- * g2_attn_1q. */
-#define G2_SCRATCH_FLOATS ((size_t)64 * 65536)
+/* Library scratch: K slices of g2_matvec (at most 8 of 65536 columns) and the
+ * attention chunk partials of g2_attn_1q, which graphs that captured these
+ * calls go on using; K splits of g2_matmul (as many as fit), used by eager
+ * calls only. */
+#define G2_SCRATCH_FLOATS ((size_t)8 * 65536)
+#define G2_GEMM_PART_FLOATS ((size_t)64 * 65536)
 #define G2_ATTN_PART_FLOATS ((size_t)64 * G2_ATTN_MAX_CHUNKS * 66)
 
 static struct {
@@ -40,6 +42,7 @@ static struct {
     hipStream_t stream;
     hipFunction_t fn[G2F_COUNT];
     float *scratch;
+    float *gemm_part;
     float *attn_part;
     int noalloc_rc;         /* g2i_noalloc_setup result at g2_init */
     char noalloc_err[256];
@@ -178,9 +181,10 @@ int g2_init(int device)
         return rc;
     }
     rc = g2i_hip(hipMalloc((void **)&G.scratch, G2_SCRATCH_FLOATS * sizeof(float)), "scratch");
+    if (!rc) rc = g2i_hip(hipMalloc((void **)&G.gemm_part, G2_GEMM_PART_FLOATS * sizeof(float)), "matmul scratch");
     if (!rc) rc = g2i_hip(hipMalloc((void **)&G.attn_part, G2_ATTN_PART_FLOATS * sizeof(float)), "attn scratch");
     if (rc) {
-        hipFree(G.scratch); hipFree(G.attn_part);
+        hipFree(G.scratch); hipFree(G.gemm_part); hipFree(G.attn_part);
         hipStreamDestroy(G.stream); hipModuleUnload(G.module);
         memset(&G, 0, sizeof G);
         return rc;
@@ -236,6 +240,7 @@ int g2_shutdown(void)
     if (!G.ready) return G2_OK;
     hipStreamSynchronize(G.stream);
     hipFree(G.scratch);
+    hipFree(G.gemm_part);
     hipFree(G.attn_part);
     hipStreamDestroy(G.stream);
     hipModuleUnload(G.module);
@@ -327,17 +332,27 @@ static int overlap(const void *p, size_t np, const void *q, size_t nq)
     return (uintptr_t)p < (uintptr_t)q + nq && (uintptr_t)q < (uintptr_t)p + np;
 }
 
-/* The launches that write and read G.scratch are enqueued without another
+/* The launches that write and read a scratch buffer are enqueued without another
  * thread's between them; the stream then keeps their order. */
 static pthread_mutex_t g_scratch = PTHREAD_MUTEX_INITIALIZER;
 static void scratch_lock(void) { pthread_mutex_lock(&g_scratch); }
 static void scratch_unlock(void) { pthread_mutex_unlock(&g_scratch); }
 
+/* Whether the library's stream records a graph.  Its replays may run on any
+ * stream, beside each other and beside eager calls, so what is recorded of
+ * g2_matmul shares no buffer: forms without K splits. */
+static int capturing(void)
+{
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(G.stream, &s) != hipSuccess || s != hipStreamCaptureStatusNone;
+}
+
 /* The GEMM kernel for M x N x K, by the estimated time (us) of each form
  * (g2_matmul.hip): the direct form on 16- or 32-row tiles of 32 columns (K
  * steps of 32 dealt to 8 waves), 64 x 64 tiles and 128 x 128 tiles of two
  * alternating wave groups, both with K in ks splits added by a second launch,
- * and 128 x 128 tiles of two and more work-groups per CU.  A form's step costs its latency while
+ * and 128 x 128 tiles of two and more work-groups per CU; with `whole`, the
+ * forms without K splits.  A form's step costs its latency while
  * the CUs hold at most one work-group each, and its throughput times the
  * work-groups per CU beyond; up to nearly two, some CUs hold two and decide.
  * The constants are fitted to MI355X times of 45 shapes (8..1024 rows, 258 to
@@ -347,13 +362,11 @@ static void scratch_unlock(void) { pthread_mutex_unlock(&g_scratch); }
  * 512 x 1024 x 1024: 19 / 15 / 25 / 19 / 60; 256 x 1280 x 5120: 61 / 58 / 113
  * / 34 / 276; 333 x 6400 x 1600: 117 / 97 / 74 / - / 94; 1024 x 50257 x 1600:
  * - / - / 1200 / - / 880. */
-enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128, XG_DUO };
-
 static double xg_load(double per_cu) { return per_cu <= 1 ? per_cu : per_cu < 1.7 ? 1.7 : per_cu; }
 
-static int xg_pick(long M, long N, long K, int *splits)
+int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
 {
-    const double cus = g2i_cus(), steps = (double)((K + 31) / 32);
+    const double cus = num_cus, steps = (double)((K + 31) / 32);
     double best = 1e300;
     int pick = XG_64;
     *splits = 1;
@@ -365,7 +378,7 @@ static int xg_pick(long M, long N, long K, int *splits)
     }
     const double tiles = (double)((N + 63) / 64) * (double)((M + 63) / 64), mn = (double)M * (double)N;
     for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
-        if (ks > 1 && (ks * mn > (double)G2_SCRATCH_FLOATS || 2 * ks > steps)) break;
+        if (ks > 1 && (whole || ks * mn > (double)G2_GEMM_PART_FLOATS || 2 * ks > steps)) break;
         const double t = 0.3 + 0.42 * xg_load(tiles * ks / cus);
         double us = 3 + steps / ks * (t > 0.7 ? t : 0.7);
         if (ks > 1) us += 5 + (2 * ks + 1) * mn * sizeof(float) / 6e6;
@@ -377,7 +390,7 @@ static int xg_pick(long M, long N, long K, int *splits)
         if (us < best) { best = us; pick = XG_128; *splits = 1; }
         const double tiles = (double)((N + 127) / 128) * (double)((M + 127) / 128);
         for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
-            if (ks > 1 && (ks * mn > (double)G2_SCRATCH_FLOATS || 2 * ks > steps || tiles * ks > cus)) break;
+            if (ks > 1 && (whole || ks * mn > (double)G2_GEMM_PART_FLOATS || 2 * ks > steps || tiles * ks > cus)) break;
             /* a step with all CUs at it for several rounds: 1.4 us (1024 x
              * 50257 x 1600: 907 us against 871 on xgemm128, 753 against 686
              * with fp16 B) */
@@ -398,7 +411,9 @@ static int gemm_kn(int f16, const float *A, const void *B, const float *bias, fl
     g2_gemm_args a;
     memset(&a, 0, sizeof a);
     a.A = A; a.B = B; a.bias = bias; a.C = C; a.M = M; a.N = N; a.K = K;
-    const int pick = xg_pick(M, N, K, &a.ksplit), duo = pick == XG_DUO;
+    int pick = g2i_matmul_pick(g2i_cus(), M, N, K, 0, &a.ksplit);
+    if (a.ksplit > 1 && capturing()) pick = g2i_matmul_pick(g2i_cus(), M, N, K, 1, &a.ksplit);
+    const int duo = pick == XG_DUO;
     switch (pick) {
     case XG_DIRECT16:
         return g2i_launch(f16 ? G2F_XSKINNY1_F16 : G2F_XSKINNY1_F32, cdiv(N, 32) * cdiv(M, 16), 1, 512, &a);
@@ -412,7 +427,7 @@ static int gemm_kn(int f16, const float *A, const void *B, const float *bias, fl
     const int part = duo ? (f16 ? G2F_XDUO_PART_F16 : G2F_XDUO_PART_F32)
                          : (f16 ? G2F_XGEMM64_PART_F16 : G2F_XGEMM64_PART_F32);
     if (a.ksplit == 1) return g2i_launch(whole, tiles, 1, threads, &a);
-    a.part = G.scratch;
+    a.part = G.gemm_part;
     const unsigned sum = cdiv((long)M * N, 1024);
     scratch_lock();
     int rc = g2i_launch(part, tiles, (unsigned)a.ksplit, threads, &a);

@@ -61,6 +61,9 @@ int g2_device_name(char *buf, int len, int *compute_units);
  * reference, whose queue is main.c:537): every launch of the library goes to
  * it, so a caller may capture the library's calls into its own HIP graph
  * (hipStreamBeginCapture on this stream, the calls, hipStreamEndCapture).
+ * A recorded g2_matvec and g2_attn_1q may go on using a buffer of the library:
+ * replay graphs that hold them one after another and on this stream, or not
+ * beside other calls.  A recorded g2_matmul uses its operands only.
  * NULL before g2_init. */
 void *g2_stream(void);
 

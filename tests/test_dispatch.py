@@ -1,8 +1,12 @@
-"""The operators' choice of kernel, on the CPU: which forms a call may take
-where its result lies in the memory of its operands.  A work-group of a
-one-launch form writes while others still read, so these calls take forms
-that read everything first; no GPU is involved, the addresses are numbers."""
+"""The operators' choice of kernel, on the CPU.
+
+Which forms a call may take where its result lies in the memory of its
+operands: a work-group of a one-launch form writes while others still read, so
+these calls take forms that read everything first.  And g2_matmul's forms under
+graph capture, which share no buffer.  No GPU is involved, the addresses are
+numbers."""
 import ctypes as C
+import random
 
 import pytest
 
@@ -28,3 +32,23 @@ def test_attention_in_one_launch_reads_what_it_does_not_write(NH, S, T):
         assert fn(q, k, v, o, T, D, S) == 1
     for o in (k, k - (D - 1) * F, kend - F, v, v - (D - 1) * F, vend - F):
         assert fn(q, k, v, o, T, D, S) == 0
+
+
+def matmul_pick(M, N, K, whole=False, cus=256):
+    fn = lib.g2i_matmul_pick
+    fn.argtypes = [C.c_int] + [C.c_long] * 3 + [C.c_int, C.POINTER(C.c_int)]
+    splits = C.c_int()
+    return fn(cus, M, N, K, whole, C.byref(splits)), splits.value
+
+
+def test_captured_matmul_has_no_splits():
+    rng = random.Random(7)
+    split = 0
+    for _ in range(3000):
+        M, N, K = (int(2 ** rng.uniform(0, e)) for e in (10, 16, 14))
+        split += matmul_pick(M, N, K)[1] > 1
+        assert matmul_pick(M, N, K, whole=True)[1] == 1
+        form, ks = matmul_pick(M, N, K)
+        if ks == 1:  # without splits both choose alike
+            assert matmul_pick(M, N, K, whole=True) == (form, 1)
+    assert split > 100

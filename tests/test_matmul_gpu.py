@@ -6,6 +6,7 @@ in K splits, 128x128 tiles) on ragged edges: one row or column past a tile,
 odd column counts (a column pair that the last column begins), K below one
 step of 32, one past it, and splits that end in a partial step.
 """
+import ctypes as C
 import time
 
 import numpy as np
@@ -143,6 +144,47 @@ def test_matmul_time_by_values(g2, M, N, K):
     rows[:, K // 2] = np.inf
     assert seconds(rows, B) < 8 * plain
     assert seconds(A * np.float32(2.0 ** -125), B) < 8 * plain
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 200, 4100), (257, 5121, 1281)])
+def test_matmul_captured(g2, M, N, K):
+    """Sizes whose eager call splits K through the library's buffer: a recorded
+    call, replayed on a stream of its own beside eager split calls of other
+    operands, gives the recorded product every time, and the eager calls
+    theirs."""
+    hip, vp = C.CDLL("libamdhip64.so"), C.c_void_p
+    hip.hipStreamBeginCapture.argtypes = [vp, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [vp, C.POINTER(vp)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(vp), vp, vp, vp, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [vp, vp]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [vp]
+    hip.hipStreamCreateWithFlags.argtypes = [C.POINTER(vp), C.c_uint]
+    hip.hipStreamSynchronize.argtypes = hip.hipStreamDestroy.argtypes = [vp]
+    sets, dev = [operands(M, N, K, False, s) for s in (1, 2)], []
+    for A, B, bias in sets:
+        dev.append((g2.to_device(A), g2.to_device(B), g2.to_device(bias), g2.DevBuf(4 * M * N)))
+    refs = [(A.astype(np.float64) @ B.astype(np.float64) + bias) for A, B, bias in sets]
+    stream, side, graph, exe = g2._lib.g2_stream(), vp(), vp(), vp()
+    assert hip.hipStreamCreateWithFlags(C.byref(side), 1) == 0
+    g2.sync()
+    assert hip.hipStreamBeginCapture(stream, 1) == 0  # hipStreamCaptureModeThreadLocal
+    g2.matmul(*dev[0], M, N, K)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(exe), graph, None, None, 0) == 0
+    try:
+        for rep in range(20):
+            assert hip.hipGraphLaunch(exe, side) == 0
+            for _ in range(3):
+                g2.matmul(*dev[1], M, N, K)
+            assert hip.hipStreamSynchronize(side) == 0
+            g2.sync()
+            for d, ref in zip(dev, refs):
+                got = d[3].download(np.float32, M * N).reshape(M, N)
+                assert np.linalg.norm(got - ref) <= 2e-6 * np.linalg.norm(ref), f"replay {rep}"
+    finally:
+        hip.hipGraphExecDestroy(exe)
+        hip.hipGraphDestroy(graph)
+        hip.hipStreamDestroy(side)
 
 
 @pytest.mark.parametrize("P", [70, 300, 1000])
