@@ -145,6 +145,10 @@ unsigned g2i_rows_grid(int N, int K, int f16);
 /* g2_matmul's form for M x N x K on num_cus CUs and its K splits (1 if whole). */
 enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128, XG_DUO };
 int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits);
+/* Whether C lies in A or B: such a call takes XG_64 whole, whose work-groups
+ * read all that a tile needs before they write it, so a product of at most 64
+ * columns over its own A, or of one tile anywhere, is right. */
+int g2i_matmul_in_place(const float *A, const void *B, size_t b_size, const float *C, long M, long N, long K);
 /* Single-query attention over `chunks` key chunks: one launch where
  * g2i_attn_one_launch allows it (lengths given by the caller, 0 otherwise),
  * else partials, then merge. */

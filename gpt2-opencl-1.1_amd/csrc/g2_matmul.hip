@@ -346,6 +346,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
             for (int j = 0; j < JB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
         again_tile<BT, BNK>(a.A, B, M, N, K, m0 + wm * (BM / 2), n, s0 * 32, min(s1 * 32, K), acc);
+        __syncthreads(); /* before any wave writes: C may lie in A or B */
     }
 
     float *C = EPI == GEPI_PARTIAL ? a.part + (size_t)blockIdx.y * M * N : a.C;

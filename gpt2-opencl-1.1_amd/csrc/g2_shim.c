@@ -364,6 +364,12 @@ static int capturing(void)
  * - / - / 1200 / - / 880. */
 static double xg_load(double per_cu) { return per_cu <= 1 ? per_cu : per_cu < 1.7 ? 1.7 : per_cu; }
 
+int g2i_matmul_in_place(const float *A, const void *B, size_t b_size, const float *C, long M, long N, long K)
+{
+    const size_t nc = (size_t)M * N * sizeof(float);
+    return overlap(C, nc, A, (size_t)M * K * sizeof(float)) || overlap(C, nc, B, (size_t)K * N * b_size);
+}
+
 int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
 {
     const double cus = num_cus, steps = (double)((K + 31) / 32);
@@ -412,7 +418,10 @@ static int gemm_kn(int f16, const float *A, const void *B, const float *bias, fl
     memset(&a, 0, sizeof a);
     a.A = A; a.B = B; a.bias = bias; a.C = C; a.M = M; a.N = N; a.K = K;
     int pick = g2i_matmul_pick(g2i_cus(), M, N, K, 0, &a.ksplit);
-    if (a.ksplit > 1 && capturing()) pick = g2i_matmul_pick(g2i_cus(), M, N, K, 1, &a.ksplit);
+    if (g2i_matmul_in_place(A, B, f16 ? 2 : 4, C, M, N, K)) {
+        pick = XG_64;
+        a.ksplit = 1;
+    } else if (a.ksplit > 1 && capturing()) pick = g2i_matmul_pick(g2i_cus(), M, N, K, 1, &a.ksplit);
     const int duo = pick == XG_DUO;
     switch (pick) {
     case XG_DIRECT16:

@@ -52,3 +52,14 @@ def test_captured_matmul_has_no_splits():
         if ks == 1:  # without splits both choose alike
             assert matmul_pick(M, N, K, whole=True) == (form, 1)
     assert split > 100
+
+
+@pytest.mark.parametrize("b_size", [4, 2])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (64, 64, 64), (300, 48, 48), (10, 2000, 700)])
+def test_matmul_over_its_operands(M, N, K, b_size):
+    fn = lib.g2i_matmul_in_place
+    fn.argtypes = [C.c_void_p] * 2 + [C.c_size_t, C.c_void_p] + [C.c_long] * 3
+    A, B = 1 << 30, 1 << 32
+    for base, size in ((A, M * K * F), (B, K * N * b_size)):
+        for at, over in ((0, 1), (size - b_size, 1), (size, 0), (F - M * N * F, 1), (-M * N * F, 0)):
+            assert fn(A, B, b_size, base + at, M, N, K) == over

@@ -146,6 +146,20 @@ def test_matmul_time_by_values(g2, M, N, K):
     assert seconds(A * np.float32(2.0 ** -125), B) < 8 * plain
 
 
+@pytest.mark.parametrize("small", [False, True], ids=["ordinary", "recomputed"])
+@pytest.mark.parametrize("M,N", [(1, 64), (5, 33), (64, 64), (300, 64), (2000, 17)])
+def test_matmul_over_a(g2, M, N, small):
+    """X = X W in place, W of at most 64 columns; also where tiles are
+    computed again on the fp32 instruction."""
+    A, B, bias = operands(M, N, N, False, 6)
+    if small:
+        A, B = A * np.float32(2.0 ** -120), B * np.float32(2.0 ** 120)
+    dA = g2.to_device(A)
+    g2.matmul(dA, g2.to_device(B), g2.to_device(bias), dA, M, N, N)
+    bound = dot_bound(np.abs(A).astype(np.float64), np.abs(B).astype(np.float64), N)
+    assert_close_bound(dA.download(np.float32, M * N).reshape(M, N), oracle.matmul(A, B, bias, M, N, N), bound, what="in place")
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 200, 4100), (257, 5121, 1281)])
 def test_matmul_captured(g2, M, N, K):
     """Sizes whose eager call splits K through the library's buffer: a recorded
