@@ -149,6 +149,7 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
  * read all that a tile needs before they write it, so a product of at most 64
  * columns over its own A, or of one tile anywhere, is right. */
 int g2i_matmul_in_place(const float *A, const void *B, size_t b_size, const float *C, long M, long N, long K);
+int g2i_attn_out_groups(const float *scores, const float *v_cache, const float *out, int T, int D, int DH);
 /* Single-query attention over `chunks` key chunks: one launch where
  * g2i_attn_one_launch allows it (lengths given by the caller, 0 otherwise),
  * else partials, then merge. */

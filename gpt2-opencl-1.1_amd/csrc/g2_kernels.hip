@@ -517,36 +517,43 @@ G2K void g2k_attn_softmax(const g2_softmax_args a)
     }
 }
 
-/* ---- attn_out_1q (math.cl:459-476): grid ceil(D/16), block 1024: 16 dims x
- * 64 positions at a time (j = row, row + 64, ...), four ahead; the 64 sums of
- * a dim are added over a wave's four rows, then over the 16 waves in order. */
+/* ---- attn_out_1q (math.cl:459-476): block 1024: 16 dims x 64 positions at a
+ * time (j = row, row + 64, ...), four ahead; the 64 sums of a dim are added
+ * over a wave's four rows, then over the 16 waves in order.  Grid
+ * ceil(D / (16 groups)), groups <= 4 of 16 dims one after the other, written
+ * when all are done. */
 extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout_args a)
 {
-    __shared__ float red[16][16];
-    const int tid = threadIdx.x, d = blockIdx.x * 16 + (tid & 15), dc = min(d, a.D - 1);
-    const float *srow = a.scores + (size_t)(dc / a.DH) * G2_KV_MAX_SEQ;
-    float o = 0.f;
-    for (int j0 = tid >> 4; j0 < a.T; j0 += 256) {
-        float p[4], v[4];
+    __shared__ float red[16][16], res[64];
+    const int tid = threadIdx.x, d0 = blockIdx.x * 16 * a.groups;
+    for (int g = 0; g < a.groups; ++g) {
+        const int dc = min(d0 + 16 * g + (tid & 15), a.D - 1);
+        const float *srow = a.scores + (size_t)(dc / a.DH) * G2_KV_MAX_SEQ;
+        float o = 0.f;
+        for (int j0 = tid >> 4; j0 < a.T; j0 += 256) {
+            float p[4], v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = j0 + 64 * u;
-            p[u] = j < a.T ? srow[j] : 0.f;
-            v[u] = j < a.T ? a.v_cache[(size_t)j * a.D + dc] : 0.f;
+            for (int u = 0; u < 4; ++u) {
+                const int j = j0 + 64 * u;
+                p[u] = j < a.T ? srow[j] : 0.f;
+                v[u] = j < a.T ? a.v_cache[(size_t)j * a.D + dc] : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) o = fmaf(p[u], v[u], o);
         }
+        o += __shfl_xor(o, 16);
+        o += __shfl_xor(o, 32);
+        if ((tid & 63) < 16) red[tid >> 6][tid & 15] = o;
+        __syncthreads();
+        if (tid < 16) {
+            float s = 0.f;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) o = fmaf(p[u], v[u], o);
+            for (int w = 0; w < 16; ++w) s += red[w][tid];
+            res[16 * g + tid] = s;
+        }
+        __syncthreads();
     }
-    o += __shfl_xor(o, 16);
-    o += __shfl_xor(o, 32);
-    if ((tid & 63) < 16) red[tid >> 6][tid & 15] = o;
-    __syncthreads();
-    if (tid < 16 && d < a.D) {
-        float s = 0.f;
-#pragma unroll
-        for (int w = 0; w < 16; ++w) s += red[w][tid];
-        a.out[a.out_base + d] = s;
-    }
+    if (tid < 16 * a.groups && d0 + tid < a.D) a.out[a.out_base + d0 + tid] = res[tid];
 }
 
 /* ---- a prompt's attention on the reference path: the three operators above

@@ -621,6 +621,15 @@ int g2_attn_softmax_1q(float *scores, int T_kv, int NH)
     return g2i_launch(G2F_ATTN_SOFTMAX, (unsigned)NH, 1, 256, &a);
 }
 
+/* 16-dim groups of a work-group: one, for four times the work-groups; four
+ * where the output lies in the operands (up to 64 dims are then one
+ * work-group's, read before they are written). */
+int g2i_attn_out_groups(const float *scores, const float *v_cache, const float *out, int T, int D, int DH)
+{
+    const size_t f = sizeof(float), n = (size_t)D * f, heads = (size_t)(D - 1) / (size_t)DH;
+    return overlap(out, n, scores, (heads * G2_MAX_SEQ + (size_t)T) * f) || overlap(out, n, v_cache, (size_t)T * n) ? 4 : 1;
+}
+
 int g2_attn_out_1q(const float *scores, const float *v_cache, float *out, int T_kv, int D,
                    int DH, int out_base)
 {
@@ -628,8 +637,9 @@ int g2_attn_out_1q(const float *scores, const float *v_cache, float *out, int T_
     if (!scores || !v_cache || !out) return g2i_err(G2_E_ARG, "g2_attn_out_1q: NULL buffer");
     if (T_kv <= 0 || T_kv > G2_MAX_SEQ || D <= 0 || DH <= 0 || out_base < 0)
         return g2i_err(G2_E_ARG, "g2_attn_out_1q: bad sizes");
-    g2_attnout_args a = { scores, v_cache, out, T_kv, D, DH, out_base };
-    return g2i_launch(G2F_ATTN_OUT, cdiv(D, 16), 1, 1024, &a);
+    g2_attnout_args a = { scores, v_cache, out, T_kv, D, DH, out_base,
+                          g2i_attn_out_groups(scores, v_cache, out + out_base, T_kv, D, DH) };
+    return g2i_launch(G2F_ATTN_OUT, cdiv(D, 16 * a.groups), 1, 1024, &a);
 }
 
 int g2_attn_1q(const float *qkv, const float *k_cache, const float *v_cache, float *out,

@@ -78,6 +78,20 @@ def test_fused_output_in_its_operands(g2, T):
             np.testing.assert_allclose(got, o, rtol=1e-4, atol=2e-5, err_msg=f"operand {which} + {at}")
 
 
+@pytest.mark.parametrize("D,DH,T", [(64, 64, 300), (64, 16, 1), (50, 25, 1024), (7, 7, 65)])
+def test_weighted_sum_over_its_operands(g2, D, DH, T):
+    """Up to 64 dims over the scores or the values that they are summed from."""
+    NH = D // DH
+    r = np.random.default_rng(D + T)
+    p, v = r.random((NH, 1024), np.float32), r.standard_normal((T, D)).astype(np.float32)
+    ref = np.einsum("ht,thd->hd", p[:, :T].astype(np.float64), v.astype(np.float64).reshape(T, NH, DH)).ravel()
+    for which, at in ((0, 0), (0, max(T - D, 0)), (1, 0), (1, (T - 1) * D)):
+        bufs = [g2.to_device(p), g2.to_device(v)]
+        g2.attn_out_1q(bufs[0], bufs[1], bufs[which], T, D, DH, at)
+        got = bufs[which].download(np.float32, at + D)[at:]
+        np.testing.assert_allclose(got, ref, rtol=1e-5, atol=2e-5 * np.sqrt(T), err_msg=f"operand {which} + {at}")
+
+
 @pytest.mark.parametrize("E,NH,P", [(128, 2, 1), (96, 6, 64), (160, 2, 65), (30, 2, 257), (256, 4, 1000)])
 def test_reference_prefill_attention(g2, E, NH, P):
     """The reference path's prompt attention (all rows in one launch) at head

@@ -34,6 +34,16 @@ def test_attention_in_one_launch_reads_what_it_does_not_write(NH, S, T):
         assert fn(q, k, v, o, T, D, S) == 0
 
 
+def test_attention_output_over_its_operands():
+    fn = lib.g2i_attn_out_groups
+    fn.argtypes = [C.c_void_p] * 3 + [C.c_int] * 3
+    scores, v = 1 << 24, 1 << 28
+    for D, DH, T in ((64, 64, 300), (48, 16, 7), (10, 1, 1)):
+        for base, size in ((scores, ((D - 1) // DH * 1024 + T) * F), (v, T * D * F)):
+            for at, groups in ((0, 4), (size - F, 4), (size, 1), (F - D * F, 4), (-D * F, 1)):
+                assert fn(scores, v, base + at, T, D, DH) == groups
+
+
 def matmul_pick(M, N, K, whole=False, cus=256):
     fn = lib.g2i_matmul_pick
     fn.argtypes = [C.c_int] + [C.c_long] * 3 + [C.c_int, C.POINTER(C.c_int)]
