@@ -142,6 +142,10 @@ int g2i_device_alloc(void **p, size_t bytes);
 int g2i_rows_launch(int fid_f32_64, int f16, g2_rows_args *a);
 /* Work-groups g2i_rows_launch uses for N rows of K (0 if K is invalid). */
 unsigned g2i_rows_grid(int N, int K, int f16);
+/* Whether a matvec's result lies in none of its operands, but for a bias or
+ * residual exactly in place: then one launch may write while it reads. */
+int g2i_matvec_apart(const float *A, const void *B, size_t b_size, const float *bias, const float *res, const float *C,
+                     int N, int K);
 /* g2_matmul's form for M x N x K on num_cus CUs and its K splits (1 if whole). */
 enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128, XG_DUO };
 int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits);

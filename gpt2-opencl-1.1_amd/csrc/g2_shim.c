@@ -474,7 +474,16 @@ static int matvec_launch(int f16, g2_matvec_args *a)
 /* One launch, except: a tall narrow matrix (its few work-groups would walk
  * over 128 KB each) goes in slices to the scratch, added by a second launch
  * (1600 x 6400 fp32 11 us + the launch against 20, 768 x 3072 7 against 13);
- * so does a product into memory that holds its operands. */
+ * so does a product into memory that holds its operands (bias and residual in
+ * place are read by the thread that writes there). */
+int g2i_matvec_apart(const float *A, const void *B, size_t b_size, const float *bias, const float *res, const float *C,
+                     int N, int K)
+{
+    const size_t n = (size_t)N * sizeof(float);
+    return !overlap(C, n, A, (size_t)K * sizeof(float)) && !overlap(C, n, B, (size_t)N * K * b_size) &&
+           (!bias || bias == C || !overlap(C, n, bias, n)) && (!res || res == C || !overlap(C, n, res, n));
+}
+
 static int matvec_any(int f16, const float *A, const void *B, const float *bias,
                       const float *res, float *C, int N, int K, int gelu)
 {
@@ -485,9 +494,7 @@ static int matvec_any(int f16, const float *A, const void *B, const float *bias,
     const unsigned narrow = cdiv(N, f16 ? 32 : 16);
     unsigned slices = 1;
     if (K > 2048 && narrow < 160) slices = cdiv(256, narrow) < 8 ? cdiv(256, narrow) : 8;
-    const size_t nc = (size_t)N * sizeof(float);
-    if (slices == 1 && !overlap(C, nc, A, (size_t)K * sizeof(float)) &&
-        !overlap(C, nc, B, (size_t)N * K * (f16 ? 2 : 4))) {
+    if (slices == 1 && g2i_matvec_apart(A, B, f16 ? 2 : 4, bias, res, C, N, K)) {
         g2_matvec_args a = { A, B, C, bias, res, N, K, 1, gelu ? 1 : 0 };
         return matvec_launch(f16, &a);
     }
@@ -519,6 +526,10 @@ static int matvec_sk_any(int f16, const float *A, const void *B, float *partial,
     if (!A || !B || !partial) return g2i_err(G2_E_ARG, "g2_matvec_sk: NULL buffer");
     if (N <= 0 || K <= 0 || (N & 3)) return g2i_err(G2_E_ARG, "g2_matvec_sk: N must be a positive multiple of 4");
     if (kslice < 1 || kslice > 8) return g2i_err(G2_E_ARG, "g2_matvec_sk: kslice %d not in 1..8", kslice);
+    /* one slice over its operands goes as g2_matvec does; of several, one would
+     * write what the others read in any form */
+    if (kslice == 1 && N <= 65536 && !g2i_matvec_apart(A, B, f16 ? 2 : 4, NULL, NULL, partial, N, K))
+        return matvec_any(f16, A, B, NULL, NULL, partial, N, K, 0);
     g2_matvec_args a = { A, B, partial, NULL, NULL, N, K, kslice, 0 };
     return matvec_launch(f16, &a);
 }

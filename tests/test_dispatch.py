@@ -44,6 +44,20 @@ def test_attention_output_over_its_operands():
                 assert fn(scores, v, base + at, T, D, DH) == groups
 
 
+@pytest.mark.parametrize("b_size", [4, 2])
+@pytest.mark.parametrize("N,K", [(1, 1), (64, 300), (700, 20)])
+def test_matvec_over_its_operands(N, K, b_size):
+    fn = lib.g2i_matvec_apart
+    fn.argtypes = [C.c_void_p] * 2 + [C.c_size_t] + [C.c_void_p] * 3 + [C.c_int] * 2
+    A, B, bias, res = 1 << 24, 1 << 28, 1 << 30, 1 << 31
+    for base, size in ((A, K * F), (B, N * K * b_size), (bias, N * F), (res, N * F)):
+        for at in (0, size - b_size, F - N * F, size, -N * F):
+            apart = at in (size, -N * F) or (at == 0 and base in (bias, res))
+            assert fn(A, B, b_size, bias, res, base + at, N, K) == apart
+            if base in (bias, res):
+                assert fn(A, B, b_size, None, None, base + at, N, K) == 1
+
+
 def matmul_pick(M, N, K, whole=False, cus=256):
     fn = lib.g2i_matmul_pick
     fn.argtypes = [C.c_int] + [C.c_long] * 3 + [C.c_int, C.POINTER(C.c_int)]

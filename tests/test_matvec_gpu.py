@@ -50,6 +50,31 @@ def test_matvec_in_place(g2, N, K):
     assert_close_bound(dA.download(np.float32, N), exact(A, B, bias, res), dot_bound(np.abs(A), np.abs(B), K), what="in place")
 
 
+@pytest.mark.parametrize("N", [33, 64])
+@pytest.mark.parametrize("shift", [-1, 1, 16])
+def test_matvec_over_a_shifted_residual(g2, N, shift):
+    """Up to 64 columns, a wave's, over the residual or the bias a few elements on."""
+    A, B, bias, res = operands(N, 300, False, 8)
+    ref, bound = exact(A, B, bias, res), dot_bound(np.abs(A), np.abs(B), 300)
+    pad = np.zeros(16, np.float32)
+    for which in (0, 1):
+        held = g2.to_device(np.concatenate([pad, (bias, res)[which], pad]))
+        other = g2.to_device((res, bias)[which])
+        pair = (held.offset(64), other) if which == 0 else (other, held.offset(64))
+        g2.matvec(g2.to_device(A), g2.to_device(B), *pair, held.offset(64 + 4 * shift), N, 300)
+        got = held.download(np.float32, N + 32)[16 + shift:][:N]
+        assert_close_bound(got, ref, bound, what="shifted")
+
+
+@pytest.mark.parametrize("N,K", [(256, 256), (64, 700), (128, 128)])
+def test_matvec_sk_in_place(g2, N, K):
+    """One slice over A, up to 256 columns."""
+    A, B, _, _ = operands(N, K, False, 10)
+    dA = g2.to_device(A)
+    g2.matvec_sk(dA, g2.to_device(B), dA, N, K, 1)
+    assert_close_bound(dA.download(np.float32, N), exact(A, B, 0, 0), dot_bound(np.abs(A), np.abs(B), K), what="in place")
+
+
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
 @pytest.mark.parametrize("N,K,ks", [(4, 3, 8), (12, 2, 5), (36, 1025, 3), (1028, 700, 7), (2564, 6400, 8)])
 def test_matvec_sk_edges(g2, N, K, ks, f16):
