@@ -146,8 +146,14 @@ unsigned g2i_rows_grid(int N, int K, int f16);
  * residual exactly in place: then one launch may write while it reads. */
 int g2i_matvec_apart(const float *A, const void *B, size_t b_size, const float *bias, const float *res, const float *C,
                      int N, int K);
+/* Columns of one matvec launch, 16 threads to a column at this width and fewer
+ * than 2^32 in a launch: more go in several. */
+#define G2_MV_LAUNCH_COLS (1l << 27)
 /* g2_matmul's form for M x N x K on num_cus CUs and its K splits (1 if whole). */
 enum { XG_DIRECT16, XG_DIRECT32, XG_64, XG_128, XG_DUO };
+/* Rows of N columns that one launch of XG_64 takes (its threads stay below
+ * 2^32; 0 where one row of tiles is too wide); more go in several. */
+long g2i_matmul_rows(long N);
 int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits);
 /* Whether C lies in A or B: such a call takes XG_64 whole, whose work-groups
  * read all that a tile needs before they write it, so a product of at most 64

@@ -109,16 +109,17 @@ typedef struct {
 } g2_skepi_args;
 #define G2_SKEPI_MAXKS 12 /* slices g2k_splitk_epi reads */
 
-/* Reference-layout matvec B[K,N]: slice s of nslice sums k = s, s + nslice,
- * ... (math.cl:229-246) to out[s*N + n], then + bias, + residual, GELU (each
- * optional; NULL, NULL, 0 with slices).  Grid (column groups, nslice). */
+/* Reference-layout matvec, N columns of B[K,ld]: slice s of nslice sums k = s,
+ * s + nslice, ... (math.cl:229-246) to out[s*ld + n], then + bias, + residual,
+ * GELU (each optional; NULL, NULL, 0 with slices).  Grid (column groups,
+ * nslice). */
 typedef struct {
     const float *A;
     const void *B;
     float *out;
     const float *bias;
     const float *residual;
-    int N, K, nslice, apply_gelu;
+    int N, K, nslice, apply_gelu, ld;
 } g2_matvec_args;
 
 /* reduce_partial (math.cl:249-280). */

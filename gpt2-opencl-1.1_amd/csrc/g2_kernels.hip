@@ -118,14 +118,14 @@ __device__ void matvec_impl(const g2_matvec_args &a)
     typedef _Float16 f16x8u __attribute__((ext_vector_type(8), aligned(2)));
     __shared__ float red[16][CL * V];
     const int tid = threadIdx.x, cl = tid & (CL - 1), rg = tid / CL;
-    const int N = a.N, K = a.K, ns = a.nslice;
+    const int N = a.N, K = a.K, ns = a.nslice, ld = a.ld;
     const int col = (blockIdx.x * CL + cl) * V, base = min(col, max(N - V, 0));
     const WT *B = (const WT *)a.B + base;
     float acc[V];
 #pragma unroll
     for (int e = 0; e < V; ++e) acc[e] = 0.f;
     auto row = [&](int k, float (&w)[V]) {
-        const WT *p = B + (size_t)k * N;
+        const WT *p = B + (size_t)k * ld;
         if (N < V) { /* one vector would leave the row */
 #pragma unroll
             for (int e = 0; e < V; ++e) w[e] = e < N ? (float)p[e] : 0.f;
@@ -186,7 +186,7 @@ __device__ void matvec_impl(const g2_matvec_args &a)
     if (a.bias) v += a.bias[n];
     if (a.residual) v += a.residual[n];
     if (a.apply_gelu) v = gelu_f(v);
-    a.out[(size_t)blockIdx.y * N + n] = v;
+    a.out[(size_t)blockIdx.y * ld + n] = v;
 }
 #define G2_MATVEC(name, WT, CL) \
     extern "C" __global__ __launch_bounds__(1024) void name(const g2_matvec_args a) { matvec_impl<WT, CL>(a); }

@@ -370,6 +370,11 @@ int g2i_matmul_in_place(const float *A, const void *B, size_t b_size, const floa
     return overlap(C, nc, A, (size_t)M * K * sizeof(float)) || overlap(C, nc, B, (size_t)K * N * b_size);
 }
 
+/* Threads of a launch: fewer than 2^32. */
+static int grid_fits(long tiles, long threads) { return tiles <= (long)(UINT32_MAX / (unsigned)threads); }
+
+long g2i_matmul_rows(long N) { return 64 * ((long)(UINT32_MAX / 256u) / ((N + 63) / 64)); }
+
 int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
 {
     const double cus = num_cus, steps = (double)((K + 31) / 32);
@@ -380,7 +385,7 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
         const double per_cu = xg_load((double)((N + 31) / 32) * (double)((M + 16 * r - 1) / (16 * r)) / cus);
         const double t = r == 1 ? per_cu : 1.6 * per_cu, latency = r == 1 ? 1.0 : 1.4;
         const double us = 3 + (double)(long)((steps + 7) / 8) * (t > latency ? t : latency);
-        if (us < best) { best = us; pick = r == 1 ? XG_DIRECT16 : XG_DIRECT32; }
+        if (us < best && grid_fits(((N + 31) / 32) * ((M + 16 * r - 1) / (16 * r)), 512)) { best = us; pick = r == 1 ? XG_DIRECT16 : XG_DIRECT32; }
     }
     const double tiles = (double)((N + 63) / 64) * (double)((M + 63) / 64), mn = (double)M * (double)N;
     for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
@@ -391,10 +396,10 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
         if (us < best) { best = us; pick = XG_64; *splits = ks; }
     }
     if (N >= 2) {
-        const double t = 0.5 + 1.25 * ((double)((N + 127) / 128) * (double)((M + 127) / 128) / cus);
-        const double us = 3 + steps * (t > 1.85 ? t : 1.85);
-        if (us < best) { best = us; pick = XG_128; *splits = 1; }
         const double tiles = (double)((N + 127) / 128) * (double)((M + 127) / 128);
+        const double t = 0.5 + 1.25 * (tiles / cus);
+        const double us = 3 + steps * (t > 1.85 ? t : 1.85);
+        if (us < best && grid_fits((long)tiles, 256)) { best = us; pick = XG_128; *splits = 1; }
         for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
             if (ks > 1 && (whole || ks * mn > (double)G2_GEMM_PART_FLOATS || 2 * ks > steps || tiles * ks > cus)) break;
             /* a step with all CUs at it for several rounds: 1.4 us (1024 x
@@ -402,7 +407,7 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
              * with fp16 B) */
             double duo = 4 + steps / ks * (tiles * ks > cus ? 1.4 : 1.05) * ceil(tiles * ks / cus);
             if (ks > 1) duo += 5 + ks * mn * sizeof(float) * (1 / 2.6e6 + 1 / 6e6);
-            if (duo < best) { best = duo; pick = XG_DUO; *splits = ks; }
+            if (duo < best && grid_fits((long)tiles, 512)) { best = duo; pick = XG_DUO; *splits = ks; }
         }
     }
     return pick;
@@ -417,6 +422,11 @@ static int gemm_kn(int f16, const float *A, const void *B, const float *bias, fl
     g2_gemm_args a;
     memset(&a, 0, sizeof a);
     a.A = A; a.B = B; a.bias = bias; a.C = C; a.M = M; a.N = N; a.K = K;
+    const long most = g2i_matmul_rows(N);
+    if (M > most && most > 0) { /* beyond one launch of any form: some rows, then the rest */
+        const int rc = gemm_kn(f16, A, B, bias, C, (int)most, N, K);
+        return rc ? rc : gemm_kn(f16, A + (size_t)most * K, B, bias, C + (size_t)most * N, (int)(M - most), N, K);
+    }
     int pick = g2i_matmul_pick(g2i_cus(), M, N, K, 0, &a.ksplit);
     if (g2i_matmul_in_place(A, B, f16 ? 2 : 4, C, M, N, K)) {
         pick = XG_64;
@@ -468,7 +478,16 @@ static int matvec_launch(int f16, g2_matvec_args *a)
     int shape = 2; /* CL = 4 << shape */
     while (shape > 0 && cdiv(a->N, (4u << shape) * v) * (unsigned)a->nslice < 160) --shape;
     const int fid = (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + 2 * shape;
-    return g2i_launch(fid, cdiv(a->N, (4u << shape) * v), (unsigned)a->nslice, 1024, a);
+    const long N = a->N;
+    for (long n0 = 0; n0 < N; n0 += G2_MV_LAUNCH_COLS) { /* (no bias or residual where N is above one launch) */
+        g2_matvec_args w = *a;
+        w.N = (int)(N - n0 < G2_MV_LAUNCH_COLS ? N - n0 : G2_MV_LAUNCH_COLS);
+        w.B = (const char *)a->B + n0 * (f16 ? 2 : 4);
+        w.out = a->out + n0;
+        const int rc = g2i_launch(fid, cdiv(w.N, (4u << shape) * v), (unsigned)a->nslice, 1024, &w);
+        if (rc) return rc;
+    }
+    return G2_OK;
 }
 
 /* One launch, except: a tall narrow matrix (its few work-groups would walk
@@ -495,10 +514,10 @@ static int matvec_any(int f16, const float *A, const void *B, const float *bias,
     unsigned slices = 1;
     if (K > 2048 && narrow < 160) slices = cdiv(256, narrow) < 8 ? cdiv(256, narrow) : 8;
     if (slices == 1 && g2i_matvec_apart(A, B, f16 ? 2 : 4, bias, res, C, N, K)) {
-        g2_matvec_args a = { A, B, C, bias, res, N, K, 1, gelu ? 1 : 0 };
+        g2_matvec_args a = { A, B, C, bias, res, N, K, 1, gelu ? 1 : 0, N };
         return matvec_launch(f16, &a);
     }
-    g2_matvec_args a = { A, B, G.scratch, NULL, NULL, N, K, (int)slices, 0 };
+    g2_matvec_args a = { A, B, G.scratch, NULL, NULL, N, K, (int)slices, 0, N };
     g2_reduce_args r = { G.scratch, bias, res, C, N, (int)slices, gelu ? 1 : 0 };
     scratch_lock();
     int rc = matvec_launch(f16, &a);
@@ -530,7 +549,7 @@ static int matvec_sk_any(int f16, const float *A, const void *B, float *partial,
      * write what the others read in any form */
     if (kslice == 1 && N <= 65536 && !g2i_matvec_apart(A, B, f16 ? 2 : 4, NULL, NULL, partial, N, K))
         return matvec_any(f16, A, B, NULL, NULL, partial, N, K, 0);
-    g2_matvec_args a = { A, B, partial, NULL, NULL, N, K, kslice, 0 };
+    g2_matvec_args a = { A, B, partial, NULL, NULL, N, K, kslice, 0, N };
     return matvec_launch(f16, &a);
 }
 
@@ -638,6 +657,7 @@ int g2_attn_softmax_1q(float *scores, int T_kv, int NH)
 int g2i_attn_out_groups(const float *scores, const float *v_cache, const float *out, int T, int D, int DH)
 {
     const size_t f = sizeof(float), n = (size_t)D * f, heads = (size_t)(D - 1) / (size_t)DH;
+    if (D > 1 << 24) return 4; /* a launch has fewer than 2^32 threads */
     return overlap(out, n, scores, (heads * G2_MAX_SEQ + (size_t)T) * f) || overlap(out, n, v_cache, (size_t)T * n) ? 4 : 1;
 }
 

@@ -92,6 +92,18 @@ def test_weighted_sum_over_its_operands(g2, D, DH, T):
         np.testing.assert_allclose(got, ref, rtol=1e-5, atol=2e-5 * np.sqrt(T), err_msg=f"operand {which} + {at}")
 
 
+def test_weighted_sum_wider_than_a_launch_of_16_dims(g2):
+    """2^26 + 20 dims, 64 threads each were 2^32."""
+    D = (1 << 26) + 20
+    v = (np.arange(D) % 1000).astype(np.float32)
+    p = np.zeros((1, 1024), np.float32)
+    p[0, 0] = 0.5
+    dO = g2.to_device(np.full(D + 1, 7.0, np.float32))
+    g2.attn_out_1q(g2.to_device(p), g2.to_device(v), dO, 1, D, D, 0)
+    got = dO.download(np.float32, D + 1)
+    assert (got[:D] == v / 2).all() and got[D] == 7.0
+
+
 @pytest.mark.parametrize("E,NH,P", [(128, 2, 1), (96, 6, 64), (160, 2, 65), (30, 2, 257), (256, 4, 1000)])
 def test_reference_prefill_attention(g2, E, NH, P):
     """The reference path's prompt attention (all rows in one launch) at head

@@ -87,3 +87,25 @@ def test_matmul_over_its_operands(M, N, K, b_size):
     for base, size in ((A, M * K * F), (B, K * N * b_size)):
         for at, over in ((0, 1), (size - b_size, 1), (size, 0), (F - M * N * F, 1), (-M * N * F, 0)):
             assert fn(A, B, b_size, base + at, M, N, K) == over
+
+
+def test_matmul_launches_stay_below_the_thread_limit():
+    """Sizes up to all of the memory: at most g2i_matmul_rows rows a call, in a
+    form whose launch has fewer than 2^32 threads."""
+    rows = lib.g2i_matmul_rows
+    rows.argtypes, rows.restype = [C.c_long], C.c_long
+    tile = [(16, 32, 512), (32, 32, 512), (64, 64, 256), (128, 128, 256), (128, 128, 512)]
+    rng = random.Random(3)
+    narrowed = 0
+    for _ in range(20000):
+        N, K = (int(2 ** rng.uniform(0, e)) for e in (30, 12))
+        if 2 * N * K > 2 ** 38 or rows(N) < 1:
+            continue
+        M = min(int(2 ** rng.uniform(0, 30)), max(1, 2 ** 36 // N))
+        narrowed += M > rows(N)
+        M = min(M, rows(N))
+        form, ks = matmul_pick(M, N, K)
+        bm, bn, threads = tile[form]
+        assert -(-M // bm) * -(-N // bn) * threads < 2 ** 32, (M, N, K, form)
+    assert narrowed > 10
+    assert rows(2 ** 30 - 64) == 64 and rows(2 ** 30) == 0

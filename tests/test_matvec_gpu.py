@@ -89,6 +89,20 @@ def test_matvec_sk_edges(g2, N, K, ks, f16):
         assert_close_bound(got[s * N:(s + 1) * N], ref[s], bound, what=f"slice {s}")
 
 
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+def test_matvec_sk_wider_than_a_launch(g2, f16):
+    """2^28 + 4 columns (16 threads each would be 2^32): several launches,
+    whose last has fewer columns than an fp16 vector."""
+    N = (1 << 28) + 4
+    B = np.arange(N, dtype=np.uint32).astype(np.uint16) % 1000
+    B = (g2.convert_f16(np.arange(1000, dtype=np.float32)) if f16 else np.arange(1000, dtype=np.float32))[B]
+    dP = g2.DevBuf(4 * N)
+    g2.matvec_sk(g2.to_device(np.float32([3.0])), g2.to_device(B), dP, N, 1, 1, f16=f16)
+    got = dP.download(np.float32, N)
+    want = B.view(np.float16).astype(np.float32) if f16 else B
+    assert (got == 3 * want).all()
+
+
 @pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1025, 4097])
 def test_elementwise_tails(g2, n):
     """add and gelu, four elements to a thread: every remainder, one element
