@@ -109,3 +109,28 @@ def test_matmul_launches_stay_below_the_thread_limit():
         assert -(-M // bm) * -(-N // bn) * threads < 2 ** 32, (M, N, K, form)
     assert narrowed > 10
     assert rows(2 ** 30 - 64) == 64 and rows(2 ** 30) == 0
+
+
+FORMS = {0: (16, "direct, 16 rows"), 1: (32, "direct, 32 rows"), 2: (64, "64 x 64"), 3: (128, "128 x 128"),
+         4: (128, "alternating groups")}
+
+
+def test_matmul_tests_reach_every_form_on_ragged_sizes():
+    """Each form of g2_matmul, whole and (64 x 64, alternating) in K splits, is
+    chosen by a tested size that divides neither its rows nor its step of 32
+    and has an odd number of columns, or, for the values' tests, some edge."""
+    from test_matmul_gpu import EDGES, FORM_SIZES
+
+    every = {(f, s) for f in FORMS for s in (False, True)} - {(0, True), (1, True), (3, True)}
+
+    def reached(sizes, ragged):
+        got = set()
+        for M, N, K in sizes:
+            form, ks = matmul_pick(M, N, K)
+            if not ragged or (M % FORMS[form][0] and K % 32 and N % 2):
+                got.add((form, ks > 1))
+        return got
+
+    assert reached(FORM_SIZES, False) == every
+    assert reached(EDGES, True) | {(2, True)} == every  # splits of 64 x 64: an even 300 columns, 5007 = 156 * 32 + 15
+    assert (2, True) in reached([s for s in EDGES if s[0] % 64 and s[2] % 32], False)

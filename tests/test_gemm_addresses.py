@@ -9,8 +9,7 @@ a launch.  It checks that the loads stay inside the matrices, the K slice
 and the LDS ring, that every fragment read finds the chunk its product
 needs, that the outputs of a tile are each written once and the partial
 slices stay inside their buffer, for every GEMM of the fp16 prefill (qkv,
-proj, fc, fc2) at GPT-2 small to XL width and prompt lengths from 65 (the
-first that takes this kernel) to 1023, with the slice count the host picks
+proj, fc, fc2) at GPT-2 small to XL width and prompt lengths from 1 to 1023, with the slice count the host picks
 on MI355X's 256 CUs.  Planted mistakes (the activation row clamp removed, a
 narrower read swizzle, slices that drop the remainder steps) must be
 caught.  No GPU is involved.
@@ -27,7 +26,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "gpt2-opencl-1.1_amd", "csrc")
 
 WIDTHS = (768, 1024, 1280, 1600)
-PROMPTS = (65, 100, 127, 128, 129, 200, 256, 300, 512, 640, 777, 1000, 1023)
+PROMPTS = (1, 8, 37, 64, 65, 100, 127, 128, 129, 200, 256, 300, 512, 640, 777, 1000, 1023)
 
 
 def define(header, name):

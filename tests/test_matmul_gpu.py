@@ -1,10 +1,13 @@
-"""g2_matmul's forms at the sizes where they can go wrong, and the values
-that bf16 parts cannot carry, against the CPU oracle's fp32 product.
+"""g2_matmul's forms at the sizes where they can go wrong, the values that
+bf16 parts cannot carry and the accuracy that the parts are there for, against
+the CPU oracle's fp32 product and against 64 bits.
 
-The sizes put each form (direct 16- and 32-row tiles, 64x64 tiles whole and
-in K splits, 128x128 tiles) on ragged edges: one row or column past a tile,
+The sizes put each form (direct 16- and 32-row tiles, 64x64 tiles whole and in
+K splits, 128x128 tiles of several work-groups per CU, and of alternating wave
+groups whole and in K splits) on ragged edges: one row or column past a tile,
 odd column counts (a column pair that the last column begins), K below one
-step of 32, one past it, and splits that end in a partial step.
+step of 32, one past it, and splits that end in a partial step.  That they do
+is checked against the choice itself in test_dispatch.py.
 """
 import ctypes as C
 import time
@@ -37,14 +40,20 @@ def product(g2, A, B, bias, f16):
     return got[:M * N].reshape(M, N)
 
 
-@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
-@pytest.mark.parametrize("M,N,K", [
-    (1, 1, 1), (1, 1, 40), (17, 1, 65), (3, 2, 31),            # one column: no pairs
-    (16, 31, 32), (17, 33, 33), (15, 65, 257), (33, 97, 300),  # direct
-    (65, 129, 1000), (40, 300, 5007), (130, 257, 2049),        # direct or splits
-    (333, 1601, 96), (470, 2305, 70), (257, 5121, 1281),       # 64 x 64
+EDGES = [
+    (1, 1, 1), (1, 1, 40), (17, 1, 65), (3, 2, 31),            # 64 x 64; one column: no pairs
+    (16, 31, 32), (333, 1601, 96), (470, 2305, 70),            # 64 x 64
+    (40, 300, 5007),                                           # 64 x 64 in 12 splits
+    (17, 33, 33), (15, 65, 257), (33, 97, 300), (65, 129, 1000), (130, 257, 2049),  # direct, 16 rows
+    (50, 3203, 259), (18, 5755, 1389),                         # direct, 32 rows
     (700, 8321, 70), (641, 12801, 32),                         # 128 x 128
-])
+    (118, 20173, 1191), (200, 9001, 300),                      # 128 x 128, alternating groups
+    (257, 5121, 1281),                                         # alternating groups in 2 splits
+]
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("M,N,K", EDGES)
 def test_matmul_edges(g2, M, N, K, f16):
     A, B, bias = operands(M, N, K, f16, M + N + K)
     bound = dot_bound(np.abs(A).astype(np.float64), np.abs(B).astype(np.float64), K)
@@ -52,8 +61,14 @@ def test_matmul_edges(g2, M, N, K, f16):
     assert_close_bound(product(g2, A, B, None, f16), oracle.matmul(A, B, None, M, N, K), bound, what="no bias")
 
 
+# a ragged size per form: direct 16 and 32 rows, 64x64 whole and split, 128x128 of
+# several work-groups per CU, of alternating wave groups whole and split
+FORM_SIZES = [(20, 70, 100), (18, 5755, 1389), (470, 2305, 70), (70, 200, 4100), (700, 8321, 70), (118, 20173, 1191),
+              (257, 5121, 1281)]
+
+
 @pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
-@pytest.mark.parametrize("M,N,K", [(20, 70, 100), (70, 200, 4100), (470, 2305, 70), (700, 8321, 70)])
+@pytest.mark.parametrize("M,N,K", FORM_SIZES)
 def test_matmul_special_values(g2, M, N, K, f16):
     """Rows with an infinity, a NaN, a value that rounds past bf16's largest,
     and rows of magnitudes whose low parts bf16 cannot hold."""
@@ -74,10 +89,55 @@ def test_matmul_special_values(g2, M, N, K, f16):
     assert (np.abs(got[fin].astype(np.float64) - ref[fin]) <= bound[fin] + 1e-45).all()
 
 
-# one size per form: direct 16 and 32 rows, 64x64 whole and split, 128x128 of
-# several work-groups per CU, of alternating wave groups whole and split
-FORM_SIZES = [(20, 70, 100), (18, 5755, 1389), (470, 2305, 70), (70, 200, 4100), (700, 8321, 70), (118, 20173, 1191),
-              (257, 5121, 1281)]
+def sum_bound(K):
+    """What the norm of K random terms' fp32 sum may be off by, of its own: a
+    product's left-out parts are 2^-24 of it at most, and the sum takes about
+    K / 5 roundings (six instructions per 32 k) of at most 2^-24 of a partial
+    sum that grows to its own size, which add up to some sqrt(K / 15) of them.
+    Measured 0.5 to 5 times 2^-24 for K 70 to 4100; without the third parts
+    it is 57 times (test_matmul_bound.py)."""
+    return 2.0 ** -24 * (3 + np.sqrt(K) / 3)
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("M,N,K", FORM_SIZES)
+def test_matmul_accuracy(g2, M, N, K, f16):
+    """Every row's and every column's error, in the norm, against 64 bits."""
+    r = np.random.default_rng(M)
+    A, B = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    if f16:
+        B = B.astype(np.float16).astype(np.float32)
+    ref = A.astype(np.float64) @ B.astype(np.float64)
+    err = product(g2, A, B, None, f16) - ref
+    for axis in (0, 1):
+        assert (np.linalg.norm(err, axis=axis) <= sum_bound(K) * np.linalg.norm(ref, axis=axis)).all()
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("M,N,K", FORM_SIZES)
+def test_matmul_low_parts(g2, M, N, K, f16):
+    """Results that rest on the second and third parts: a row of A or a column
+    of B that picks one row or column of the other is that one, every bit; a
+    row of pairs whose products cancel but for 2^-12; factors whose left-out
+    products are the largest."""
+    r = np.random.default_rng(N)
+    A, B = r.standard_normal((M, K)).astype(np.float32), r.standard_normal((K, N)).astype(np.float32)
+    A[1], B[:, 1] = 0, 0
+    A[1, K - 1], B[K - 3, 1] = 1, 1
+    H = K // 2
+    A[2, H:2 * H] = A[2, :H]
+    B[H:2 * H, 5] = -B[:H, 5] * np.float32(1 + 2.0 ** -12)
+    A[3], B[:, 4] = 1 + 2.0 ** -8 - 2.0 ** -17, 1 + 2.0 ** -8 - 2.0 ** -17
+    if f16:
+        B = B.astype(np.float16).astype(np.float32)
+    got = product(g2, A, B, None, f16)
+    np.testing.assert_array_equal(got[1], B[K - 1])
+    np.testing.assert_array_equal(got[:, 1], A[:, K - 3])
+    exact = A.astype(np.float64) @ B.astype(np.float64)
+    terms = np.linalg.norm(A[2].astype(np.float64) * B[:, 5])
+    assert abs(got[2, 5] - exact[2, 5]) <= 4 * sum_bound(K) * terms  # one output: four deviations
+    # K equal terms: a rounding of up to 2^-24 of the whole for each of K / 5 steps
+    assert abs(got[3, 4] / exact[3, 4] - 1) <= 2.0 ** -24 * (2 + K / 10)
 
 
 def sized(r, shape, e):

@@ -1,14 +1,14 @@
 """GPU parity of the fused prefill with fp16 weights, whose matmuls run on
 the fp16 matrix cores with the fp32 activations split into two fp16 halves
-(g2k_hgemm_*): last-position logits against the CPU oracle (1e-4: the
+(g2k_hgemm2_*, 128x128 tiles): last-position logits against the CPU oracle (1e-4: the
 oracle runs in fp32 on the same fp16-rounded weights) and against the
 fp32-MFMA GEMM of the same library (G2_PREFILL_F32MFMA=1), which the split
 must match to fp32-level accumulation differences, at GPT-2 XL width and
-for ragged prompt lengths (not multiples of the 64-row tile) up to the
-1023-position limit.  The lengths cover the 64x64 GEMM (P <= 64), the
-128x128 GEMM with qkv and fc as K slices (100: 6 and 5 slices; 200, 256:
-3 and 2) and run whole (1023 rows), with proj and fc2 as 2 to 8 slices
-summed with the following LayerNorm.
+for ragged prompt lengths (not multiples of a tile's rows) up to the
+1023-position limit.  The lengths cover qkv and fc as K slices (100 rows and
+fewer: 6 and 5 slices; 200, 256: 3 and 2) and run whole (1023 rows), with proj
+and fc2 as 2 to 8 slices summed with the following LayerNorm.  The 64x64 GEMM
+(g2k_hgemm_*), which only G2_PREFILL_GEMM64=1 takes, is compared with it.
 """
 import numpy as np
 import pytest
@@ -48,15 +48,15 @@ def test_prefill_split_fp16_mfma(g2, monkeypatch, P):
         f"P {P}: gpu argmax {int(np.argmax(lg_h))}, oracle {int(np.argmax(ref))}, oracle top-2 gap {top2[1] - top2[0]:.3e}"
 
 
-@pytest.mark.parametrize("P", [65, 200, 512, 1023])
+@pytest.mark.parametrize("P", [1, 37, 64, 65, 200, 512, 1023])
 def test_prefill_gemm_tiles_agree(g2, monkeypatch, P):
-    """Prompts of more than 64 rows run the 128x128-tile GEMM (operands
-    staged through LDS by asynchronous loads, activations split into their
-    fp16 halves by the kernels that produce them); it sums every output in
-    the order of the 64x64-tile GEMM (G2_PREFILL_GEMM64=1), which splits
-    the stored fp32 activations itself.  The logits agree to fp32 rounding
-    (1e-5; 2.4e-6 to 3.2e-6 measured at P 65 to 1023: the two forms split K
-    into different slices and sum them in different kernels)."""
+    """Prompts run the 128x128-tile GEMM (operands staged through LDS by
+    asynchronous loads, activations split into their fp16 halves by the
+    kernels that produce them); it sums every output in the order of the
+    64x64-tile GEMM (G2_PREFILL_GEMM64=1), which splits the stored fp32
+    activations itself.  The logits agree to fp32 rounding (1e-5; 2.4e-6 to
+    3.2e-6 measured at P 65 to 1023: the two forms split K into different
+    slices and sum them in different kernels)."""
     cfg = g2.make_config(2, 1600, 25, vocab_size=50257)
     w = g2.synth_weights(cfg, SEED, f16_round=True)
     prompt = random_prompt(P, cfg.vocab_size, 200 + P)
