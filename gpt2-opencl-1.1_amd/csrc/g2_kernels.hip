@@ -638,8 +638,8 @@ G2K void g2k_attn_rows(const g2_attnrows_args a)
  * reference matmul is in g2_matmul.hip)
  *
  * Tile 64x64x16, 256 threads = 2x2 waves of 32x32, each wave a 2x2 grid of
- * v_mfma_f32_16x16x4f32.  A [M,K] fp32 row-major; B [K,N] (BKN) or [N,K]
- * (BNK), fp32 or fp16 (widened when staged to LDS).  LDS tiles hold
+ * v_mfma_f32_16x16x4f32.  A [M,K] fp32 row-major; B [N,K] fp32 or fp16
+ * (widened when staged to LDS).  LDS tiles hold
  * As[m][k] and Bs[n][k] so both fragments read 4 consecutive k per lane
  * group.  Epilogues as in g2_gemm_args.
  * MFMA 16x16x4 f32 operand layout: lane l supplies A[l%16][l/16] and
@@ -686,7 +686,7 @@ __device__ __forceinline__ void epi_add(f32x4 (&acc)[2][2], const g2_gemm_args &
     }
 }
 
-template <typename BT, bool BNK, int EPI>
+template <typename BT, int EPI>
 __device__ void gemm_impl(const g2_gemm_args &a)
 {
     constexpr int BM = 64, BN = 64, BK = 16, LDK = BK + 1;
@@ -719,7 +719,7 @@ __device__ void gemm_impl(const g2_gemm_args &a)
             for (int e = 0; e < 4; ++e) As[r * LDK + kq + e] = v[e];
         }
         /* B tile into Bs[n][k] */
-        if (BNK) {
+        {
             const int r = tid >> 2, kq = (tid & 3) * 4;
             const int gn = n0 + r, gk = k0 + kq;
             float v[4] = {0.f, 0.f, 0.f, 0.f};
@@ -731,18 +731,6 @@ __device__ void gemm_impl(const g2_gemm_args &a)
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) Bs[r * LDK + kq + e] = v[e];
-        } else {
-            const int kr = tid >> 4, nq = (tid & 15) * 4;
-            const int gk = k0 + kr, gn = n0 + nq;
-            float v[4] = {0.f, 0.f, 0.f, 0.f};
-            if (gk < K) {
-                const size_t base = (size_t)gk * N + gn;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (gn + e < N) v[e] = ldw(B, base + e);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) Bs[(nq + e) * LDK + kr] = v[e];
         }
         __syncthreads();
 #pragma unroll
@@ -795,17 +783,17 @@ __device__ void gemm_impl(const g2_gemm_args &a)
             }
 }
 
-#define G2_GEMM(name, BT, BNK, EPI) \
-    G2K void name(const g2_gemm_args a) { gemm_impl<BT, BNK, EPI>(a); }
+#define G2_GEMM(name, BT, EPI) \
+    G2K void name(const g2_gemm_args a) { gemm_impl<BT, EPI>(a); }
 
-G2_GEMM(g2k_gemm_nk_f32_store, float, true, GEPI_STORE)
-G2_GEMM(g2k_gemm_nk_f16_store, _Float16, true, GEPI_STORE)
-G2_GEMM(g2k_gemm_nk_f32_gelu, float, true, GEPI_GELU)
-G2_GEMM(g2k_gemm_nk_f16_gelu, _Float16, true, GEPI_GELU)
-G2_GEMM(g2k_gemm_nk_f32_resid, float, true, GEPI_RESID)
-G2_GEMM(g2k_gemm_nk_f16_resid, _Float16, true, GEPI_RESID)
-G2_GEMM(g2k_gemm_nk_f32_qkv, float, true, GEPI_QKV)
-G2_GEMM(g2k_gemm_nk_f16_qkv, _Float16, true, GEPI_QKV)
+G2_GEMM(g2k_gemm_nk_f32_store, float, GEPI_STORE)
+G2_GEMM(g2k_gemm_nk_f16_store, _Float16, GEPI_STORE)
+G2_GEMM(g2k_gemm_nk_f32_gelu, float, GEPI_GELU)
+G2_GEMM(g2k_gemm_nk_f16_gelu, _Float16, GEPI_GELU)
+G2_GEMM(g2k_gemm_nk_f32_resid, float, GEPI_RESID)
+G2_GEMM(g2k_gemm_nk_f16_resid, _Float16, GEPI_RESID)
+G2_GEMM(g2k_gemm_nk_f32_qkv, float, GEPI_QKV)
+G2_GEMM(g2k_gemm_nk_f16_qkv, _Float16, GEPI_QKV)
 
 /* ======================================================================
  * fp32-weight GEMM of the fused prefill, C = A . W^T with W [N,K] packed

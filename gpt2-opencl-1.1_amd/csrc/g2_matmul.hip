@@ -6,8 +6,8 @@
  * p1), p3 = bf16(v - p1 - p2), 8 significant bits each, both differences
  * exact; an fp16 value is the sum of two.  A product of two fp32 values is
  * then six bf16 products, p1q1 + p1q2 + p2q1 + p2q2 + p1q3 + p3q1 (five with
- * an fp16 factor, whose q3 is zero); the ones left out are below 2^-25 of
- * it.  The products are exact in fp32 and summed in fp32 by
+ * an fp16 factor, whose q3 is zero); the ones left out, p2q3 and p3q2 first,
+ * are about 2^-24 of it at most.  The products are exact in fp32 and summed in fp32 by
  * v_mfma_f32_16x16x32_bf16, which takes 32 k per instruction at 16 times the
  * rate of the fp32 instruction (4 k): a sixth of 32 k against 4 k leaves
  * 2.7 times the fp32 peak and fewer roundings of the running sum.
@@ -182,13 +182,13 @@ __device__ __forceinline__ int tile_of(int w, int T)
  * 1.85 us, its conversions, LDS traffic and products one after the other
  * (xduo_impl is for that).  Taken back: two steps in flight, two LDS buffers,
  * all fragments read ahead, raised wave priority (each within 5%). */
-template <typename BT, bool BNK, int EPI, int BM, int BN>
+template <typename BT, int EPI, int BM, int BN>
 __device__ void xgemm_impl(const g2_gemm_args &a)
 {
     using namespace xg;
     constexpr int PB = sizeof(BT) == 4 ? 3 : 2;
-    constexpr int SA = BM * 16 + 64, SB = BN * 16 + (BNK ? 64 : 0); /* octet plane strides, bytes */
-    constexpr int RA = BM / 64, RB = BN / 64;                       /* octets (BNK, A) or columns a thread stages */
+    constexpr int SA = BM * 16 + 64, SB = BN * 16; /* octet plane strides, bytes */
+    constexpr int RA = BM / 64, RB = BN / 64;                       /* octets (A) or columns (B) a thread stages */
     constexpr int IB = BM / 32, JB = BN / 32;                       /* 16-blocks of a wave */
     constexpr int ST = 3 * 4 * SA + PB * 4 * SB;                    /* bytes of a step's tiles */
     __shared__ __attribute__((aligned(16))) unsigned char lds[ST];
@@ -205,18 +205,15 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     const int sf = min(s1, K >> 5); /* steps s0 .. sf - 1 are whole */
     const BT *B = (const BT *)a.B;
 
-    const int ar = tid >> 2, ao = (tid & 3) * 4; /* row-major staging: row (+ 64 i), k offset */
+    const int ar = tid >> 2, ao = (tid & 3) * 4; /* A: row (+ 64 i), k offset */
     const float *ap[RA];
 #pragma unroll
     for (int i = 0; i < RA; ++i) ap[i] = a.A + (size_t)min(m0 + ar + 64 * i, M - 1) * K + ao;
-    /* [K,N] staging: column (pair), octet; the pair that the last column
+    /* B: column (pair), octet; the pair that the last column
      * begins is loaded one column early */
     const int bc = tid & 63, bo = wave;
-    const bool late = !BNK && n0 + bc * RB + RB - 1 == N;
-    const BT *bp[RB];
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-        bp[i] = BNK ? B + (size_t)min(n0 + ar + 64 * i, N - 1) * K + ao : B + min(n0 + bc * RB, N - RB);
+    const bool late = n0 + bc * RB + RB - 1 == N;
+    const BT *bp = B + min(n0 + bc * RB, N - RB);
 
     float av[RA][8], bv[RB][8];
     /* whole step t (past the last one: that one again, unused) */
@@ -226,26 +223,19 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
         for (int i = 0; i < RA; ++i)
 #pragma unroll
             for (int h = 0; h < 2; ++h) *(f32x4 *)(av[i] + 4 * h) = *(const f32x4u *)(ap[i] + k + 16 * h);
-        if constexpr (BNK) {
 #pragma unroll
-            for (int i = 0; i < RB; ++i)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) *(f32x4 *)(bv[i] + 4 * h) = *(const f32x4u *)((const float *)bp[i] + k + 16 * h);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const size_t o = (size_t)(k + 4 * bo + koff(e)) * N;
-                if constexpr (RB == 1) {
-                    bv[0][e] = ldw(bp[0], o);
-                } else if constexpr (sizeof(BT) == 4) {
-                    const f32x2 w = *(const f32x2u *)((const float *)bp[0] + o);
-                    bv[0][e] = w.x;
-                    bv[RB - 1][e] = w.y;
-                } else {
-                    const f16x2u w = *(const f16x2u *)((const _Float16 *)bp[0] + o);
-                    bv[0][e] = (float)w.x;
-                    bv[RB - 1][e] = (float)w.y;
-                }
+        for (int e = 0; e < 8; ++e) {
+            const size_t o = (size_t)(k + 4 * bo + koff(e)) * N;
+            if constexpr (RB == 1) {
+                bv[0][e] = ldw(bp, o);
+            } else if constexpr (sizeof(BT) == 4) {
+                const f32x2 w = *(const f32x2u *)((const float *)bp + o);
+                bv[0][e] = w.x;
+                bv[RB - 1][e] = w.y;
+            } else {
+                const f16x2u w = *(const f16x2u *)((const _Float16 *)bp + o);
+                bv[0][e] = (float)w.x;
+                bv[RB - 1][e] = (float)w.y;
             }
         }
     };
@@ -257,7 +247,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
             for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
         }
-        if constexpr (!BNK && RB == 2) {
+        if constexpr (RB == 2) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) bv[0][e] = late ? bv[1][e] : bv[0][e];
         }
@@ -267,7 +257,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
             parts8<PB>(bv[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < PB; ++q)
-                *(u32x4 *)(lds + 12 * SA + (4 * q + (BNK ? (tid & 3) : bo)) * SB + ((BNK ? ar : bc) + 64 * i) * 16) = p[q];
+                *(u32x4 *)(lds + 12 * SA + (4 * q + bo) * SB + (bc + 64 * i) * 16) = p[q];
         }
     };
 
@@ -276,9 +266,9 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     for (int i = 0; i < IB; ++i)
 #pragma unroll
         for (int j = 0; j < JB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    /* column block j of the wave: positions 16 j of its half (BNK, BN 64), or
+    /* column block j of the wave: positions 16 j of its half (BN 64), or
      * (JB 4) blocks 0, 1 of the even columns and 2, 3 of the odd ones */
-    constexpr bool PAIR = !BNK && RB == 2;
+    constexpr bool PAIR = RB == 2;
     const int arow = (lane >> 4) * SA + (wm * (BM / 2) + (lane & 15)) * 16;
     const int brow = 12 * SA + (lane >> 4) * SB + (wn * (PAIR ? BN / 4 : BN / 2) + (lane & 15)) * 16;
     auto bblk = [](int j) { return PAIR ? (j & (JB / 2 - 1)) * 256 + (j / (JB / 2)) * (BN / 2) * 16 : j * 256; };
@@ -317,8 +307,8 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
         for (int i = 0; i < RB; ++i)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int kk = k + koff(e) + (BNK ? ao : 4 * bo);
-                bv[i][e] = kk < K ? (BNK ? ldw(bp[i], k + koff(e)) : ldw(bp[0], (size_t)kk * N + i)) : 0.f;
+                const int kk = k + koff(e) + 4 * bo;
+                bv[i][e] = kk < K ? ldw(bp, (size_t)kk * N + i) : 0.f;
             }
         __syncthreads();
         store();
@@ -345,7 +335,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
         for (int i = 0; i < IB; ++i)
 #pragma unroll
             for (int j = 0; j < JB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        again_tile<BT, BNK>(a.A, B, M, N, K, m0 + wm * (BM / 2), n, s0 * 32, min(s1 * 32, K), acc);
+        again_tile<BT, false>(a.A, B, M, N, K, m0 + wm * (BM / 2), n, s0 * 32, min(s1 * 32, K), acc);
         __syncthreads(); /* before any wave writes: C may lie in A or B */
     }
 
@@ -382,14 +372,14 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
         }
 }
 
-#define G2_XGEMM(name, BT, BNK, EPI, BM, BN, OCC) \
-    extern "C" __global__ __launch_bounds__(256, OCC) void name(const g2_gemm_args a) { xgemm_impl<BT, BNK, EPI, BM, BN>(a); }
-G2_XGEMM(g2k_xgemm128_f32, float, false, GEPI_STORE, 128, 128, 2)
-G2_XGEMM(g2k_xgemm128_f16, _Float16, false, GEPI_STORE, 128, 128, 2)
-G2_XGEMM(g2k_xgemm64_f32, float, false, GEPI_STORE, 64, 64, 3)
-G2_XGEMM(g2k_xgemm64_f16, _Float16, false, GEPI_STORE, 64, 64, 3)
-G2_XGEMM(g2k_xgemm64_part_f32, float, false, GEPI_PARTIAL, 64, 64, 3)
-G2_XGEMM(g2k_xgemm64_part_f16, _Float16, false, GEPI_PARTIAL, 64, 64, 3)
+#define G2_XGEMM(name, BT, EPI, BM, BN, OCC) \
+    extern "C" __global__ __launch_bounds__(256, OCC) void name(const g2_gemm_args a) { xgemm_impl<BT, EPI, BM, BN>(a); }
+G2_XGEMM(g2k_xgemm128_f32, float, GEPI_STORE, 128, 128, 2)
+G2_XGEMM(g2k_xgemm128_f16, _Float16, GEPI_STORE, 128, 128, 2)
+G2_XGEMM(g2k_xgemm64_f32, float, GEPI_STORE, 64, 64, 3)
+G2_XGEMM(g2k_xgemm64_f16, _Float16, GEPI_STORE, 64, 64, 3)
+G2_XGEMM(g2k_xgemm64_part_f32, float, GEPI_PARTIAL, 64, 64, 3)
+G2_XGEMM(g2k_xgemm64_part_f16, _Float16, GEPI_PARTIAL, 64, 64, 3)
 
 /* C = (part[0] + ... + part[ks-1]) + bias, the splits in order; four
  * elements of the M x N matrix per thread, ks <= G2_XG_MAXKS. */

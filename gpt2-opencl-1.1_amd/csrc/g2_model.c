@@ -1123,8 +1123,7 @@ static int fused_prefill(g2_model *m, int P)
      * whose results agree to fp32 rounding */
     const char *p64 = getenv("G2_PREFILL_GEMM64");
     const int big = h && !(p64 && p64[0] == '1');
-    /* fp32 weights: the 64x64 fp32-MFMA GEMM with K steps of 32 streamed
-     * through LDS, split-K for short prompts */
+    /* fp32 weights: prefill_sgemm's forms (sg_pick) */
     const int sg = !f16 && E % 32 == 0 && F % 32 == 0;
     const int f_qkv = big ? G2F_HGEMM2_QKV : h ? G2F_HGEMM_QKV : (f16 ? G2F_GEMM_NK_F16_QKV : G2F_GEMM_NK_F32_QKV);
     const int f_resid = h ? G2F_HGEMM_RESID : (f16 ? G2F_GEMM_NK_F16_RESID : G2F_GEMM_NK_F32_RESID);
