@@ -41,6 +41,7 @@ extern "C" {
     X(EMBED_F32, "g2k_embed_f32") X(EMBED_F16, "g2k_embed_f16")               \
     X(SPLIT_KV, "g2k_split_kv") X(ATTN_SCORES, "g2k_attn_scores")             \
     X(ATTN_SOFTMAX, "g2k_attn_softmax") X(ATTN_OUT, "g2k_attn_out")           \
+    X(ATTN_OUT4, "g2k_attn_out4")                                             \
     X(ATTN_PART, "g2k_attn_part") X(ATTN_PART_S, "g2k_attn_part_s")           \
     X(ATTN_MERGE, "g2k_attn_merge") X(ARGMAX_MERGE, "g2k_argmax_merge")       \
     X(ATTN_SHORT, "g2k_attn_short") X(ATTN_SHORT_S, "g2k_attn_short_s")       \

@@ -190,7 +190,7 @@ typedef struct {
     const float *scores;
     const float *v_cache;
     float *out;
-    int T, D, DH, out_base, groups;
+    int T, D, DH, out_base;
 } g2_attnout_args;
 
 /* A prompt's causal attention by rows (g2k_attn_rows): out[P][D] from the

@@ -520,14 +520,17 @@ G2K void g2k_attn_softmax(const g2_softmax_args a)
 /* ---- attn_out_1q (math.cl:459-476): block 1024: 16 dims x 64 positions at a
  * time (j = row, row + 64, ...), four ahead; the 64 sums of a dim are added
  * over a wave's four rows, then over the 16 waves in order.  Grid
- * ceil(D / (16 groups)), groups <= 4 of 16 dims one after the other, written
- * when all are done. */
-extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout_args a)
+ * ceil(D / (16 GROUPS)); four groups of 16 dims go one after the other and are
+ * written when all are done (one kernel for both cost the common case 0.4 of
+ * its 3.4 us). */
+template <int GROUPS>
+__device__ void attn_out_impl(const g2_attnout_args &a)
 {
-    __shared__ float red[16][16], res[64];
-    const int tid = threadIdx.x, d0 = blockIdx.x * 16 * a.groups;
-    for (int g = 0; g < a.groups; ++g) {
-        const int dc = min(d0 + 16 * g + (tid & 15), a.D - 1);
+    __shared__ float red[GROUPS][16][16];
+    const int tid = threadIdx.x, d0 = blockIdx.x * 16 * GROUPS + (tid & 15);
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+        const int dc = min(d0 + 16 * g, a.D - 1);
         const float *srow = a.scores + (size_t)(dc / a.DH) * G2_KV_MAX_SEQ;
         float o = 0.f;
         for (int j0 = tid >> 4; j0 < a.T; j0 += 256) {
@@ -543,18 +546,19 @@ extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout
         }
         o += __shfl_xor(o, 16);
         o += __shfl_xor(o, 32);
-        if ((tid & 63) < 16) red[tid >> 6][tid & 15] = o;
-        __syncthreads();
-        if (tid < 16) {
-            float s = 0.f;
-#pragma unroll
-            for (int w = 0; w < 16; ++w) s += red[w][tid];
-            res[16 * g + tid] = s;
-        }
-        __syncthreads();
+        if ((tid & 63) < 16) red[g][tid >> 6][tid & 15] = o;
     }
-    if (tid < 16 * a.groups && d0 + tid < a.D) a.out[a.out_base + d0 + tid] = res[tid];
+    __syncthreads();
+    const int g = GROUPS == 1 ? 0 : tid >> 4, d = d0 + 16 * g;
+    if (tid < 16 * GROUPS && d < a.D) {
+        float s = 0.f;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) s += red[g][w][tid & 15];
+        a.out[a.out_base + d] = s;
+    }
 }
+extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out(const g2_attnout_args a) { attn_out_impl<1>(a); }
+extern "C" __global__ __launch_bounds__(1024) void g2k_attn_out4(const g2_attnout_args a) { attn_out_impl<4>(a); }
 
 /* ---- a prompt's attention on the reference path: the three operators above
  * for every row i of qkv [P][3D] over positions 0..i, scores kept in LDS; grid

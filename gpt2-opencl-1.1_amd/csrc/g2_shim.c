@@ -668,9 +668,9 @@ int g2_attn_out_1q(const float *scores, const float *v_cache, float *out, int T_
     if (!scores || !v_cache || !out) return g2i_err(G2_E_ARG, "g2_attn_out_1q: NULL buffer");
     if (T_kv <= 0 || T_kv > G2_MAX_SEQ || D <= 0 || DH <= 0 || out_base < 0)
         return g2i_err(G2_E_ARG, "g2_attn_out_1q: bad sizes");
-    g2_attnout_args a = { scores, v_cache, out, T_kv, D, DH, out_base,
-                          g2i_attn_out_groups(scores, v_cache, out + out_base, T_kv, D, DH) };
-    return g2i_launch(G2F_ATTN_OUT, cdiv(D, 16 * a.groups), 1, 1024, &a);
+    const int groups = g2i_attn_out_groups(scores, v_cache, out + out_base, T_kv, D, DH);
+    g2_attnout_args a = { scores, v_cache, out, T_kv, D, DH, out_base };
+    return g2i_launch(groups == 1 ? G2F_ATTN_OUT : G2F_ATTN_OUT4, cdiv(D, 16 * groups), 1, 1024, &a);
 }
 
 int g2_attn_1q(const float *qkv, const float *k_cache, const float *v_cache, float *out,
