@@ -37,17 +37,21 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef _Float16 f16x2u __attribute__((ext_vector_type(2), aligned(2)));
 
-/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts; `lossy`
- * is set where three may not be all of a value.  Two are, of any fp16 value. */
+/* Eight consecutive k as the fragments (8 bf16 per lane) of P parts, and of
+ * three what is left for the third: look() sets `lossy` where that may not be
+ * all of it.  Two are, of any fp16 value. */
 template <int P>
-__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], bool &lossy)
+__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], float (&rest)[8])
 {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         f32x2 r = {v[2 * e], v[2 * e + 1]};
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-            if (P == 3 && p == 2) lossy |= __builtin_amdgcn_classf(r.x, 0x90) | __builtin_amdgcn_classf(r.y, 0x90);
+            if (P == 3 && p == 2) {
+                rest[2 * e] = r.x;
+                rest[2 * e + 1] = r.y;
+            }
             const unsigned w = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2));
             o[p][e] = w;
             if (p + 1 < P) {
@@ -56,6 +60,20 @@ __device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], bool 
             }
         }
     }
+}
+
+__device__ __forceinline__ void look(bool &lossy, const float (&rest)[8])
+{
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) lossy |= __builtin_amdgcn_classf(rest[e], 0x90) | __builtin_amdgcn_classf(rest[e + 1], 0x90);
+}
+
+template <int P>
+__device__ __forceinline__ void parts8(const float (&v)[8], u32x4 (&o)[P], bool &lossy)
+{
+    float rest[8];
+    parts8<P>(v, o, rest);
+    if constexpr (P == 3) look(lossy, rest);
 }
 
 __device__ __forceinline__ f32x4 mma(const u32x4 &a, const u32x4 &b, const f32x4 &c)
@@ -194,6 +212,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     __shared__ __attribute__((aligned(16))) unsigned char lds[ST];
     __shared__ unsigned words[4];
     bool lossy = false;
+    constexpr bool LATE = PB == 3; /* operands tested beside the products (fp16 B: 10% slower, a wave per SIMD lost) */
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int M = a.M, N = a.N, K = a.K;
@@ -215,7 +234,7 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
     const bool late = n0 + bc * RB + RB - 1 == N;
     const BT *bp = B + min(n0 + bc * RB, N - RB);
 
-    float av[RA][8], bv[RB][8];
+    float av[RA][8], bv[RB][8], ra[RA][8], rb[RB][8];
     /* whole step t (past the last one: that one again, unused) */
     auto load = [&](int t) {
         const int k = min(t, sf - 1) * 32;
@@ -243,7 +262,8 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RA; ++i) {
             u32x4 p[3];
-            parts8<3>(av[i], p, lossy);
+            if constexpr (LATE) parts8<3>(av[i], p, ra[i]);
+            else parts8<3>(av[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < 3; ++q) *(u32x4 *)(lds + (4 * q + (tid & 3)) * SA + (ar + 64 * i) * 16) = p[q];
         }
@@ -254,7 +274,8 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             u32x4 p[PB];
-            parts8<PB>(bv[i], p, lossy);
+            if constexpr (LATE) parts8<PB>(bv[i], p, rb[i]);
+            else parts8<PB>(bv[i], p, lossy);
 #pragma unroll
             for (int q = 0; q < PB; ++q)
                 *(u32x4 *)(lds + 12 * SA + (4 * q + bo) * SB + (bc + 64 * i) * 16) = p[q];
@@ -284,6 +305,12 @@ __device__ void xgemm_impl(const g2_gemm_args &a)
 #pragma unroll
             for (int q = 0; q < 3; ++q) f[q] = *(const u32x4 *)(lds + arow + 4 * q * SA + i * 256);
             mma_parts<PB, JB>(acc[i], f, b);
+            if (LATE && i == 0) {
+#pragma unroll
+                for (int x = 0; x < RA; ++x) look(lossy, ra[x]);
+#pragma unroll
+                for (int x = 0; x < RB; ++x) look(lossy, rb[x]);
+            }
         }
     };
 
