@@ -184,19 +184,21 @@ __device__ __forceinline__ int tile_of(int w, int T)
  * the steps of a split (gridDim.y splits of whole steps, GEPI_PARTIAL) in
  * order.  A step's tiles are loaded to registers one step ahead, split into
  * their parts and stored to LDS as [part][k octet][row] 16-byte fragments, so
- * a fragment read takes 16 consecutive rows of an octet (no bank conflicts);
- * the octet planes of row-major operands are padded by 64 bytes so that the
- * four octets of four rows that 16 lanes store fall on distinct banks.  B
+ * a fragment read takes 16 consecutive rows of an octet.  The octet planes of
+ * A are padded by 64 bytes so that the four octets of four rows that 16 lanes
+ * store fall on distinct banks; SQ_LDS_BANK_CONFLICT is a third of
+ * SQ_LDS_IDX_ACTIVE all the same, 16 cycles to each of A's stores.  B
  * [K,N]: a lane loads a column pair (BN 128) or a column (BN 64) of eight k
  * rows, so the transposition is a choice of registers; column n of a 128-wide
  * tile sits at position n / 2 + 64 (n odd), which makes a lane's two column
  * blocks neighbours in memory.  N >= 2 for BN 128; nothing else is asked of
  * M, N, K or alignment.
  *
- * Measured on MI355X (N(0,1) by N(0,0.02)): 1024 x 50257 x 1600 in 0.80 ms
- * with fp32 B (1.24 PFLOP/s of bf16 products, above the 1.14 that a library
- * bf16 product of 8192^3 reaches; the fp32-instruction kernel before: 3.35
- * ms), 0.66 ms with fp16 B (3.05).  With one work-group per CU a step takes
+ * Measured on MI355X (N(0,1) by N(0,0.02)): 1024 x 50257 x 1600 in 0.84 to
+ * 0.89 ms with fp32 B (1.11 to 1.17 PFLOP/s of bf16 products; a library bf16
+ * product of 8192^3 reaches 1.14; the fp32-instruction kernel before: 3.35
+ * ms), 0.67 to 0.69 ms with fp16 B (3.05); the matrix cores are busy 56 and
+ * 65% of the CUs' busy cycles.  With one work-group per CU a step takes
  * 1.85 us, its conversions, LDS traffic and products one after the other
  * (xduo_impl is for that).  Taken back: two steps in flight, two LDS buffers,
  * all fragments read ahead, raised wave priority (each within 5%). */
@@ -447,9 +449,10 @@ G2K void g2k_xgemm_sum(const g2_gemm_args a)
  * added at the end.  Staging as in xgemm_impl.  Epilogues as g2_gemm_args
  * describes them; GEPI_PARTIAL: gridDim.y splits of whole steps.  A step
  * takes 1.02 us (0.75 at BM 64; 1.85 in xgemm_impl at one work-group per CU),
- * of which the products alone 0.79 and the reads in front of them 0.2; W
- * [N,K] of n_embd 1280 by 256 rows: fc 24 us in three splits (the fp32
- * instruction, whole: 47), fc2 25 in twelve (34), qkv 20 in four (30). */
+ * of which the products alone 0.79 and the reads in front of them 0.2; the
+ * matrix cores are busy 42% of the CUs' busy cycles (56% whole with fp16 B).
+ * W [N,K] of n_embd 1280 by 256 rows: fc 27 us in three splits (the fp32
+ * instruction, whole: 47), fc2 27 in twelve (34), qkv 22 in four (30). */
 template <typename BT, bool BNK, int EPI, int BM>
 __device__ void xduo_impl(const g2_gemm_args &a)
 {

@@ -1017,7 +1017,8 @@ static int prefill_resid(g2_model *m, const float *A, const uint16_t *Ah, const 
  * the fastest or equal; us of the GEMM alone as sgemm / 64 x 128 / 128 x 128
  * with their splits, n_embd 1280: fc 100 rows 28.8 / 17.2 / 17.3, 256 rows
  * 47.5 / 32.4 / 24.0, 512 rows 72.3 / 55.3 / 46.7; fc2 26.3 / 18.0 / 22.6,
- * 33.5 / 28.1 / 24.8, 60.4 / 47.8 / 38.9; proj 256 rows 12.0 / 11.2 / 12.6. */
+ * 33.5 / 28.1 / 24.8, 60.4 / 47.8 / 38.9; proj 256 rows 12.0 / 11.2 / 12.6
+ * (the bf16 forms without their test of the operands, 1 to 3% of them). */
 enum { SG_FORM_F32, SG_FORM_DUO64, SG_FORM_DUO128 };
 
 static int sg_pick(int M, int N, int K, int *splits)
@@ -1118,8 +1119,8 @@ static int fused_prefill(g2_model *m, int P)
     const int h = f16 && E % 64 == 0 && F % 64 == 0 && !(pe && pe[0] == '1');
     /* the 128x128 tiles for every prompt: short ones leave most of a tile's
      * rows unused, but their K splits stream the weights from all CUs, which
-     * is what bounds them (8 tokens: 774M 2.2 ms against 4.0 on the 64x64
-     * tiles, 1.5B 3.3 against 6.3).  G2_PREFILL_GEMM64=1 keeps the 64x64 ones,
+     * is what bounds them (8 tokens: 774M 2.0 ms against 4.0 on the 64x64
+     * tiles, 1.5B 3.1 against 6.3).  G2_PREFILL_GEMM64=1 keeps the 64x64 ones,
      * whose results agree to fp32 rounding */
     const char *p64 = getenv("G2_PREFILL_GEMM64");
     const int big = h && !(p64 && p64[0] == '1');

@@ -355,13 +355,16 @@ static int capturing(void)
  * forms without K splits.  A form's step costs its latency while
  * the CUs hold at most one work-group each, and its throughput times the
  * work-groups per CU beyond; up to nearly two, some CUs hold two and decide.
- * The constants are fitted to MI355X times of 45 shapes (8..1024 rows, 258 to
- * 50257 columns, K 267..6400, both weight types): the pick is the fastest
- * form or within 10% of it on 41.  Examples, us of direct 16 / direct 32 / 64
- * x 64 / its best split / 128 x 128: 96 x 768 x 3072: 14 / 20 / 69 / 16 / -;
- * 512 x 1024 x 1024: 19 / 15 / 25 / 19 / 60; 256 x 1280 x 5120: 61 / 58 / 113
- * / 34 / 276; 333 x 6400 x 1600: 117 / 97 / 74 / - / 94; 1024 x 50257 x 1600:
- * - / - / 1200 / - / 880. */
+ * The constants are fitted to MI355X times; on 45 shapes (8..1024 rows, 258 to
+ * 50257 columns, K 267..5907) with both weight types the pick is the fastest
+ * form or within 10% of it on 87 of 90 (37 x 10569 x 1205: 10.2%, 22 x 9814 x
+ * 5293: 25 and 17%); profiles/matmul_forms.md has every form's time at each.  Examples, us with fp32
+ * B of direct 16 / direct 32 / 64 x 64 / its best split / 128 x 128 /
+ * alternating groups / their best split: 96 x 768 x 3072: 16 / 21 / 77 / 16 /
+ * 168 / 109 / 20; 512 x 1024 x 1024: 21 / 17 / 29 / 20 / 60 / 41 / 22; 256 x
+ * 1280 x 5120: 63 / 61 / 126 / 35 / 277 / 178 / 31; 333 x 6400 x 1600: 114 /
+ * 94 / 79 / - / 97 / 66 / -; 1024 x 50257 x 1600: - / - / 1140 / - / 883 / 896
+ * / -. */
 static double xg_load(double per_cu) { return per_cu <= 1 ? per_cu : per_cu < 1.7 ? 1.7 : per_cu; }
 
 int g2i_matmul_in_place(const float *A, const void *B, size_t b_size, const float *C, long M, long N, long K)
@@ -403,7 +406,7 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
         for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
             if (ks > 1 && (whole || ks * mn > (double)G2_GEMM_PART_FLOATS || 2 * ks > steps || tiles * ks > cus)) break;
             /* a step with all CUs at it for several rounds: 1.4 us (1024 x
-             * 50257 x 1600: 907 us against 871 on xgemm128, 753 against 686
+             * 50257 x 1600: 896 us against 883 on xgemm128, 751 against 686
              * with fp16 B) */
             double duo = 4 + steps / ks * (tiles * ks > cus ? 1.4 : 1.05) * ceil(tiles * ks / cus);
             if (ks > 1) duo += 5 + ks * mn * sizeof(float) * (1 / 2.6e6 + 1 / 6e6);

@@ -61,9 +61,9 @@ int g2_device_name(char *buf, int len, int *compute_units);
  * reference, whose queue is main.c:537): every launch of the library goes to
  * it, so a caller may capture the library's calls into its own HIP graph
  * (hipStreamBeginCapture on this stream, the calls, hipStreamEndCapture).
- * A recorded g2_matvec and g2_attn_1q may go on using a buffer of the library:
- * replay graphs that hold them one after another and on this stream, or not
- * beside other calls.  A recorded g2_matmul uses its operands only.
+ * A recorded g2_matvec, g2_matvec_sk or g2_attn_1q may go on using a buffer
+ * of the library: replay graphs that hold them one after another and on this
+ * stream, or not beside other calls.  A recorded g2_matmul uses its operands only.
  * NULL before g2_init. */
 void *g2_stream(void);
 
@@ -81,7 +81,10 @@ int g2_sync(void);                                             /* clFinish      
 /* ---- operators (main.c launch_* helpers; kernels math.cl) ----------------- */
 
 /* launch_matmul, main.c:1518-1535 (kernel main.c:603-684):
- * C[M,N] = A[M,K] B[K,N] (+bias[N]); all row-major fp32. */
+ * C[M,N] = A[M,K] B[K,N] (+bias[N]); all row-major fp32.  fp32 accuracy for
+ * any operands; values below 2^-103 (not zero) in magnitude and sums that are
+ * not finite make a call up to four times as long.  C may lie in A or B where
+ * N <= 64 and its rows are A's own, or where M <= 64 and N <= 64. */
 int g2_matmul(const float *A, const float *B, const float *bias, float *C,
               int M, int N, int K);
 /* Same with B stored as IEEE half (fp16 weights, fp32 accumulation). */
