@@ -36,6 +36,7 @@ extern "C" {
     X(MVSK4_F32, "g2k_mvsk_f32_4") X(MVSK4_F16, "g2k_mvsk_f16_4")       \
     X(MVSK8_F32, "g2k_mvsk_f32_8") X(MVSK8_F16, "g2k_mvsk_f16_8")       \
     X(MVSK16_F32, "g2k_mvsk_f32_16") X(MVSK16_F16, "g2k_mvsk_f16_16")   \
+    X(MVSK64_F32, "g2k_mvsk_f32_64")                                          \
     X(REDUCE, "g2k_reduce") X(LAYERNORM, "g2k_layernorm")                     \
     X(ADD, "g2k_add") X(GELU, "g2k_gelu")                                     \
     X(EMBED_F32, "g2k_embed_f32") X(EMBED_F16, "g2k_embed_f16")               \
@@ -143,6 +144,8 @@ int g2i_device_alloc(void **p, size_t bytes);
 int g2i_rows_launch(int fid_f32_64, int f16, g2_rows_args *a);
 /* Work-groups g2i_rows_launch uses for N rows of K (0 if K is invalid). */
 unsigned g2i_rows_grid(int N, int K, int f16);
+/* g2_matvec's column lanes (of 16 bytes) to a work-group and its K slices. */
+int g2i_matvec_form(int num_cus, int f16, int N, int K, int *slices);
 /* Whether a matvec's result lies in none of its operands, but for a bias or
  * residual exactly in place: then one launch may write while it reads. */
 int g2i_matvec_apart(const float *A, const void *B, size_t b_size, const float *bias, const float *res, const float *C,

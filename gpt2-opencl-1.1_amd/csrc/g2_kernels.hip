@@ -193,6 +193,7 @@ __device__ void matvec_impl(const g2_matvec_args &a)
 G2_MATVEC(g2k_mvsk_f32_4, float, 4)
 G2_MATVEC(g2k_mvsk_f32_8, float, 8)
 G2_MATVEC(g2k_mvsk_f32_16, float, 16)
+G2_MATVEC(g2k_mvsk_f32_64, float, 64)
 G2_MATVEC(g2k_mvsk_f16_4, _Float16, 4)
 G2_MATVEC(g2k_mvsk_f16_8, _Float16, 8)
 G2_MATVEC(g2k_mvsk_f16_16, _Float16, 16)

@@ -470,34 +470,83 @@ int g2_matmul_f16(const float *A, const uint16_t *B, const float *bias, float *C
 }
 
 /* Column lanes of a matvec work-group (CL lanes of 16 bytes): 16 (256 bytes of
- * a row per work-group, the best of HBM's rate), fewer where that leaves under
- * 160 work-groups for the chip; four at least (64 bytes; two were slower).
- * us with 4 / 8 / 16: 6400 x 1600 fp32 (400 / 200 / 100 work-groups) 17.6 /
- * 11.0 / 13.6, fp16 (200 / 100 / 50) 9.1 / 10.7 / 17.6; 50257 x 768 fp32 63 /
- * 44 / 37. */
-static int matvec_launch(int f16, g2_matvec_args *a)
+ * a row per work-group), fewer where that leaves under 160 work-groups for the
+ * chip; four at least (64 bytes; two were slower).  us with 4 / 8 / 16: 6400 x
+ * 1600 fp32 (400 / 200 / 100 work-groups) 17.6 / 11.0 / 13.6, fp16 (200 / 100 /
+ * 50) 9.1 / 10.7 / 17.6; 50257 x 768 fp32 63 / 44 / 37. */
+static int matvec_lanes(int f16, long N, int slices)
+{
+    const int v = f16 ? 8 : 4;
+    int cl = 16;
+    while (cl > 4 && (N + cl * v - 1) / (cl * v) * slices < 160) cl /= 2;
+    return cl;
+}
+
+/* Long columns of large matrices (K >= 2048, 50 MB): by estimated time (us) of
+ * the lanes and slices, since a few work-groups too many cost a whole round
+ * over the chip.  A column group's time at K 6400 is `one` for a lone
+ * work-group and `round` while all CUs have one; `rate` is what these lanes
+ * get out of memory (bytes per us, rate1 in one round of whole columns); slices
+ * cost 4 us with the second launch.  Fitted to MI355X times of 26
+ * widths from 512 to 50257 with matrices that no cache holds; us of the rule
+ * above / the choice / two launches of 256 columns by up to 64 slices each (the
+ * form before): 10000 x 6400 fp16 56 (313 work-groups of 4 lanes) / 31 (16
+ * lanes, 3 slices) / 42; 10000 x 6400 fp32 69 / 46 (64 lanes, 5) / 61; 25000 x
+ * 6400 131 / 111 (64 lanes, 2) / 122; 20000 x 6400 fp16 65 / 56 / 57.  Smaller
+ * or shorter ones: one launch, but for tall narrow matrices, whose few
+ * work-groups would walk over 128 KB each (1600 x 6400 fp32 11 us + the launch
+ * against 20, 768 x 3072 7 against 13). */
+int g2i_matvec_form(int num_cus, int f16, int N, int K, int *slices)
+{
+    static const struct { int cl; double one, round, rate, rate1; } forms[2][3] = {
+        { { 8, 31, 38, 3.9e6, 5.3e6 }, { 16, 44, 60, 4.9e6, 5.4e6 }, { 64, 176, 190, 6.0e6, 6.0e6 } },
+        { { 8, 35, 36, 3.9e6, 5.3e6 }, { 16, 62, 36, 4.9e6, 4.9e6 }, { 0, 0, 0, 0, 0 } },
+    };
+    const double bytes = (double)N * K * (f16 ? 2 : 4);
+    *slices = 1;
+    if (K < 2048 || bytes < 50e6) {
+        const unsigned narrow = cdiv(N, f16 ? 32 : 16);
+        if (K > 2048 && narrow < 160) *slices = cdiv(256, narrow) < 8 ? (int)cdiv(256, narrow) : 8;
+        return matvec_lanes(f16, N, *slices);
+    }
+    double best = 1e300;
+    int cl = 16;
+    for (int i = 0; i < 3 && forms[f16][i].cl; ++i) {
+        const double groups = cdiv(N, forms[f16][i].cl * (f16 ? 8 : 4));
+        for (int ns = 1; ns <= (i == 0 ? 1 : 8); ++ns) {
+            const double rounds = ceil(groups * ns / num_cus);
+            double us = K / 6400.0 / ns * (rounds * forms[f16][i].round > forms[f16][i].one ? rounds * forms[f16][i].round
+                                                                                              : forms[f16][i].one);
+            const double least = bytes / (ns == 1 && rounds == 1 ? forms[f16][i].rate1 : forms[f16][i].rate);
+            if (us < least) us = least;
+            if (ns > 1) us += 4;
+            if (us < best) { best = us; cl = forms[f16][i].cl; *slices = ns; }
+        }
+    }
+    return cl;
+}
+
+static int matvec_launch(int f16, int cl, g2_matvec_args *a)
 {
     const unsigned v = f16 ? 8 : 4;
-    int shape = 2; /* CL = 4 << shape */
-    while (shape > 0 && cdiv(a->N, (4u << shape) * v) * (unsigned)a->nslice < 160) --shape;
-    const int fid = (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + 2 * shape;
+    const int fid = cl == 64 ? G2F_MVSK64_F32
+                             : (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + (cl == 16 ? 4 : cl == 8 ? 2 : 0);
     const long N = a->N;
     for (long n0 = 0; n0 < N; n0 += G2_MV_LAUNCH_COLS) { /* (no bias or residual where N is above one launch) */
         g2_matvec_args w = *a;
         w.N = (int)(N - n0 < G2_MV_LAUNCH_COLS ? N - n0 : G2_MV_LAUNCH_COLS);
         w.B = (const char *)a->B + n0 * (f16 ? 2 : 4);
         w.out = a->out + n0;
-        const int rc = g2i_launch(fid, cdiv(w.N, (4u << shape) * v), (unsigned)a->nslice, 1024, &w);
+        const int rc = g2i_launch(fid, cdiv(w.N, (unsigned)cl * v), (unsigned)a->nslice, 1024, &w);
         if (rc) return rc;
     }
     return G2_OK;
 }
 
-/* One launch, except: a tall narrow matrix (its few work-groups would walk
- * over 128 KB each) goes in slices to the scratch, added by a second launch
- * (1600 x 6400 fp32 11 us + the launch against 20, 768 x 3072 7 against 13);
- * so does a product into memory that holds its operands (bias and residual in
- * place are read by the thread that writes there). */
+/* One launch where one slice is best (g2i_matvec_form); slices go to the
+ * scratch, added by a second launch; so does a product into memory that holds
+ * its operands (bias and residual in place are read by the thread that writes
+ * there). */
 int g2i_matvec_apart(const float *A, const void *B, size_t b_size, const float *bias, const float *res, const float *C,
                      int N, int K)
 {
@@ -513,17 +562,16 @@ static int matvec_any(int f16, const float *A, const void *B, const float *bias,
     if (!A || !B || !C) return g2i_err(G2_E_ARG, "g2_matvec: NULL buffer");
     if (N <= 0 || K <= 0) return g2i_err(G2_E_ARG, "g2_matvec: N and K must be positive");
     if (N > 65536) return g2i_err(G2_E_LIMIT, "g2_matvec: N=%d above 65536", N);
-    const unsigned narrow = cdiv(N, f16 ? 32 : 16);
-    unsigned slices = 1;
-    if (K > 2048 && narrow < 160) slices = cdiv(256, narrow) < 8 ? cdiv(256, narrow) : 8;
+    int slices;
+    const int cl = g2i_matvec_form(g2i_cus(), f16, N, K, &slices);
     if (slices == 1 && g2i_matvec_apart(A, B, f16 ? 2 : 4, bias, res, C, N, K)) {
         g2_matvec_args a = { A, B, C, bias, res, N, K, 1, gelu ? 1 : 0, N };
-        return matvec_launch(f16, &a);
+        return matvec_launch(f16, cl, &a);
     }
-    g2_matvec_args a = { A, B, G.scratch, NULL, NULL, N, K, (int)slices, 0, N };
-    g2_reduce_args r = { G.scratch, bias, res, C, N, (int)slices, gelu ? 1 : 0 };
+    g2_matvec_args a = { A, B, G.scratch, NULL, NULL, N, K, slices, 0, N };
+    g2_reduce_args r = { G.scratch, bias, res, C, N, slices, gelu ? 1 : 0 };
     scratch_lock();
-    int rc = matvec_launch(f16, &a);
+    int rc = matvec_launch(f16, cl, &a);
     if (!rc) rc = g2i_launch(G2F_REDUCE, cdiv(N, 256), 1, 256, &r);
     scratch_unlock();
     return rc;
@@ -553,7 +601,7 @@ static int matvec_sk_any(int f16, const float *A, const void *B, float *partial,
     if (kslice == 1 && N <= 65536 && !g2i_matvec_apart(A, B, f16 ? 2 : 4, NULL, NULL, partial, N, K))
         return matvec_any(f16, A, B, NULL, NULL, partial, N, K, 0);
     g2_matvec_args a = { A, B, partial, NULL, NULL, N, K, kslice, 0, N };
-    return matvec_launch(f16, &a);
+    return matvec_launch(f16, matvec_lanes(f16, N, kslice), &a);
 }
 
 int g2_matvec_sk(const float *A, const float *B, float *partial, int N, int K, int kslice)

@@ -134,3 +134,28 @@ def test_matmul_tests_reach_every_form_on_ragged_sizes():
     assert reached(FORM_SIZES, False) == every
     assert reached(EDGES, True) | {(2, True)} == every  # splits of 64 x 64: an even 300 columns, 5007 = 156 * 32 + 15
     assert (2, True) in reached([s for s in EDGES if s[0] % 64 and s[2] % 32], False)
+
+
+def matvec_form(f16, N, K, cus=256):
+    slices = C.c_int()
+    return lib.g2i_matvec_form(cus, int(f16), N, K, C.byref(slices)), slices.value
+
+
+def test_matvec_forms():
+    """The lanes and slices that the large matrices' test is there for, no
+    choice outside the kernels and the scratch (eight slices of 65536), and no
+    work-groups of a second round for a fifth of the chip: 10000 x 6400 fp16
+    had 313 of them on 256 CUs."""
+    from test_matvec_gpu import LARGE
+
+    assert {matvec_form(*c)[0] for c in LARGE} == {8, 16, 64}
+    assert {matvec_form(*c)[1] > 1 for c in LARGE if matvec_form(*c)[0] == 16} == {True}
+    rng = random.Random(11)
+    for _ in range(5000):
+        f16, N, K = rng.random() < 0.5, int(2 ** rng.uniform(0, 16)), int(2 ** rng.uniform(0, 14))
+        lanes, slices = matvec_form(f16, N, K)
+        assert lanes in ((4, 8, 16) if f16 else (4, 8, 16, 64)) and 1 <= slices <= 8 and slices <= K
+    for f16, N, K in ((True, 10000, 6400), (False, 10000, 6400), (False, 20000, 6400), (False, 25000, 4096)):
+        lanes, slices = matvec_form(f16, N, K)
+        rounds = -(-N // (lanes * (8 if f16 else 4))) * slices / 256
+        assert rounds / -(-rounds // 1) > 0.75

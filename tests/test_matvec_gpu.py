@@ -1,7 +1,7 @@
 """g2_matvec and g2_matvec_sk at the sizes where their launches can go wrong:
 rows shorter than one 16-byte vector, columns past the last whole vector or
 column group, K below and above the rows that a work-group takes at once, the
-column-lane choices, the sliced form of tall narrow matrices, operands at odd
+column-lane choices, the sliced forms of tall narrow and of large matrices, operands at odd
 addresses and results that overlap an operand; and the elementwise operators'
 and the LayerNorm's remainders; against the CPU oracle."""
 import numpy as np
@@ -39,6 +39,22 @@ def test_matvec_edges(g2, N, K, f16):
         got = dC.download(np.float32, N + 8)
         assert (got[N:] == 7.0).all()  # nothing past the vector
         assert_close_bound(got[:N], exact(A, B, bias, res), bound, what="matvec")
+
+
+LARGE = [(False, 6301, 2050), (False, 9001, 2049), (False, 3126, 4100), (True, 10007, 2600), (True, 12505, 2049)]
+
+
+@pytest.mark.parametrize("f16,N,K", LARGE)
+def test_matvec_large(g2, f16, N, K):
+    """Matrices of 50 MB and more with long columns: 64, 16 and 8 lanes to a
+    work-group, in K slices that do not divide K, ragged columns; GELU and
+    residual behind the slices."""
+    A, B, bias, res = operands(N, K, f16, N)
+    dC = g2.to_device(np.concatenate([res, np.full(8, 7.0, np.float32)]))
+    g2.matvec(g2.to_device(A), g2.to_device(g2.convert_f16(B) if f16 else B), g2.to_device(bias), dC, dC, N, K, f16=f16)
+    got = dC.download(np.float32, N + 8)
+    assert (got[N:] == 7.0).all()
+    assert_close_bound(got[:N], exact(A, B, bias, res), dot_bound(np.abs(A), np.abs(B), K), what="matvec")
 
 
 @pytest.mark.parametrize("N,K", [(768, 768), (100, 2500)])
