@@ -324,13 +324,44 @@ __device__ __forceinline__ void qkv_store4(const qkv_dst &d, int mb, int M, int 
 /* ---- layernorm (math.cl:283-311): one work-group per row, two-pass mean and
  * biased variance, eps 1e-5, out = (x-mean)*inv_std*gamma + beta.  SPLIT:
  * the row is written as fp16 halves (g2_lnsplit_args), same arithmetic. */
+/* A row of at most 256 V in registers, parameters loaded with it: one memory
+ * latency (256 rows of 1280: 5.1 -> 3.9 us). */
+template <int V, typename ARGS, typename PUT>
+__device__ __forceinline__ void layernorm_row(const ARGS &a, const float *x, float (&red4)[4], PUT put)
+{
+    float v[V], g[V], b[V], s = 0.f, q = 0.f;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int i = min((int)threadIdx.x + 256 * k, a.E - 1);
+        v[k] = x[i];
+        g[k] = a.gamma[i];
+        b[k] = a.beta[i];
+    }
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+        if ((int)threadIdx.x + 256 * k < a.E) s += v[k];
+    const float mean = block_sum(s, red4) / (float)a.E;
+#pragma unroll
+    for (int k = 0; k < V; ++k)
+        if ((int)threadIdx.x + 256 * k < a.E) {
+            const float d = v[k] - mean;
+            q = fmaf(d, d, q);
+        }
+    const float var = block_sum(q, red4) / (float)a.E;
+    const float inv = 1.0f / sqrtf(var + 1e-5f);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int i = threadIdx.x + 256 * k;
+        if (i < a.E) put(i, fmaf((v[k] - mean) * inv, g[k], b[k]));
+    }
+}
+
+/* Rows of up to 2048 as layernorm_row, with no more loads than the row needs
+ * (8192 rows of 64: 13 us with eight a thread, 8 with one); longer ones are
+ * read three times. */
 template <bool SPLIT, typename ARGS>
 __device__ void layernorm_impl(const ARGS &a)
 {
-    /* rows of up to 2048 stay in registers, parameters loaded with them: one
-     * memory latency (256 rows of 1280: 5.1 -> 3.9 us); longer ones are
-     * read three times */
-    constexpr int V = 8;
     __shared__ float red4[4];
     const int row = blockIdx.x;
     if (row >= a.rows) return;
@@ -339,34 +370,10 @@ __device__ void layernorm_impl(const ARGS &a)
         if constexpr (SPLIT) split_store(a.hi, a.lo, (size_t)row * a.E + i, y);
         else a.out[(size_t)row * a.E + i] = y;
     };
-    if (a.E <= 256 * V) {
-        float v[V], g[V], b[V], s = 0.f, q = 0.f;
-#pragma unroll
-        for (int k = 0; k < V; ++k) {
-            const int i = min((int)threadIdx.x + 256 * k, a.E - 1);
-            v[k] = x[i];
-            g[k] = a.gamma[i];
-            b[k] = a.beta[i];
-        }
-#pragma unroll
-        for (int k = 0; k < V; ++k)
-            if ((int)threadIdx.x + 256 * k < a.E) s += v[k];
-        const float mean = block_sum(s, red4) / (float)a.E;
-#pragma unroll
-        for (int k = 0; k < V; ++k)
-            if ((int)threadIdx.x + 256 * k < a.E) {
-                const float d = v[k] - mean;
-                q = fmaf(d, d, q);
-            }
-        const float var = block_sum(q, red4) / (float)a.E;
-        const float inv = 1.0f / sqrtf(var + 1e-5f);
-#pragma unroll
-        for (int k = 0; k < V; ++k) {
-            const int i = threadIdx.x + 256 * k;
-            if (i < a.E) put(i, fmaf((v[k] - mean) * inv, g[k], b[k]));
-        }
-        return;
-    }
+    if (a.E <= 256) return layernorm_row<1>(a, x, red4, put);
+    if (a.E <= 512) return layernorm_row<2>(a, x, red4, put);
+    if (a.E <= 1024) return layernorm_row<4>(a, x, red4, put);
+    if (a.E <= 2048) return layernorm_row<8>(a, x, red4, put);
     float s = 0.f;
     for (int i = threadIdx.x; i < a.E; i += 256) s += x[i];
     const float mean = block_sum(s, red4) / (float)a.E;
