@@ -398,7 +398,7 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
         if (ks > 1) us += 5 + (2 * ks + 1) * mn * sizeof(float) / 6e6;
         if (us < best) { best = us; pick = XG_64; *splits = ks; }
     }
-    if (N >= 2) {
+    if (N >= 2 && steps > 1) { /* one step: the larger tile's epilogue is all that differs (512 x 10000 x 1 9 us, 11) */
         const double tiles = (double)((N + 127) / 128) * (double)((M + 127) / 128);
         const double t = 0.5 + 1.25 * (tiles / cus);
         const double us = 3 + steps * (t > 1.85 ? t : 1.85);

@@ -42,11 +42,11 @@ def product(g2, A, B, bias, f16):
 
 EDGES = [
     (1, 1, 1), (1, 1, 40), (17, 1, 65), (3, 2, 31),            # 64 x 64; one column: no pairs
-    (16, 31, 32), (333, 1601, 96), (470, 2305, 70),            # 64 x 64
+    (16, 31, 32), (333, 1601, 96), (470, 2305, 70), (641, 12801, 32),  # 64 x 64
     (40, 300, 5007),                                           # 64 x 64 in 12 splits
     (17, 33, 33), (15, 65, 257), (33, 97, 300), (65, 129, 1000), (130, 257, 2049),  # direct, 16 rows
     (50, 3203, 259), (18, 5755, 1389),                         # direct, 32 rows
-    (700, 8321, 70), (641, 12801, 32),                         # 128 x 128
+    (700, 8321, 70), (657, 12803, 40),                         # 128 x 128
     (118, 20173, 1191), (200, 9001, 300),                      # 128 x 128, alternating groups
     (257, 5121, 1281),                                         # alternating groups in 2 splits
 ]
