@@ -1041,7 +1041,9 @@ static int sg_pick(int M, int N, int K, int *splits)
     for (int form = SG_FORM_DUO64; form <= SG_FORM_DUO128; ++form) {
         const int rows = form == SG_FORM_DUO64 ? 64 : 128;
         const unsigned tiles = cdivu(N, 128) * cdivu(M, (unsigned)rows);
-        for (int k = form == SG_FORM_DUO64 ? 2 : 1; k <= G2_SKEPI_MAXKS && 2 * k <= nk; ++k) {
+        /* a whole tile of fewer than 8 steps: its fill and epilogue, not its
+         * steps, take the time (n_embd 128, 512 rows: qkv 13.8 us against 8.8) */
+        for (int k = form == SG_FORM_DUO64 || nk < 8 ? 2 : 1; k <= G2_SKEPI_MAXKS && 2 * k <= nk; ++k) {
             if (k > 1 && tiles * (unsigned)k > cus) break;
             const double rounds = ceil(tiles * k / cus); /* several, all CUs at it: a third slower */
             const double us = 4 + (double)nk / k * (rows == 64 ? 0.75 : rounds > 1 ? 1.4 : 1.02) * rounds +
@@ -1117,13 +1119,14 @@ static int fused_prefill(g2_model *m, int P)
      * fp32-MFMA GEMM for comparison */
     const char *pe = getenv("G2_PREFILL_F32MFMA");
     const int h = f16 && E % 64 == 0 && F % 64 == 0 && !(pe && pe[0] == '1');
-    /* the 128x128 tiles for every prompt: short ones leave most of a tile's
-     * rows unused, but their K splits stream the weights from all CUs, which
-     * is what bounds them (8 tokens: 774M 2.0 ms against 4.0 on the 64x64
-     * tiles, 1.5B 3.1 against 6.3).  G2_PREFILL_GEMM64=1 keeps the 64x64 ones,
+    /* the 128x128 tiles, but for prompts of up to 64 rows and n_embd up to 256
+     * (n_embd 128, 8 rows, four layers 168 us against 183; 256: 196, 195; 384:
+     * 234, 206): short ones leave most of a tile's rows unused, but their K
+     * splits stream the weights from all CUs, which is what bounds them (8
+     * tokens: 774M 2.0 ms against 4.0 on the 64x64 tiles, 1.5B 3.1 against 6.3).  G2_PREFILL_GEMM64=1 keeps the 64x64 ones,
      * whose results agree to fp32 rounding */
     const char *p64 = getenv("G2_PREFILL_GEMM64");
-    const int big = h && !(p64 && p64[0] == '1');
+    const int big = h && (P > 64 || E > 256) && !(p64 && p64[0] == '1');
     /* fp32 weights: prefill_sgemm's forms (sg_pick) */
     const int sg = !f16 && E % 32 == 0 && F % 32 == 0;
     const int f_qkv = big ? G2F_HGEMM2_QKV : h ? G2F_HGEMM_QKV : (f16 ? G2F_GEMM_NK_F16_QKV : G2F_GEMM_NK_F32_QKV);

@@ -8,7 +8,8 @@ for ragged prompt lengths (not multiples of a tile's rows) up to the
 1023-position limit.  The lengths cover qkv and fc as K slices (100 rows and
 fewer: 6 and 5 slices; 200, 256: 3 and 2) and run whole (1023 rows), with proj
 and fc2 as 2 to 8 slices summed with the following LayerNorm.  The 64x64 GEMM
-(g2k_hgemm_*), which only G2_PREFILL_GEMM64=1 takes, is compared with it.
+(g2k_hgemm_*), which short prompts of models up to n_embd 256 and
+G2_PREFILL_GEMM64=1 take, is compared with it.
 """
 import numpy as np
 import pytest
@@ -144,3 +145,19 @@ def test_prefill_f32_forms(g2, E, NH, P):
     got = m.logits().copy()
     m.free()
     np.testing.assert_allclose(got, ref, rtol=2e-4, atol=2e-4)
+
+
+@pytest.mark.parametrize("f16", [False, True], ids=["f32", "f16"])
+@pytest.mark.parametrize("E,P", [(128, 1), (128, 64), (256, 64), (256, 65), (320, 64), (128, 300), (256, 700)])
+def test_prefill_narrow_models(g2, E, P, f16):
+    """Widths and prompts on both sides of the choice between the 64x64 and the
+    128x128 fp16 tiles, and of the fp32 forms for few K steps, against the
+    oracle: every logit within 2e-4 (as above)."""
+    cfg = g2.make_config(2, E, E // 64, vocab_size=1000)
+    w = g2.synth_weights(cfg, SEED, f16_round=f16, affine=True)
+    prompt = random_prompt(P, cfg.vocab_size, E + P)
+    ref = oracle.Model(cfg, w).generate(prompt, 1, logit_steps=1)[2][0]
+    m = g2.Model.from_host(cfg, w, g2.F16 if f16 else g2.F32, g2.PATH_FUSED)
+    m.prefill(prompt)
+    np.testing.assert_allclose(m.logits(), ref, rtol=2e-4, atol=2e-4)
+    m.free()
