@@ -36,7 +36,7 @@ extern "C" {
     X(MVSK4_F32, "g2k_mvsk_f32_4") X(MVSK4_F16, "g2k_mvsk_f16_4")       \
     X(MVSK8_F32, "g2k_mvsk_f32_8") X(MVSK8_F16, "g2k_mvsk_f16_8")       \
     X(MVSK16_F32, "g2k_mvsk_f32_16") X(MVSK16_F16, "g2k_mvsk_f16_16")   \
-    X(MVSK64_F32, "g2k_mvsk_f32_64")                                          \
+    X(MVSK64_F32, "g2k_mvsk_f32_64") X(MVSK16D_F16, "g2k_mvsk_f16_16d")       \
     X(REDUCE, "g2k_reduce") X(LAYERNORM, "g2k_layernorm")                     \
     X(ADD, "g2k_add") X(GELU, "g2k_gelu")                                     \
     X(EMBED_F32, "g2k_embed_f32") X(EMBED_F16, "g2k_embed_f16")               \

@@ -111,7 +111,7 @@ template <> __device__ __forceinline__ float ldw<_Float16>(const _Float16 *p, si
  * 20 with fp16 (47); 768 x 3072 in four slices 7 (85: one lane per four
  * columns walked its slice alone).  Eight rows ahead instead of four: 39 and
  * 23 us for 50257 x 768, no gain elsewhere. */
-template <typename WT, int CL>
+template <typename WT, int CL, int S>
 __device__ void matvec_impl(const g2_matvec_args &a)
 {
     constexpr int V = 16 / sizeof(WT), RG = 1024 / CL;
@@ -121,9 +121,16 @@ __device__ void matvec_impl(const g2_matvec_args &a)
     const int N = a.N, K = a.K, ns = a.nslice, ld = a.ld;
     const int col = (blockIdx.x * CL + cl) * V, base = min(col, max(N - V, 0));
     const WT *B = (const WT *)a.B + base;
-    float acc[V];
+    /* A thread's rows in S sums, every S-th row to each: more lanes and fewer
+     * slices leave it more rows, and their error should be no larger (fp32
+     * takes four sums without registers that it lacks; two made 40000 x 6400
+     * fp16 50% slower, a work-group per CU less) */
+    constexpr int U = 4;
+    float sum[S][V], (&acc)[V] = sum[0];
 #pragma unroll
-    for (int e = 0; e < V; ++e) acc[e] = 0.f;
+    for (int u = 0; u < S; ++u)
+#pragma unroll
+        for (int e = 0; e < V; ++e) sum[u][e] = 0.f;
     auto row = [&](int k, float (&w)[V]) {
         const WT *p = B + (size_t)k * ld;
         if (N < V) { /* one vector would leave the row */
@@ -139,7 +146,6 @@ __device__ void matvec_impl(const g2_matvec_args &a)
             for (int e = 0; e < V; ++e) w[e] = (float)v[e];
         }
     };
-    constexpr int U = 4;
     const long step = (long)RG * ns;
     long k = blockIdx.y + (long)rg * ns;
     for (; k + (U - 1) * step < K; k += U * step) {
@@ -152,7 +158,7 @@ __device__ void matvec_impl(const g2_matvec_args &a)
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
-            for (int e = 0; e < V; ++e) acc[e] = fmaf(x[u], w[u][e], acc[e]);
+            for (int e = 0; e < V; ++e) sum[u % S][e] = fmaf(x[u], w[u][e], sum[u % S][e]);
     }
     {
         float x[U - 1], w[U - 1][V];
@@ -166,8 +172,14 @@ __device__ void matvec_impl(const g2_matvec_args &a)
         for (int u = 0; u < U - 1; ++u)
             if (k + u * step < K)
 #pragma unroll
-                for (int e = 0; e < V; ++e) acc[e] = fmaf(x[u], w[u][e], acc[e]);
+                for (int e = 0; e < V; ++e) sum[u % S][e] = fmaf(x[u], w[u][e], sum[u % S][e]);
     }
+#pragma unroll
+    for (int h = S / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int u = 0; u < h; ++u)
+#pragma unroll
+            for (int e = 0; e < V; ++e) sum[u][e] += sum[u + h][e];
 #pragma unroll
     for (int o = CL; o < 64; o <<= 1)
 #pragma unroll
@@ -188,15 +200,16 @@ __device__ void matvec_impl(const g2_matvec_args &a)
     if (a.apply_gelu) v = gelu_f(v);
     a.out[(size_t)blockIdx.y * ld + n] = v;
 }
-#define G2_MATVEC(name, WT, CL) \
-    extern "C" __global__ __launch_bounds__(1024) void name(const g2_matvec_args a) { matvec_impl<WT, CL>(a); }
-G2_MATVEC(g2k_mvsk_f32_4, float, 4)
-G2_MATVEC(g2k_mvsk_f32_8, float, 8)
-G2_MATVEC(g2k_mvsk_f32_16, float, 16)
-G2_MATVEC(g2k_mvsk_f32_64, float, 64)
-G2_MATVEC(g2k_mvsk_f16_4, _Float16, 4)
-G2_MATVEC(g2k_mvsk_f16_8, _Float16, 8)
-G2_MATVEC(g2k_mvsk_f16_16, _Float16, 16)
+#define G2_MATVEC(name, WT, CL, S) \
+    extern "C" __global__ __launch_bounds__(1024) void name(const g2_matvec_args a) { matvec_impl<WT, CL, S>(a); }
+G2_MATVEC(g2k_mvsk_f32_4, float, 4, 1)
+G2_MATVEC(g2k_mvsk_f32_8, float, 8, 1)
+G2_MATVEC(g2k_mvsk_f32_16, float, 16, 4)
+G2_MATVEC(g2k_mvsk_f32_64, float, 64, 4)
+G2_MATVEC(g2k_mvsk_f16_4, _Float16, 4, 1)
+G2_MATVEC(g2k_mvsk_f16_8, _Float16, 8, 1)
+G2_MATVEC(g2k_mvsk_f16_16, _Float16, 16, 1)
+G2_MATVEC(g2k_mvsk_f16_16d, _Float16, 16, 2)
 
 /* ---- reduce_partial (math.cl:249-280): slices added in order, then bias,
  * residual, GELU.  residual may alias C (each n is read then written by the

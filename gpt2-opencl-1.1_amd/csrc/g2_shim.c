@@ -526,11 +526,12 @@ int g2i_matvec_form(int num_cus, int f16, int N, int K, int *slices)
     return cl;
 }
 
-static int matvec_launch(int f16, int cl, g2_matvec_args *a)
+/* `two`: 16 lanes of fp16 with two sums to a thread. */
+static int matvec_launch(int f16, int cl, int two, g2_matvec_args *a)
 {
     const unsigned v = f16 ? 8 : 4;
-    const int fid = cl == 64 ? G2F_MVSK64_F32
-                             : (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + (cl == 16 ? 4 : cl == 8 ? 2 : 0);
+    const int fid = two ? G2F_MVSK16D_F16 : cl == 64 ? G2F_MVSK64_F32
+                        : (f16 ? G2F_MVSK4_F16 : G2F_MVSK4_F32) + (cl == 16 ? 4 : cl == 8 ? 2 : 0);
     const long N = a->N;
     for (long n0 = 0; n0 < N; n0 += G2_MV_LAUNCH_COLS) { /* (no bias or residual where N is above one launch) */
         g2_matvec_args w = *a;
@@ -566,12 +567,13 @@ static int matvec_any(int f16, const float *A, const void *B, const float *bias,
     const int cl = g2i_matvec_form(g2i_cus(), f16, N, K, &slices);
     if (slices == 1 && g2i_matvec_apart(A, B, f16 ? 2 : 4, bias, res, C, N, K)) {
         g2_matvec_args a = { A, B, C, bias, res, N, K, 1, gelu ? 1 : 0, N };
-        return matvec_launch(f16, cl, &a);
+        return matvec_launch(f16, cl, 0, &a);
     }
     g2_matvec_args a = { A, B, G.scratch, NULL, NULL, N, K, slices, 0, N };
     g2_reduce_args r = { G.scratch, bias, res, C, N, slices, gelu ? 1 : 0 };
     scratch_lock();
-    int rc = matvec_launch(f16, cl, &a);
+    /* from three slices on the 16 lanes stand where 4 would have less to sum */
+    int rc = matvec_launch(f16, cl, f16 && cl == 16 && slices >= 3, &a);
     if (!rc) rc = g2i_launch(G2F_REDUCE, cdiv(N, 256), 1, 256, &r);
     scratch_unlock();
     return rc;
@@ -601,7 +603,7 @@ static int matvec_sk_any(int f16, const float *A, const void *B, float *partial,
     if (kslice == 1 && N <= 65536 && !g2i_matvec_apart(A, B, f16 ? 2 : 4, NULL, NULL, partial, N, K))
         return matvec_any(f16, A, B, NULL, NULL, partial, N, K, 0);
     g2_matvec_args a = { A, B, partial, NULL, NULL, N, K, kslice, 0, N };
-    return matvec_launch(f16, matvec_lanes(f16, N, kslice), &a);
+    return matvec_launch(f16, matvec_lanes(f16, N, kslice), 0, &a);
 }
 
 int g2_matvec_sk(const float *A, const float *B, float *partial, int N, int K, int kslice)
