@@ -358,9 +358,9 @@ static int capturing(void)
  * The constants are fitted to MI355X times; on 45 shapes (8..1024 rows, 258 to
  * 50257 columns, K 267..5907) with both weight types the pick is the fastest
  * form or within 10% of it on 87 of 90 (37 x 10569 x 1205: 10.2%, 22 x 9814 x
- * 5293: 25 and 17%); profiles/matmul_forms.md has every form's time at each.  Examples, us with fp32
- * B of direct 16 / direct 32 / 64 x 64 / its best split / 128 x 128 /
- * alternating groups / their best split: 96 x 768 x 3072: 16 / 21 / 77 / 16 /
+ * 5293: 25 and 17%); profiles/matmul_forms.md has every form's time at each.
+ * Examples, us with fp32 B of direct 16 / direct 32 / 64 x 64 / its best split
+ * / 128 x 128 / alternating groups / their best split: 96 x 768 x 3072: 16 / 21 / 77 / 16 /
  * 168 / 109 / 20; 512 x 1024 x 1024: 21 / 17 / 29 / 20 / 60 / 41 / 22; 256 x
  * 1280 x 5120: 63 / 61 / 126 / 35 / 277 / 178 / 31; 333 x 6400 x 1600: 114 /
  * 94 / 79 / - / 97 / 66 / -; 1024 x 50257 x 1600: - / - / 1140 / - / 883 / 896
@@ -388,7 +388,10 @@ int g2i_matmul_pick(int num_cus, long M, long N, long K, int whole, int *splits)
         const double per_cu = xg_load((double)((N + 31) / 32) * (double)((M + 16 * r - 1) / (16 * r)) / cus);
         const double t = r == 1 ? per_cu : 1.6 * per_cu, latency = r == 1 ? 1.0 : 1.4;
         const double us = 3 + (double)(long)((steps + 7) / 8) * (t > latency ? t : latency);
-        if (us < best && grid_fits(((N + 31) / 32) * ((M + 16 * r - 1) / (16 * r)), 512)) { best = us; pick = r == 1 ? XG_DIRECT16 : XG_DIRECT32; }
+        if (us < best && grid_fits(((N + 31) / 32) * ((M + 16 * r - 1) / (16 * r)), 512)) {
+            best = us;
+            pick = r == 1 ? XG_DIRECT16 : XG_DIRECT32;
+        }
     }
     const double tiles = (double)((N + 63) / 64) * (double)((M + 63) / 64), mn = (double)M * (double)N;
     for (int ks = 1; ks <= G2_XG_MAXKS; ++ks) {
